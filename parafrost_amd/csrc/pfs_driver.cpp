@@ -1408,12 +1408,13 @@ bool Simplifier::ve() {
   stage_begin(S_VE);
   DB db = make_db(cur_);
   u32* sc = P<u32>(scal_);
-  k_list_sizes(db, P<u32>(pv_), E_, 2, P<u32>(vsz_), st_);
-  scan_u32(P<u32>(vsz_), P<u32>(vbase_), E_, sc, tmp_.p, st_);
-  const u32 S = read_u32(sc);
-  mem_.ensure(scratch_, std::max<size_t>(S, 1) * 4, 0, st_);
-  VeDecision d{P<u32>(type_), P<u32>(def_), P<u32>(vncls_), P<u32>(vnlits_), P<u32>(vnstack_),
-               P<u32>(scratch_), P<u32>(vbase_)};
+  u32 S = 0;
+  if (opt.proof_en) {  // room for the lines of EQU substitutions: the list entries
+    k_list_sizes(db, P<u32>(pv_), E_, 2, P<u32>(vsz_), st_);
+    scan_u32(P<u32>(vsz_), P<u32>(vbase_), E_, sc, tmp_.p, st_);
+    S = read_u32(sc);
+  }
+  VeDecision d{P<u32>(type_), P<u32>(def_), P<u32>(vncls_), P<u32>(vnlits_), P<u32>(vnstack_)};
   k_ve_decide(db, opt, P<u32>(pv_), E_, d, work_order(), P<u32>(vrest_), P<u32>(lsum_), tmp_.p, st_);
   scan_u32(P<u32>(vncls_), P<u32>(clsb_), E_, sc, tmp_.p, st_);
   scan_u32(P<u32>(vnlits_), P<u32>(litb_), E_, sc + 1, tmp_.p, st_);

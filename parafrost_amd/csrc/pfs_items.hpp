@@ -59,6 +59,86 @@ PF_HD u64 at_min64(u64* p, u64 v) {
 #endif
 }
 
+// ---------------------------------------------------------------- lane groups
+// Groups of G consecutive lanes of a wavefront may share one variable
+// (gl = 0..G-1 is the lane's place in its group; G = 1 is one lane per
+// variable).  group_first returns the lowest j in [0, n) with pred(j), n if
+// none: the group tests j = gl, gl + G, ... and takes the lowest hit of the
+// first stride that has one, which is the sequential scan's answer; pred
+// must not change memory.  What changes one clause after another (the SUB
+// actions) is the group's first lane's; what touches every clause of a list
+// alike (staging, marks, counts) is shared out, a clause to a lane;
+// group_sync orders the writes before the group's next reads of the
+// variable's LDS copy.
+template <class P>
+PF_HD u32 group_first(u32 n, u32 gl, u32 G, P pred) {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (G > 1) {
+    const u32 g0 = (threadIdx.x & 63) - gl;
+    const u64 gmask = (G >= 64 ? ~0ull : ((1ull << G) - 1)) << g0;
+    for (u32 j0 = 0; j0 < n; j0 += G) {
+      const u32 j = j0 + gl;
+      const bool hit = j < n && pred(j);
+      const u64 m = __ballot(hit) & gmask;
+      if (m) return j0 + (u32)(__ffsll((long long)m) - 1) - g0;
+    }
+    return n;
+  }
+#endif
+  for (u32 j = 0; j < n; j++)
+    if (pred(j)) return j;
+  return n;
+}
+PF_HD void group_sync() {
+#ifdef __HIP_DEVICE_COMPILE__
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#endif
+}
+// the lowest j in [from, n) with pred(j), n if none (as group_first)
+template <class P>
+PF_HD u32 group_first_from(u32 from, u32 n, u32 gl, u32 G, P pred) {
+  if (from >= n) return n;
+  return from + group_first(n - from, gl, G, [&](u32 j) { return pred(from + j); });
+}
+// reductions over the G lanes of a group (G a power of two, groups aligned)
+PF_HD u32 group_min(u32 x, u32 G) {
+#ifdef __HIP_DEVICE_COMPILE__
+  for (u32 d = 1; d < G; d <<= 1) x = min(x, (u32)__shfl_xor(x, d, 64));
+#endif
+  return x;
+}
+PF_HD u32 group_sum(u32 x, u32 G) {
+#ifdef __HIP_DEVICE_COMPILE__
+  for (u32 d = 1; d < G; d <<= 1) x += (u32)__shfl_xor(x, d, 64);
+#endif
+  return x;
+}
+// exclusive prefix sum over the group's lanes; *total gets the group's sum
+PF_HD u32 group_excl_scan(u32 x, u32 gl, u32 G, u32* total) {
+#ifdef __HIP_DEVICE_COMPILE__
+  u32 y = x;
+  for (u32 d = 1; d < G; d <<= 1) {
+    const u32 t = (u32)__shfl_up(y, d, 64);
+    if (gl >= d) y += t;
+  }
+  *total = (u32)__shfl(y, (int)((threadIdx.x & 63) - gl + G - 1), 64);
+  return y - x;
+#else
+  *total = x;
+  return 0;
+#endif
+}
+PF_HD bool group_any(bool x, u32 gl, u32 G) {
+#ifdef __HIP_DEVICE_COMPILE__
+  if (G > 1) {
+    const u64 gmask = (G >= 64 ? ~0ull : ((1ull << G) - 1)) << ((threadIdx.x & 63) - gl);
+    return (__ballot(x) & gmask) != 0;
+  }
+#endif
+  return x;
+}
+
 // ---------------------------------------------------------------- clause access
 struct CL {
   u32* l;
@@ -140,30 +220,41 @@ PF_HD u32 lview_words(const DB& db, u32 v) {
   return n;
 }
 PF_HD u64 lview_bound(u32 nlists, u64 sizes) { return 2 + 3 * (u64)nlists + sizes; }
-// copies the lists of v into w[0, cap); false (w partly written) when they
-// do not fit
-PF_HD bool lview_stage(const DB& db, u32 v, u32* w, u32 cap, LView& lv) {
+// Copies the lists of v into w[0, cap); false (w partly written) when they
+// do not fit.  On a group the entries are shared out, a clause to a lane,
+// and a prefix sum over the lanes places the records: the three dependent
+// loads of an entry (handle, header, literals) are waited for once per G
+// entries instead of once per entry, which is what a variable's staging
+// costs (latency, not bytes).
+PF_HD bool lview_stage(const DB& db, u32 v, u32* w, u32 cap, LView& lv, u32 gl = 0, u32 G = 1) {
   const u32 p = V2L(v);
   const OLV a = olist(db, p), b = olist(db, NEGL(p));
-  u32 at = 2 + a.n + b.n;
+  const u32 nt = a.n + b.n;
+  u32 at = 2 + nt;
   if ((u64)at > cap) return false;
-  w[0] = a.n;
-  w[1] = b.n;
-  for (u32 s = 0; s < 2; s++) {
-    const OLV ol = s ? b : a;
-    u32* offs = w + 2 + (s ? a.n : 0);
-    for (u32 i = 0; i < ol.n; i++) {
-      const u32 c = ol.r[i];
-      const u32 h = db.lits[c];
-      const u32 n = hdr_size(h);
-      if ((u64)at + 2 + n > cap) return false;
-      const u32* l = clits(db, c);
-      offs[i] = at;
-      w[at] = c;
-      w[at + 1] = h;
-      for (u32 q = 0; q < n; q++) w[at + 2 + q] = l[q];
-      at += 2 + n;
+  if (gl == 0) {
+    w[0] = a.n;
+    w[1] = b.n;
+  }
+  for (u32 i0 = 0; i0 < nt; i0 += G) {
+    const u32 i = i0 + gl;
+    u32 c = 0, h = 0, n = 0, need = 0, tot;
+    if (i < nt) {
+      c = i < a.n ? a.r[i] : b.r[i - a.n];
+      h = db.lits[c];
+      n = hdr_size(h);
+      need = 2 + n;
     }
+    const u32 r = at + group_excl_scan(need, gl, G, &tot);
+    if ((u64)at + tot > cap) return false;
+    if (i < nt) {
+      const u32* l = clits(db, c);
+      w[2 + i] = r;
+      w[r] = c;
+      w[r + 1] = h;
+      for (u32 q = 0; q < n; q++) w[r + 2 + q] = l[q];
+    }
+    at += tot;
   }
   lv = LView{w, p};
   return true;
@@ -172,7 +263,9 @@ PF_HD bool lview_stage(const DB& db, u32 v, u32* w, u32 cap, LView& lv) {
 // records hold the pool handle, the three header words and the literals;
 // w[0] and w[1] are the current sizes of the positive and the negative
 // list, w[2] and w[3] their first words (offset arrays), w[4] the first
-// record.  sview_commit writes back what changed.
+// record.  The header word holds the size now (bits 0-11), the staged size
+// (bits 12-23) and the flags, so that sview_commit finds the records
+// without reading the pool; it writes back what changed.
 struct SView {
   u32* w;
   u32 lit;
@@ -182,13 +275,14 @@ PF_HD OLV olist(const SView& v, u32 lit) {
   return lit == v.lit ? OLV{v.w + v.w[2], v.w[0]} : OLV{v.w + v.w[3], v.w[1]};
 }
 PF_HD u32 cid(const SView& v, u32 c) { return v.w[c]; }
-PF_HD u32 csize(const SView& v, u32 c) { return hdr_size(v.w[c + 1]); }
+constexpr u32 SV_MAX = 0xFFFu;  // largest clause an SView holds
+PF_HD u32 csize(const SView& v, u32 c) { return v.w[c + 1] & SV_MAX; }
 PF_HD u8 cflags(const SView& v, u32 c) { return hdr_flags(v.w[c + 1]); }
 PF_HD u32 csig(const SView& v, u32 c) { return v.w[c + 2]; }
 PF_HD u32 clbd(const SView& v, u32 c) { return v.w[c + 3]; }
 PF_HD u32* clits(const SView& v, u32 c) { return v.w + c + 4; }
 PF_HD void set_cflags(const SView& v, u32 c, u8 f) { v.w[c + 1] = (v.w[c + 1] & CL_MAX_SIZE) | ((u32)f << 24); }
-PF_HD void set_csize(const SView& v, u32 c, u32 n) { v.w[c + 1] = (v.w[c + 1] & ~CL_MAX_SIZE) | n; }
+PF_HD void set_csize(const SView& v, u32 c, u32 n) { v.w[c + 1] = (v.w[c + 1] & ~SV_MAX) | n; }
 PF_HD void set_csig(const SView& v, u32 c, u32 sig) { v.w[c + 2] = sig; }
 PF_HD void set_clbd(const SView& v, u32 c, u32 lbd) { v.w[c + 3] = lbd; }
 PF_HD CL clause(const SView& v, u32 c) { return CL{clits(v, c), csize(v, c)}; }
@@ -216,64 +310,77 @@ PF_HD u32 sview_words(const DB& db, u32 v) {
   return n;
 }
 PF_HD u64 sview_bound(u32 nlists, u64 sizes) { return 4 + (CL_HDR + 2) * (u64)nlists + sizes; }
-PF_HD bool sview_stage(const DB& db, u32 v, u32* w, u32 cap, SView& sv) {
+PF_HD bool sview_stage(const DB& db, u32 v, u32* w, u32 cap, SView& sv, u32 gl = 0, u32 G = 1) {
   const u32 p = V2L(v);
   const OLV a = olist(db, p), b = olist(db, NEGL(p));
-  u32 at = 4 + a.n + b.n;
+  const u32 nt = a.n + b.n;
+  u32 at = 4 + nt;
   if ((u64)at > cap) return false;
-  w[0] = a.n;
-  w[1] = b.n;
-  w[2] = 4;
-  w[3] = 4 + a.n;
-  for (u32 s = 0; s < 2; s++) {
-    const OLV ol = s ? b : a;
-    u32* offs = w + w[2 + s];
-    for (u32 i = 0; i < ol.n; i++) {
-      const u32 c = ol.r[i];
-      const u32* h = chead(db, c);
-      const u32 n = hdr_size(h[0]);
-      if ((u64)at + CL_HDR + 1 + n > cap) return false;
-      offs[i] = at;
-      w[at] = c;
-      for (u32 q = 0; q < CL_HDR + n; q++) w[at + 1 + q] = h[q];
-      at += CL_HDR + 1 + n;
+  if (gl == 0) {
+    w[0] = a.n;
+    w[1] = b.n;
+    w[2] = 4;
+    w[3] = 4 + a.n;
+  }
+  for (u32 i0 = 0; i0 < nt; i0 += G) {  // shared out as in lview_stage
+    const u32 i = i0 + gl;
+    u32 c = 0, h = 0, n = 0, need = 0, tot;
+    if (i < nt) {
+      c = i < a.n ? a.r[i] : b.r[i - a.n];
+      h = db.lits[c];
+      n = hdr_size(h);
+      need = CL_HDR + 1 + n;
     }
+    const u32 r = at + group_excl_scan(need, gl, G, &tot);
+    if ((u64)at + tot > cap || group_any(n > SV_MAX, gl, G)) return false;
+    if (i < nt) {
+      const u32* l = chead(db, c);
+      w[4 + i] = r;
+      w[r] = c;
+      w[r + 1] = (h & ~CL_MAX_SIZE) | (n << 12) | n;
+      for (u32 q = 1; q < CL_HDR + n; q++) w[r + 1 + q] = l[q];
+    }
+    at += tot;
   }
   sv = SView{w, p, db.assign};
   return true;
 }
-// writes back the changed clauses (walked in staging order: a record spans
-// the clause's size in the pool, which changes only here) and the lists
-// that lost entries
-PF_HD void sview_commit(const DB& db, const SView& v, u32 np0, u32 nn0) {
-  u32 at = 4 + np0 + nn0;
-  for (u32 i = 0; i < np0 + nn0; i++) {
-    const u32 c = v.w[at];
-    u32* h = chead(db, c);
-    const u32 n0 = hdr_size(h[0]);
-    const u32 hl = v.w[at + 1];
-    if (hdr_size(hl) != n0) {
-      const u32 n = hdr_size(hl);
-      for (u32 q = 0; q < n; q++) h[CL_HDR + q] = v.w[at + 4 + q];
+// writes back the changed clauses (every lane of the group walks the
+// records in staging order, each commits its share) and the lists that lost
+// entries
+PF_HD void sview_commit(const DB& db, const SView& v, u32 np0, u32 nn0, u32 gl = 0, u32 G = 1) {
+  const u32 nt = np0 + nn0;
+  u32 at = 4 + nt;
+  for (u32 i0 = 0; i0 < nt; i0 += G) {
+    u32 mine = 0;
+    for (u32 i = i0; i < nt && i < i0 + G; i++) {
+      if (i - i0 == gl) mine = at;
+      at += CL_HDR + 1 + ((v.w[at + 1] >> 12) & SV_MAX);
     }
-    if (hl != h[0]) h[0] = hl;
-    if (v.w[at + 2] != h[1]) h[1] = v.w[at + 2];
-    if (v.w[at + 3] != h[2]) h[2] = v.w[at + 3];
-    at += CL_HDR + 1 + n0;
+    if (!mine) continue;
+    const u32 hl = v.w[mine + 1], n = hl & SV_MAX;
+    u32* h = chead(db, v.w[mine]);
+    const u32 now = (hl & ~CL_MAX_SIZE) | n;
+    const u32 h0 = h[0], h1 = h[1], h2 = h[2];
+    if (n != ((hl >> 12) & SV_MAX))
+      for (u32 q = 0; q < n; q++) h[CL_HDR + q] = v.w[mine + 4 + q];
+    if (now != h0) h[0] = now;
+    if (v.w[mine + 2] != h1) h[1] = v.w[mine + 2];
+    if (v.w[mine + 3] != h2) h[2] = v.w[mine + 3];
   }
   for (u32 s = 0; s < 2; s++) {
     const u32 lit = v.lit | s, n = v.w[s];
     if (n == (s ? nn0 : np0)) continue;
     u32* r = db.ot_refs + db.ot_off[lit];
     const u32* offs = v.w + v.w[2 + s];
-    for (u32 j = 0; j < n; j++) r[j] = v.w[offs[j]];
-    db.ot_size[lit] = n;
+    for (u32 j = gl; j < n; j += G) r[j] = v.w[offs[j]];
+    if (gl == 0) db.ot_size[lit] = n;
   }
 }
 // writes the molten marks the searches changed back to the pool
-PF_HD void lview_commit(const DB& db, const LView& v) {
+PF_HD void lview_commit(const DB& db, const LView& v, u32 gl = 0, u32 G = 1) {
   const u32 n = v.w[0] + v.w[1];
-  for (u32 i = 0; i < n; i++) {
+  for (u32 i = gl; i < n; i += G) {
     const u32 r = v.w[2 + i];
     const u32 c = v.w[r];
     const u8 lf = hdr_flags(v.w[r + 1]), gf = cflags(db, c);
@@ -704,59 +811,6 @@ PF_HD bool selfsub_lits(u32 x, u32 fx, CL sm, CL lr) {
   return false;
 }
 // subsume.h:105-121: is 'cand' subsumed by an earlier entry of the list
-// Groups of G consecutive lanes of a wavefront may share one variable
-// (gl = 0..G-1 is the lane's place in its group; G = 1 is one lane per
-// variable).  group_first returns the lowest j in [0, n) with pred(j), n if
-// none: the group tests j = gl, gl + G, ... and takes the lowest hit of the
-// first stride that has one, which is the sequential scan's answer; pred
-// must not change memory.  The group's first lane does every write (the
-// SUB actions), group_sync orders those writes before the group's next
-// reads of the variable's LDS copy.
-template <class P>
-PF_HD u32 group_first(u32 n, u32 gl, u32 G, P pred) {
-#ifdef __HIP_DEVICE_COMPILE__
-  if (G > 1) {
-    const u32 g0 = (threadIdx.x & 63) - gl;
-    const u64 gmask = (G >= 64 ? ~0ull : ((1ull << G) - 1)) << g0;
-    for (u32 j0 = 0; j0 < n; j0 += G) {
-      const u32 j = j0 + gl;
-      const bool hit = j < n && pred(j);
-      const u64 m = __ballot(hit) & gmask;
-      if (m) return j0 + (u32)(__ffsll((long long)m) - 1) - g0;
-    }
-    return n;
-  }
-#endif
-  for (u32 j = 0; j < n; j++)
-    if (pred(j)) return j;
-  return n;
-}
-PF_HD void group_sync() {
-#ifdef __HIP_DEVICE_COMPILE__
-  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-#endif
-}
-// the lowest j in [from, n) with pred(j), n if none (as group_first)
-template <class P>
-PF_HD u32 group_first_from(u32 from, u32 n, u32 gl, u32 G, P pred) {
-  if (from >= n) return n;
-  return from + group_first(n - from, gl, G, [&](u32 j) { return pred(from + j); });
-}
-// reductions over the G lanes of a group (G a power of two, groups aligned)
-PF_HD u32 group_min(u32 x, u32 G) {
-#ifdef __HIP_DEVICE_COMPILE__
-  for (u32 d = 1; d < G; d <<= 1) x = min(x, (u32)__shfl_xor(x, d, 64));
-#endif
-  return x;
-}
-PF_HD u32 group_sum(u32 x, u32 G) {
-#ifdef __HIP_DEVICE_COMPILE__
-  for (u32 d = 1; d < G; d <<= 1) x += (u32)__shfl_xor(x, d, 64);
-#endif
-  return x;
-}
-// subsume.h:105-121: is 'cand' subsumed by an earlier entry of the list
 template <class D>
 PF_HD bool subsume_cand(const D& db, OLV ol, u32 end, u32 cand, SubLocal& sl, u32 gl = 0, u32 G = 1) {
   const u32 csz = csize(db, cand), csg = csig(db, cand);
@@ -803,7 +857,7 @@ PF_HD bool selfsubsume_cand(const D& db, u32 x, u32 fx, OLV ol, u32 cand, u32 p,
   return true;
 }
 // subsume.h:27-37
-PF_HD void update_ol(const DB& db, u32 lit) {
+PF_HD void update_ol(const DB& db, u32 lit, u32, u32) {
   u32* r = db.ot_refs + db.ot_off[lit];
   const u32 n = db.ot_size[lit];
   u32 j = 0;
@@ -814,17 +868,29 @@ PF_HD void update_ol(const DB& db, u32 lit) {
   }
   db.ot_size[lit] = j;
 }
-PF_HD void update_ol(const SView& v, u32 lit) {
+// on a group, G entries at a time: all are read before the kept ones move
+// down
+PF_HD void update_ol(const SView& v, u32 lit, u32 gl, u32 G) {
   const u32 s = lit == v.lit ? 0u : 1u;
   u32* r = v.w + v.w[2 + s];
   const u32 n = v.w[s];
-  u32 j = 0;
-  for (u32 i = 0; i < n; i++) {
-    const u32 c = r[i];
-    if (is_molten(v, c)) freeze(v, c);
-    else if (!is_deleted(v, c)) r[j++] = c;
+  u32 j = 0, tot;
+  for (u32 i0 = 0; i0 < n; i0 += G) {
+    const u32 i = i0 + gl;
+    u32 c = 0;
+    bool keep = false;
+    if (i < n) {
+      c = r[i];
+      if (is_molten(v, c)) freeze(v, c);
+      else keep = !is_deleted(v, c);
+    }
+    const u32 at = j + group_excl_scan(keep ? 1u : 0u, gl, G, &tot);
+    group_sync();
+    if (keep) r[at] = c;
+    j += tot;
   }
-  v.w[s] = j;
+  group_sync();
+  if (gl == 0) v.w[s] = j;
 }
 // subsume.h:144-179 + the list-size gate of elimination.cpp:121-124, for
 // elected variable v (index k in elected order)
@@ -849,14 +915,13 @@ PF_HD void sub_var(const D& db, const Options& o, u32 v, u32 k, const SubOut& ou
       if (out.vis.ulit[v] == p) np = 0;
       else nn = 0;
     }
-    if (gl == 0)
-      for (u32 q = 0; q < 2; q++) {
-        const OLV ol = olist(db, p | q);
-        for (u32 i = 0; i < ol.n; i++) {
-          const u32 c = ol.r[i];
-          if (!is_deleted(db, c) && sub_visible_unit(out.vis, k, clause(db, c))) set_deleted(db, c);
-        }
+    for (u32 q = 0; q < 2; q++) {
+      const OLV ol = olist(db, p | q);
+      for (u32 i = gl; i < ol.n; i += G) {
+        const u32 c = ol.r[i];
+        if (!is_deleted(db, c) && sub_visible_unit(out.vis, k, clause(db, c))) set_deleted(db, c);
       }
+    }
     group_sync();
   }
   if ((int)np > o.sub_limit || (int)nn > o.sub_limit) return;
@@ -878,7 +943,7 @@ PF_HD void sub_var(const D& db, const Options& o, u32 v, u32 k, const SubOut& ou
       selfsubsume_cand(db, p, n, olist(db, n), c, p, sl, o.lbd_tier1, gl, G);
       subsume_cand(db, poss, i, c, sl, gl, G);
     }
-    if (gl == 0) update_ol(db, p);
+    update_ol(db, p, gl, G);
     group_sync();
   }
   {
@@ -890,7 +955,7 @@ PF_HD void sub_var(const D& db, const Options& o, u32 v, u32 k, const SubOut& ou
       selfsubsume_cand(db, n, p, olist(db, p), c, p, sl, o.lbd_tier1, gl, G);
       subsume_cand(db, negs, i, c, sl, gl, G);
     }
-    if (gl == 0) update_ol(db, n);
+    update_ol(db, n, gl, G);
     group_sync();
   }
   if (gl) return;  // the group's first lane holds the units
@@ -927,14 +992,13 @@ struct SubSnap {
 };
 // D: the pool, or the variable's staged SView before its SUB run changes it
 template <class D>
-PF_HD void sub_snapshot_var(const D& db, u32 v, u32 k, const SubSnap& s) {
-  u32 e = s.base[k];
+PF_HD void sub_snapshot_var(const D& db, u32 v, u32 k, const SubSnap& s, u32 gl = 0, u32 G = 1) {
+  u32 base = s.base[k];
   for (u32 q = 0; q < 2; q++) {
     const OLV ol = olist(db, V2L(v) | q);
-    if (q == 0) s.np[k] = ol.n;
-    else s.nn[k] = ol.n;
-    for (u32 j = 0; j < ol.n; j++, e++) {
-      const u32 c = ol.r[j];
+    if (gl == 0) (q == 0 ? s.np : s.nn)[k] = ol.n;
+    for (u32 j = gl; j < ol.n; j += G) {
+      const u32 c = ol.r[j], e = base + j;
       if (!is_deleted(db, c)) s.owner[cid(db, c)] = k;  // live clauses have one elected owner
       s.ref[e] = cid(db, c);
       s.flg[e] = cflags(db, c);
@@ -942,6 +1006,7 @@ PF_HD void sub_snapshot_var(const D& db, u32 v, u32 k, const SubSnap& s) {
       s.sig[e] = csig(db, c);
       s.lbd[e] = clbd(db, c);
     }
+    base += ol.n;
   }
 }
 PF_HD void sub_restore_var(const DB& db, u32 v, u32 k, const SubSnap& s) {
@@ -990,15 +1055,13 @@ struct VeDecision {
   u32* ncls;      // resolvents of size > 1
   u32* nlits;     // their pool words (headers + literals)
   u32* nstack;    // eliminated-stack words
-  u32* scratch;   // per variable scratch (fan-in literals)
-  u32* scr_base;  // per variable start in scratch
 };
 
 template <class D>
-PF_HD u32 count_orgs(const D& db, OLV ol) {
+PF_HD u32 count_orgs(const D& db, OLV ol, u32 gl = 0, u32 G = 1) {
   u32 n = 0;
-  for (u32 i = 0; i < ol.n; i++) n += is_original(db, ol.r[i]);
-  return n;
+  for (u32 i = gl; i < ol.n; i += G) n += is_original(db, ol.r[i]);
+  return group_sum(n, G);
 }
 template <class D>
 PF_HD u32 count_lits_before(const D& db, OLV ol) {
@@ -1059,96 +1122,94 @@ PF_HD bool count_res(const D& db, const Options& o, u32 x, int clsbefore, OLV me
   return false;
 }
 template <class D>
-PF_HD void freeze_binaries(const D& db, OLV ol) {  // simplify.h:204-211
-  for (u32 i = 0; i < ol.n; i++) {
-    const u32 c = ol.r[i];
-    if (is_original(db, c) && csize(db, c) == 2) freeze(db, c);
-  }
-}
-// equivalence.h:89-131
+PF_HD bool org_binary(const D& db, u32 c) { return is_original(db, c) && csize(db, c) == 2; }
 template <class D>
-PF_HD u32 find_sfanin(const D& db, u32 gate_out, OLV ol) {
-  u32 imp = 0;
-  int nImps = 0;
-  for (u32 i = 0; i < ol.n; i++) {
+PF_HD void freeze_binaries(const D& db, OLV ol, u32 gl = 0, u32 G = 1) {  // simplify.h:204-211
+  for (u32 i = gl; i < ol.n; i += G) {
     const u32 c = ol.r[i];
-    if (is_original(db, c) && csize(db, c) == 2) {
-      const u32* l = clits(db, c);
-      imp = FLIP(l[0] ^ l[1] ^ gate_out);
-      melt(db, c);
-      nImps++;
-    }
-    if (nImps > 1) return 0;
+    if (org_binary(db, c) && is_molten(db, c)) freeze(db, c);
   }
-  return imp;
+  group_sync();
 }
+// the literal a binary clause of the list of dx implies when dx is true
 template <class D>
-PF_HD u32 find_equ_gate(const D& db, u32 p) {
+PF_HD u32 implied(const D& db, u32 c, u32 dx) {
+  const u32* l = clits(db, c);
+  return FLIP(l[0] ^ l[1] ^ dx);
+}
+// equivalence.h:89-131: the list of p holds exactly one original binary
+// clause and the list of -p its converse; both are melted
+template <class D>
+PF_HD u32 find_equ_gate(const D& db, u32 p, u32 gl = 0, u32 G = 1) {
   const u32 n = NEGL(p);
   const OLV poss = olist(db, p), negs = olist(db, n);
-  u32 first = find_sfanin(db, p, poss);
-  if (first) {
-    u32 second = n, def = first;
-    if (second < first) first = second, second = def;
-    for (u32 i = 0; i < negs.n; i++) {
+  u32 nb = 0, bin = 0;
+  for (u32 i = gl; i < poss.n; i += G)
+    if (org_binary(db, poss.r[i])) nb++, bin = poss.r[i];
+  if (group_sum(nb, G) == 1) {
+    bin = group_sum(nb ? bin : 0u, G);  // one lane has it
+    const u32 def = implied(db, bin, p), first = def < n ? def : n, second = def < n ? n : def;
+    const u32 j = group_first(negs.n, gl, G, [&](u32 i) {
       const u32 c = negs.r[i];
-      if (is_original(db, c) && csize(db, c) == 2) {
-        const u32* l = clits(db, c);
-        if (l[0] == first && l[1] == second) {
-          melt(db, c);
-          return def;
-        }
+      if (!org_binary(db, c)) return false;
+      const u32* l = clits(db, c);
+      return l[0] == first && l[1] == second;
+    });
+    if (j < negs.n) {
+      if (gl == 0) {
+        melt(db, bin);
+        melt(db, negs.r[j]);
       }
+      group_sync();
+      return def;
     }
   }
-  freeze_binaries(db, poss);
+  freeze_binaries(db, poss, gl, G);
   return 0;
 }
-// and.h:25-86; 'out' is per-variable scratch
+// and.h:25-86.  The gate's long clause holds -dx and the literals implied by
+// the original binary clauses of dx, all of them and no other.  A clause of
+// -dx with one literal more than there are binaries is that clause iff each
+// of its other literals is implied by some binary: its literals are
+// distinct, so as many binaries then imply as many different literals.
 template <class D>
-PF_HD bool find_ao_gate(const D& db, const Options& o, u32 dx, int nOrgCls, u32* out, int& nAddedCls,
-                        u32& nAddedLits) {
-  const u32 x = ABS(dx);
+PF_HD bool find_ao_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int& nAddedCls, u32& nAddedLits,
+                        u32 gl = 0, u32 G = 1) {
   const OLV it = olist(db, dx);
-  u32 nout = 0, sig = 0;
-  for (u32 i = 0; i < it.n; i++) {
-    const u32 c = it.r[i];
-    if (is_original(db, c) && csize(db, c) == 2) {
-      const u32* l = clits(db, c);
-      const u32 imp = FLIP(l[0] ^ l[1] ^ dx);
-      out[nout++] = imp;
-      sig |= MAPHASH(imp);
-      melt(db, c);
-    }
-  }
-  if (nout > 1) {
+  u32 nb = 0;
+  for (u32 i = gl; i < it.n; i += G) nb += org_binary(db, it.r[i]);
+  nb = group_sum(nb, G);
+  if (nb > 1) {
     const u32 f = FLIP(dx);
-    out[nout++] = f;
-    sig |= MAPHASH(f);
-    for (u32 i = 1; i < nout; i++) {  // ascending order (distinct literals)
-      const u32 t = out[i];
-      u32 j = i;
-      while (j > 0 && out[j - 1] > t) { out[j] = out[j - 1]; j--; }
-      out[j] = t;
-    }
     const OLV ot2 = olist(db, f);
-    for (u32 i = 0; i < ot2.n; i++) {
-      const u32 c = ot2.r[i];
-      if (!is_original(db, c) || csize(db, c) != nout || !sub_sig(csig(db, c), sig)) continue;
+    for (u32 from = 0; from < ot2.n; from++) {
+      from = group_first_from(from, ot2.n, gl, G, [&](u32 j) {
+        const u32 c = ot2.r[j];
+        return is_original(db, c) && csize(db, c) == nb + 1;
+      });
+      if (from == ot2.n) break;
+      const u32 c = ot2.r[from];
       const u32* l = clits(db, c);
-      bool eq = true;
-      for (u32 q = 0; q < nout && eq; q++) eq = (l[q] == out[q]);
-      if (!eq) continue;
-      melt(db, c);
-      nAddedCls = 0;
-      if (count_res(db, o, x, nOrgCls, it, ot2, nAddedCls, nAddedLits, true)) {
-        freeze(db, c);
-        break;
+      bool all = true;
+      for (u32 q = 0; q <= nb && all; q++) {
+        const u32 x = l[q];
+        if (x == f) continue;
+        bool hit = false;
+        for (u32 i = gl; i < it.n && !hit; i += G) hit = org_binary(db, it.r[i]) && implied(db, it.r[i], dx) == x;
+        all = group_any(hit, gl, G);
       }
-      return true;
+      if (!all) continue;
+      for (u32 i = gl; i < it.n; i += G)
+        if (org_binary(db, it.r[i])) melt(db, it.r[i]);
+      if (gl == 0) melt(db, c);
+      group_sync();
+      nAddedCls = 0;
+      if (!count_res(db, o, ABS(dx), nOrgCls, it, ot2, nAddedCls, nAddedLits, true, gl, G)) return true;
+      if (gl == 0) freeze(db, c);
+      break;
     }
   }
-  freeze_binaries(db, it);
+  freeze_binaries(db, it, gl, G);
   return false;
 }
 // ifthenelse.h:25-45: first (lowest id) live non-molten original ternary
@@ -1238,15 +1299,9 @@ PF_HD bool find_ite_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int
 // xor.h:31-43
 template <class D>
 PF_HD void freeze_arities(const D& db, OLV me, OLV other, u32 gl = 0, u32 G = 1) {
-  if (gl == 0) {
-    for (u32 i = 0; i < me.n; i++) {
-      const u32 c = me.r[i];
-      if (csize(db, c) > 2 && is_molten(db, c)) freeze(db, c);
-    }
-    for (u32 i = 0; i < other.n; i++) {
-      const u32 c = other.r[i];
-      if (csize(db, c) > 2 && is_molten(db, c)) freeze(db, c);
-    }
+  for (u32 i = gl; i < me.n + other.n; i += G) {
+    const u32 c = i < me.n ? me.r[i] : other.r[i - me.n];
+    if (csize(db, c) > 2 && is_molten(db, c)) freeze(db, c);
   }
   group_sync();
 }
@@ -1292,6 +1347,7 @@ PF_HD bool find_xor_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int
                          u32& nAddedLits, u32 gl = 0, u32 G = 1) {
   const u32 fx = FLIP(dx), v = ABS(dx);
   const OLV it = olist(db, dx), ot2 = olist(db, fx);
+  bool frozen = false;  // nothing is molten: a search that found no clause at all leaves nothing to freeze
   for (u32 i = 0; i < it.n; i++) {
     const u32 ci = it.r[i];
     if (!is_original(db, ci)) continue;
@@ -1302,12 +1358,13 @@ PF_HD bool find_xor_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int
     u32 kx = 0;
     while (kx < size && base[kx] != dx) kx++;
     if (kx == size) continue;  // not reached: the clause is in the list of dx
-    u32 parity = 0;
+    u32 parity = 0, found = 0;
     int itargets = 1 << arity;
-    while (--itargets && make_arity(db, parity, base, size, kx, gl, G)) {
-    }
-    if (itargets) freeze_arities(db, it, ot2, gl, G);
-    else {
+    while (--itargets && make_arity(db, parity, base, size, kx, gl, G)) found++;
+    if (itargets) {
+      if (!frozen || found) freeze_arities(db, it, ot2, gl, G);
+      frozen = true;
+    } else {
       if (gl == 0) melt(db, ci);
       group_sync();
       nAddedCls = 0;
@@ -1323,83 +1380,55 @@ PF_HD bool find_xor_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int
 // stack words written by toblivion / save_BN_gate (simplify.h:305-332,
 // equivalence.h:133-154): the originals of the side with fewer originals
 template <class D>
-PF_HD u32 stack_words(const D& db, OLV side) {
-  u32 w = 2;
-  for (u32 i = 0; i < side.n; i++) {
+PF_HD u32 stack_words(const D& db, OLV side, u32 gl = 0, u32 G = 1) {
+  u32 w = 0;
+  for (u32 i = gl; i < side.n; i += G) {
     const u32 c = side.r[i];
     if (is_original(db, c)) w += csize(db, c) + 1;
   }
-  return w;
+  return 2 + group_sum(w, G);
 }
-// bve.cpp:138-241, decision part, for elected variable v at index k, in
-// two parts: the pure, equivalence and AND/OR checks (ve_decide_gates) for
-// every elected variable, then the ITE and XOR checks and the resolvent
-// count (ve_decide_rest) for the variables the first part leaves open.
-// The first part of a failed substitution count (nAddedCls > 0 disables
-// the negative-side searches and the plain count) is carried in d.ncls[k].
+// bve.cpp:138-241, decision part, for elected variable v at index k: pure,
+// equivalence, AND/OR, ITE and XOR gates, then the plain resolvent count.
+// A failed substitution count (nAddedCls > 0) disables the searches on the
+// other side and the plain count.
+// D: the pool (DB) or the variable's lists staged in an LView
 template <class D>
-PF_HD void ve_write(const D& db, u32 k, const VeDecision& d, OLV side, u32 type, u32 def, int nAddedCls,
-                    u32 nAddedLits) {
-  d.type[k] = type;
-  d.def[k] = def;
-  const bool adds = (type == VT_RES || type == VT_SUBST) && nAddedCls;
-  d.ncls[k] = adds ? (u32)nAddedCls : 0;
-  d.nlits[k] = adds ? nAddedLits + CL_HDR * (u32)nAddedCls : 0;  // pool words
-  d.nstack[k] = type ? stack_words(db, side) : 0;
-}
-// returns false when the variable is left to ve_decide_rest
-template <class D>
-PF_HD bool ve_decide_gates(const D& db, const Options& o, u32 v, u32 k, const VeDecision& d) {
+PF_HD void ve_decide(const D& db, const Options& o, u32 v, u32 k, const VeDecision& d, u32 gl = 0, u32 G = 1) {
   const u32 p = V2L(v), n = NEGL(p);
   const OLV poss = olist(db, p), negs = olist(db, n);
-  const u32 pOrgs = count_orgs(db, poss), nOrgs = count_orgs(db, negs);
+  const u32 pOrgs = count_orgs(db, poss, gl, G), nOrgs = count_orgs(db, negs, gl, G);
   const OLV side = pOrgs > nOrgs ? negs : poss;
   u32 type = VT_NONE, def = 0;
   int nAddedCls = 0;
   u32 nAddedLits = 0;
   if (!pOrgs || !nOrgs) {
     type = VT_PURE;
-  } else if ((def = find_equ_gate(db, p)) != 0) {
+  } else if ((def = find_equ_gate(db, p, gl, G)) != 0) {
     type = VT_EQU;
   } else {
     const int nOrgCls = (int)(pOrgs + nOrgs);
-    u32* out = d.scratch + d.scr_base[k];
     if (nOrgCls > 2) {
-      if (find_ao_gate(db, o, n, nOrgCls, out, nAddedCls, nAddedLits)) type = VT_SUBST;
-      else if (!nAddedCls && find_ao_gate(db, o, p, nOrgCls, out, nAddedCls, nAddedLits)) type = VT_SUBST;
+      if (find_ao_gate(db, o, n, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
+      else if (!nAddedCls && find_ao_gate(db, o, p, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
     }
     if (!type && nOrgCls > 3) {
-      d.ncls[k] = (u32)nAddedCls;
-      return false;
+      if (find_ite_gate(db, o, p, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
+      else if (!nAddedCls && find_ite_gate(db, o, n, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
+      else if (find_xor_gate(db, o, p, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
+      else if (!nAddedCls && find_xor_gate(db, o, n, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
     }
-    if (!type && !nAddedCls && !count_res(db, o, v, nOrgCls, poss, negs, nAddedCls, nAddedLits, false))
+    if (!type && !nAddedCls && !count_res(db, o, v, nOrgCls, poss, negs, nAddedCls, nAddedLits, false, gl, G))
       type = VT_RES;
   }
-  ve_write(db, k, d, side, type, def, nAddedCls, nAddedLits);
-  return true;
-}
-// D: the pool (DB) or the variable's lists staged in an LView
-template <class D>
-PF_HD void ve_decide_rest(const D& db, const Options& o, u32 v, u32 k, const VeDecision& d, u32 gl = 0,
-                          u32 G = 1) {
-  const u32 p = V2L(v), n = NEGL(p);
-  const OLV poss = olist(db, p), negs = olist(db, n);
-  const u32 pOrgs = count_orgs(db, poss), nOrgs = count_orgs(db, negs);
-  const OLV side = pOrgs > nOrgs ? negs : poss;
-  const int nOrgCls = (int)(pOrgs + nOrgs);
-  u32 type = VT_NONE;
-  int nAddedCls = (int)d.ncls[k];
-  u32 nAddedLits = 0;
-  if (find_ite_gate(db, o, p, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
-  else if (!nAddedCls && find_ite_gate(db, o, n, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
-  else if (find_xor_gate(db, o, p, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
-  else if (!nAddedCls && find_xor_gate(db, o, n, nOrgCls, nAddedCls, nAddedLits, gl, G)) type = VT_SUBST;
-  if (!type && !nAddedCls && !count_res(db, o, v, nOrgCls, poss, negs, nAddedCls, nAddedLits, false, gl, G))
-    type = VT_RES;
-  if (gl == 0) ve_write(db, k, d, side, type, 0, nAddedCls, nAddedLits);
-}
-PF_HD void ve_decide(const DB& db, const Options& o, u32 v, u32 k, const VeDecision& d) {
-  if (!ve_decide_gates(db, o, v, k, d)) ve_decide_rest(db, o, v, k, d);
+  const u32 nstack = type ? stack_words(db, side, gl, G) : 0;
+  if (gl) return;
+  const bool adds = (type == VT_RES || type == VT_SUBST) && nAddedCls;
+  d.type[k] = type;
+  d.def[k] = def;
+  d.ncls[k] = adds ? (u32)nAddedCls : 0;
+  d.nlits[k] = adds ? nAddedLits + CL_HDR * (u32)nAddedCls : 0;  // pool words
+  d.nstack[k] = nstack;
 }
 
 // unit records appended by VE / BCP: (elected index, sequence, literal)
@@ -1440,23 +1469,27 @@ PF_HD u32 save_witness(const DB& db, u32 w, u32* st) {
 }
 // writes the eliminated-stack records of toblivion / save_BN_gate
 template <class D>
-PF_HD void save_side(const D& view, const DB& db, u32 p, u32 pOrgs, u32 nOrgs, u32* st) {
+PF_HD void save_side(const D& view, const DB& db, u32 p, u32 pOrgs, u32 nOrgs, u32* st, u32 gl = 0, u32 G = 1) {
   const u32 n = NEGL(p);
   const bool negside = pOrgs > nOrgs;
   const OLV side = olist(view, negside ? n : p);
   const u32 wit = negside ? n : p;
-  u32 w = 0;
-  for (u32 i = 0; i < side.n; i++) {
-    const u32 c = side.r[i];
-    if (is_original(view, c)) w += save_clause(view, db, c, wit, st + w);
+  u32 w = 0, tot;
+  for (u32 i0 = 0; i0 < side.n; i0 += G) {
+    const u32 i = i0 + gl, c = i < side.n ? side.r[i] : 0u;
+    const bool org = i < side.n && is_original(view, c);
+    const u32 at = w + group_excl_scan(org ? csize(view, c) + 1 : 0u, gl, G, &tot);
+    if (org) save_clause(view, db, c, wit, st + at);
+    w += tot;
   }
-  save_witness(db, negside ? p : n, st + w);
+  if (gl == 0) save_witness(db, negside ? p : n, st + w);
 }
-PF_HD void delete_lists(const DB& db, u32 p) {
+PF_HD void delete_lists(const DB& db, u32 p, u32 gl = 0, u32 G = 1) {
   for (u32 q = 0; q < 2; q++) {
     const OLV ol = olist(db, p | q);
-    for (u32 i = 0; i < ol.n; i++) set_deleted(db, ol.r[i]);
-    db.ot_size[p | q] = 0;
+    for (u32 i = gl; i < ol.n; i += G) set_deleted(db, ol.r[i]);
+    group_sync();  // every lane has read the size
+    if (gl == 0) db.ot_size[p | q] = 0;
   }
 }
 // equivalence.h:25-43: substitute def for dx in clause c (kept sorted);
@@ -1496,36 +1529,49 @@ struct VeApply {
 // L: where the variable's lists and clauses are read: the pool (DB), or a
 // staged LView for the resolvent path (which changes none of them until it
 // deletes the lists; the EQU path rewrites its clauses and reads the pool)
+// On a group the resolvent pairs (and the clauses of an EQU substitution)
+// are shared out in order, G at a time; prefix sums over the lanes give each
+// its clause index, pool words and place in the event sequence, so what is
+// written equals one lane's walk over the pairs.
 template <class L>
-PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d, const VeApply& a) {
+PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d, const VeApply& a, u32 gl = 0,
+                    u32 G = 1) {
   const u32 type = d.type[k];
   if (!type) return;
   const u32 p = V2L(v), n = NEGL(p);
   const OLV poss = olist(lv, p), negs = olist(lv, n);
-  const u32 pOrgs = count_orgs(lv, poss), nOrgs = count_orgs(lv, negs);
+  const u32 pOrgs = count_orgs(lv, poss, gl, G), nOrgs = count_orgs(lv, negs, gl, G);
   const u32 sbase = a.stack0 + a.stack_base[k];
   if (sbase + d.nstack[k] > a.stack_cap) {
-    at_add(a.error, 1u);
+    if (gl == 0) at_add(a.error, 1u);
     return;
   }
   u32* st = a.stack + sbase;
-  u32 seq = 0;
+  u32 seq = 0, tot;
   if (type == VT_EQU) {
-    save_side(db, db, p, pOrgs, nOrgs, st);
+    save_side(db, db, p, pOrgs, nOrgs, st, gl, G);
+    group_sync();
     // equivalence.h:45-87
     const u32 def = d.def[k], def_f = FLIP(def);
     for (u32 q = 0; q < 2; q++) {
-      const OLV ol = q == 0 ? negs : poss;
+      const OLV ol = q == 0 ? olist(db, n) : olist(db, p);
       const u32 dx = q == 0 ? n : p;
       const u32 sub = q == 0 ? def_f : def;  // replacement literal
-      for (u32 i = 0; i < ol.n; i++) {
-        const u32 c = ol.r[i];
-        if (is_learnt(db, c) || is_molten(db, c) || has_lit(clause(db, c), FLIP(sub))) set_deleted(db, c);
-        else if (is_original(db, c)) {
-          const u32 unit = substitute_clause(db, dx, c, sub);
-          if (unit) push_unit(a.units, k, seq++, unit);
-          else push_proof(a.proof, k, seq++, PR_ADD, c);
+      for (u32 i0 = 0; i0 < ol.n; i0 += G) {
+        const u32 i = i0 + gl, c = i < ol.n ? ol.r[i] : 0u;
+        bool line = false;
+        u32 unit = 0;
+        if (i < ol.n) {
+          if (is_learnt(db, c) || is_molten(db, c) || has_lit(clause(db, c), FLIP(sub))) set_deleted(db, c);
+          else if (is_original(db, c)) {
+            unit = substitute_clause(db, dx, c, sub);
+            line = true;
+          }
         }
+        const u32 at = seq + group_excl_scan(line ? 1u : 0u, gl, G, &tot);
+        if (unit) push_unit(a.units, k, at, unit);
+        else if (line) push_proof(a.proof, k, at, PR_ADD, c);
+        seq += tot;
       }
     }
   } else {
@@ -1539,48 +1585,52 @@ PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d
       if (olist(lv, dx).n > olist(lv, fx).n) { dx = n; fx = p; }
       const OLV me = olist(lv, dx), other = olist(lv, fx);
       u32 cid = a.cls0 + a.cls_base[k], lpos = a.lit0 + a.lit_base[k];
-      for (u32 i = 0; i < me.n; i++) {
-        const u32 ci = me.r[i];
-        if (!is_original(lv, ci)) continue;
-        const bool ma = is_molten(lv, ci);
-        const CL A = clause(lv, ci);
-        for (u32 j = 0; j < other.n; j++) {
-          const u32 cj = other.r[j];
-          if (!is_original(lv, cj)) continue;
-          if (substitute && ma == is_molten(lv, cj)) continue;
-          const CL B = clause(lv, cj);
-          const u32 len = merge_len(v, A, B);
-          if (!len) {
-            // tautology, or a unit resolvent of two literals (len counts
-            // duplicates once; a length of 0 only arises from a tautology)
-            continue;
-          }
-          if (len == 1) {
-            u32 one[2];
-            merge_out(v, A, B, one);
-            push_unit(a.units, k, seq++, one[0]);
-            continue;
-          }
-          if (cid >= a.cls_cap || lpos + CL_HDR + len > a.lit_cap) {
-            at_add(a.error, 1u);
-            return;
-          }
-          u32* h = db.lits + lpos;
-          merge_out(v, A, B, h + CL_HDR);
-          h[0] = make_hdr(len, F_ADDED);
-          h[1] = calc_sig(h + CL_HDR, len);
-          h[2] = 0;
-          db.c_off[cid] = lpos;
-          push_proof(a.proof, k, seq++, PR_ADD, lpos);
-          cid++;
-          lpos += CL_HDR + len;
+      const u32 np = me.n * other.n;
+      u32 i = gl / other.n, j = gl % other.n;  // pair q = gl, then G further each time
+      const u32 di = G / other.n, dj = G % other.n;
+      for (u32 q0 = 0; q0 < np; q0 += G) {
+        u32 len = 0, ci = 0, cj = 0;
+        if (q0 + gl < np) {
+          ci = me.r[i];
+          cj = other.r[j];
+          // a length of 0 is a tautology
+          if (is_original(lv, ci) && is_original(lv, cj) && !(substitute && is_molten(lv, ci) == is_molten(lv, cj)))
+            len = merge_len(v, clause(lv, ci), clause(lv, cj));
         }
+        // lines and units in the low half, clauses in the high half
+        const u32 e = group_excl_scan((len ? 1u : 0u) | (len > 1 ? 0x10000u : 0u), gl, G, &tot);
+        u32 wtot;
+        const u32 lp = lpos + group_excl_scan(len > 1 ? CL_HDR + len : 0u, gl, G, &wtot);
+        if (len == 1) {
+          u32 one[2];
+          merge_out(v, clause(lv, ci), clause(lv, cj), one);
+          push_unit(a.units, k, seq + (e & 0xFFFFu), one[0]);
+        } else if (len > 1) {
+          const u32 ic = cid + (e >> 16);
+          if (ic >= a.cls_cap || lp + CL_HDR + len > a.lit_cap) {
+            at_add(a.error, 1u);
+          } else {
+            u32* h = db.lits + lp;
+            merge_out(v, clause(lv, ci), clause(lv, cj), h + CL_HDR);
+            h[0] = make_hdr(len, F_ADDED);
+            h[1] = calc_sig(h + CL_HDR, len);
+            h[2] = 0;
+            db.c_off[ic] = lp;
+            push_proof(a.proof, k, seq + (e & 0xFFFFu), PR_ADD, lp);
+          }
+        }
+        seq += tot & 0xFFFFu;
+        cid += tot >> 16;
+        lpos += wtot;
+        i += di;
+        j += dj;
+        if (j >= other.n) j -= other.n, i++;
       }
     }
-    save_side(lv, db, p, pOrgs, nOrgs, st);
-    delete_lists(db, p);
+    save_side(lv, db, p, pOrgs, nOrgs, st, gl, G);
+    delete_lists(db, p, gl, G);
   }
-  db.vstate[v] = VS_MELTED;
+  if (gl == 0) db.vstate[v] = VS_MELTED;
 }
 
 // ---------------------------------------------------------------- BCE (elimination.cpp:131-167)

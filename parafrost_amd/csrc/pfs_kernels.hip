@@ -1501,6 +1501,17 @@ __device__ inline u32 lv_class(u32 need, u32 cap) {
   return q;
 }
 __device__ inline u32 lv_class_lanes(u32 q) { return q < LV_CLASSES - 1 ? 64u >> q : 64u; }
+// The least class of a launch over n variables: where they would leave
+// lanes idle, each takes the largest group that keeps the launch within
+// LV_FILL rounds of the resident wavefronts.  A variable's chain of
+// dependent loads and LDS reads is then walked G entries at a time, and the
+// chunks spread over the CUs.  Measured per launch (ve_decide_k, sub_k): 45
+// elected variables 290 + 155 -> 48 + 27 us; 3,206: 350 + 260 -> 86 + 51 us;
+// 43,123: 596 + 303 -> 220 + 151 us (LV_FILL 1 / 2 / 4 / 8: 348 / 286 / 220 /
+// 178 us there, 119 / 116 / 141 / 219 us for 12,314 variables).
+#ifndef LV_FILL
+#define LV_FILL 4
+#endif
 __global__ void lv_bounds_k(const u32* keys, u32 n, u32* starts) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n && (i == 0 || keys[i] != keys[i - 1])) starts[keys[i]] = i;
@@ -1562,11 +1573,18 @@ __device__ inline void lv_chunks(const u32* work, u32 n, u32 cap, u32* lds, F f)
   }
 }
 // LDS of each one-wavefront workgroup of the staged launches, and their
-// workgroups: as many as fit the CUs
+// workgroups: as many as fit the CUs, at most one per variable (a chunk of
+// the upper classes holds one: a workgroup per 64 variables left the chunks
+// of a small formula to one wavefront)
 #ifndef VR_LDS
 #define VR_LDS PV_LDS
 #endif
 constexpr u32 LV_BLOCKS = 256 * (160 * 1024 / VR_LDS);
+static u32 lv_floor(u32 n) {
+  u32 c = 0;
+  while (c < LV_CLASSES - 2 && ((u64)n << (c + 1)) <= (u64)LV_FILL * LV_BLOCKS * 64) c++;
+  return c;
+}
 
 // VE decisions in two launches: the gate checks (pure, equivalence,
 // AND/OR) for every elected variable, then, staged, the variables they
@@ -1579,39 +1597,35 @@ constexpr u32 LV_BLOCKS = 256 * (160 * 1024 / VR_LDS);
 #ifndef VE_CLASS_BUMP
 #define VE_CLASS_BUMP 1
 #endif
-__global__ void ve_class_k(DB db, const u32* pv, u32 n, const u32* order, u32* work, const u32* lsum, u32 cap) {
+__global__ void ve_class_k(DB db, const u32* pv, u32 n, const u32* order, u32* work, const u32* lsum, u32 cap,
+                           u32 least) {
   const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const u32 k = order ? order[t] : t;
   const u32 p = V2L(pv[k]);
   const u64 b = lview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
   u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
-  if (c < LV_CLASSES - 1) c = min(c + VE_CLASS_BUMP, LV_CLASSES - 2);
+  if (c < LV_CLASSES - 1) c = max(least, min(c + VE_CLASS_BUMP, LV_CLASSES - 2));
   work[LV_WORK_HDR + t] = LV_CLASSES - 1 - c;
   work[LV_WORK_HDR + n + t] = k;
 }
-// every elected variable on an LDS copy of its lists: the gate checks
-// (pure, equivalence, AND/OR) by the group's first lane, then, for the
-// variables they leave open, the ITE and XOR searches and the resolvent
-// count shared by the group (the checks read each clause of the lists
-// once, into LDS, instead of once per check from the pool)
+// every elected variable on an LDS copy of its lists (the checks read each
+// clause of the lists once, into LDS, instead of once per check from the
+// pool), the gate checks, searches and resolvent count shared by the group
+// (LV_FILL: a few lanes or all 64 per variable).  Bound by chains of LDS
+// reads per variable, so what counts is how many of them one lane walks.
 __global__ void ve_decide_k(DB db, Options o, const u32* pv, VeDecision d, const u32* work, u32 n, u32 cap) {
   extern __shared__ u32 lds[];
   lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
     const u32 v = pv[k];
     LView lv;
-    // every lane of the group stages the same words; the writes are the
-    // first lane's
-    if (w && lview_stage(db, v, w, slice, lv)) {
+    if (w && lview_stage(db, v, w, slice, lv, gl, G)) {
       group_sync();
-      u32 open = 0;
-      if (gl == 0) open = ve_decide_gates(lv, o, v, k, d) ? 0u : 1u;
-      open = __shfl(open, (int)((threadIdx.x & 63) - gl), 64);
-      group_sync();  // the first lane's marks in the copy are seen by the group
-      if (open) ve_decide_rest(lv, o, v, k, d, gl, G);
-      if (gl == 0) lview_commit(db, lv);
+      ve_decide(lv, o, v, k, d, gl, G);
+      group_sync();
+      lview_commit(db, lv, gl, G);
     } else if (gl == 0) {
-      if (!ve_decide_gates(db, o, v, k, d)) ve_decide_rest(db, o, v, k, d);
+      ve_decide(db, o, v, k, d);
     }
   });
 }
@@ -1620,22 +1634,23 @@ void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeD
   if (!n) return;
   const u32 cap = VR_LDS / 4;
   fill_u32(work, n, LV_WORK_HDR, st);
-  KLAUNCH(ve_class_k, grid_for(n, 256), 256, st, db, pv, n, order, work, lsum, cap);
+  KLAUNCH(ve_class_k, grid_for(n, 256), 256, st, db, pv, n, order, work, lsum, cap, lv_floor(n));
   lv_sort(work, n, tmp, st);
-  KLAUNCH_LDS(ve_decide_k, std::min<u32>(grid_for(n, VB), LV_BLOCKS), VB, VR_LDS, st, db, o, pv, d, work, n, cap);
+  KLAUNCH_LDS(ve_decide_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, o, pv, d, work, n, cap);
 }
 // SUB, staged as the VE searches (the class of a variable from the words of
 // its SView, raised by SUB_CLASS_BUMP)
 #ifndef SUB_CLASS_BUMP
 #define SUB_CLASS_BUMP 0
 #endif
-__global__ void sub_class_k(DB db, const u32* pv, const u32* idx, u32 n, u32* work, const u32* lsum, u32 cap) {
+__global__ void sub_class_k(DB db, const u32* pv, const u32* idx, u32 n, u32* work, const u32* lsum, u32 cap,
+                            u32 least) {
   const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const u32 k = idx ? idx[t] : t, p = V2L(pv[k]);
   const u64 b = sview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
   u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
-  if (c < LV_CLASSES - 1) c = min(c + SUB_CLASS_BUMP, LV_CLASSES - 2);
+  if (c < LV_CLASSES - 1) c = max(least, min(c + SUB_CLASS_BUMP, LV_CLASSES - 2));
   work[LV_WORK_HDR + t] = LV_CLASSES - 1 - c;
   work[LV_WORK_HDR + n + t] = k;
 }
@@ -1648,14 +1663,14 @@ __global__ void sub_k(DB db, Options o, const u32* pv, const u32* work, u32 n, u
   lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
     const u32 v = pv[k];
     SView sv;
-    // every lane of the group stages the same words, so the outcome is the
-    // group's; the scans are shared, the writes are the first lane's
-    if (w && sview_stage(db, v, w, slice, sv)) {
+    if (w && sview_stage(db, v, w, slice, sv, gl, G)) {
+      group_sync();
       const u32 np0 = sv.w[0], nn0 = sv.w[1];
-      if (take_snap && gl == 0) sub_snapshot_var(sv, v, k, snap);
+      if (take_snap) sub_snapshot_var(sv, v, k, snap, gl, G);
       group_sync();
       sub_var(sv, o, v, k, out, gl, G);
-      if (gl == 0) sview_commit(db, sv, np0, nn0);
+      group_sync();
+      sview_commit(db, sv, np0, nn0, gl, G);
     } else if (gl == 0) {
       if (take_snap) sub_snapshot_var(db, v, k, snap);
       sub_var(db, o, v, k, out);
@@ -1667,26 +1682,30 @@ void k_sub(const DB& db, const Options& o, const u32* pv, const u32* idx, u32 n,
   if (!n) return;
   const u32 cap = VR_LDS / 4;
   fill_u32(work, n, LV_WORK_HDR, st);
-  KLAUNCH(sub_class_k, grid_for(n, 256), 256, st, db, pv, idx, n, work, lsum, cap);
+  KLAUNCH(sub_class_k, grid_for(n, 256), 256, st, db, pv, idx, n, work, lsum, cap, lv_floor(n));
   lv_sort(work, n, tmp, st);
-  KLAUNCH_LDS(sub_k, std::min<u32>(grid_for(n, VB), LV_BLOCKS), VB, VR_LDS, st, db, o, pv, work, n, cap, out,
+  KLAUNCH_LDS(sub_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, o, pv, work, n, cap, out,
               snap ? *snap : SubSnap{}, snap ? 1u : 0u);
 }
 // VE execution, staged as the searches: the resolvent path reads the
 // variable's lists from LDS; EQU substitutions (which rewrite their clauses
-// in place) take the last class and work on the pool; variables VE keeps
-// are not placed
+// in place) work on the pool, EQU_CLASS lanes' worth or more each; variables
+// VE keeps are not placed
+constexpr u32 EQU_CLASS = 3;
 __global__ void ve_apply_class_k(DB db, const u32* pv, u32 n, const u32* type, u32* work, const u32* lsum,
-                                 u32 cap) {
+                                 u32 cap, u32 least) {
   const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   u32 key = LV_CLASSES;
-  if (type[k] == VT_EQU) {
-    key = 0;
-  } else if (type[k]) {
-    const u32 p = V2L(pv[k]);
-    const u64 b = lview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
-    key = LV_CLASSES - 1 - lv_class((u32)min(b, (u64)cap + 1), cap);
+  if (type[k]) {
+    u32 c = EQU_CLASS;
+    if (type[k] != VT_EQU) {
+      const u32 p = V2L(pv[k]);
+      const u64 b = lview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
+      c = lv_class((u32)min(b, (u64)cap + 1), cap);
+    }
+    if (c < LV_CLASSES - 1) c = max(c, least);
+    key = LV_CLASSES - 1 - c;
   }
   work[LV_WORK_HDR + k] = key;
   work[LV_WORK_HDR + n + k] = k;
@@ -1694,11 +1713,14 @@ __global__ void ve_apply_class_k(DB db, const u32* pv, u32 n, const u32* type, u
 __global__ void ve_apply_k(DB db, const u32* pv, VeDecision d, VeApply a, const u32* work, u32 n, u32 cap) {
   extern __shared__ u32 lds[];
   lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
-    if (gl) return;  // one lane per variable
     const u32 v = pv[k];
     LView lv;
-    if (w && d.type[k] != VT_EQU && lview_stage(db, v, w, slice, lv)) ve_apply(lv, db, v, k, d, a);
-    else ve_apply(db, db, v, k, d, a);
+    if (w && d.type[k] != VT_EQU && lview_stage(db, v, w, slice, lv, gl, G)) {
+      group_sync();
+      ve_apply(lv, db, v, k, d, a, gl, G);
+    } else {
+      ve_apply(db, db, v, k, d, a, gl, G);
+    }
   });
 }
 void k_ve_apply(const DB& db, const u32* pv, u32 n, const VeDecision& d, const VeApply& a, u32* work,
@@ -1706,9 +1728,9 @@ void k_ve_apply(const DB& db, const u32* pv, u32 n, const VeDecision& d, const V
   if (!n) return;
   const u32 cap = VR_LDS / 4;
   fill_u32(work, n, LV_WORK_HDR, st);
-  KLAUNCH(ve_apply_class_k, grid_for(n, 256), 256, st, db, pv, n, d.type, work, lsum, cap);
+  KLAUNCH(ve_apply_class_k, grid_for(n, 256), 256, st, db, pv, n, d.type, work, lsum, cap, lv_floor(n));
   lv_sort(work, n, tmp, st);
-  KLAUNCH_LDS(ve_apply_k, std::min<u32>(grid_for(n, VB), LV_BLOCKS), VB, VR_LDS, st, db, pv, d, a, work, n, cap);
+  KLAUNCH_LDS(ve_apply_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, pv, d, a, work, n, cap);
 }
 __global__ void bce_k(DB db, Options o, const u32* pv, const u32* type, u32 n, u32* words,
                       const u32* base, u32* stack, bool count, const u32* order) {
