@@ -323,7 +323,8 @@ pfs_status pfs_kernel_stats(pfs_ctx* ctx, uint32_t i, const char** name, double*
  * candidates (option "autotune": the first call of a formula class with at
  * least 2^20 clauses measures every tile, lane count and reservation not
  * set by "otptile" / "mislanes" / "mislds"; later calls of the class reuse
- * the fastest).  Replaces the reference's launch tuner
+ * the fastest; where it is neither tuned nor set the lane count reads 1 and
+ * the steps take as many lanes as the candidates leave idle).  Replaces the reference's launch tuner
  * (src/gpu/grid.cuh:137-229); results do not depend on the shapes. */
 pfs_status pfs_launch_shape(pfs_ctx* ctx, int32_t* otp_tile_log2, int32_t* mis_lds, int32_t* mis_lanes,
                             int32_t* tuned);

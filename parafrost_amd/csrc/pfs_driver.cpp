@@ -1010,7 +1010,7 @@ bool Simplifier::lcve() {
   a.max_occurs = opt.lcve_max_occurs == INT32_MAX ? INF : (u32)opt.lcve_max_occurs;
   a.clause_max = opt.lcve_clause_max == INT32_MAX ? INF : (u32)opt.lcve_clause_max;
   k_lcve_classify(db, a, st_);
-  k_lcve_select(db, a, P<u32>(flag_), P<u32>(cand_), P<u32>(key_), sc, tmp_.p, st_);
+  k_lcve_select(db, a, P<u32>(flag_), P<u32>(cand_), P<u32>(key_), P<u32>(pos_), sc, tmp_.p, st_);
   u32 h[4];
   d2h(h, sc, 4, st_);
   d2h(h + 2, hard, 8, st_);
@@ -1028,42 +1028,43 @@ bool Simplifier::lcve() {
   if (ncand >= (1u << 30)) throw DeviceFail{"LCVE: too many candidates for the packed positions"};
   u32* resume = P<u32>(vsz_);  // free until SUB: where each scan goes on
   // worklists of undecided candidates (the selection buffers are free now);
-  // after the first pass over all candidates, passes are queued eight at a
-  // time with the list lengths kept on the device in a ring of three
+  // after the first pass over all candidates, passes are queued MIS_QUEUE at
+  // a time with the list lengths kept on the device in a ring of three
   // counters (sc[12..14]: pass p reads ring[p % 3], appends to
   // ring[(p + 1) % 3] and clears ring[(p + 2) % 3] for the next pass; sc[6]
-  // counts the passes that had work)
+  // counts the passes that had work).  A pass tries each of its candidates
+  // until it is decided, MIS_TRIES times at most, so one or two passes
+  // finish an election as a rule, and the ones queued cost 3 us each when
+  // there is nothing left.
+  constexpr u32 MIS_QUEUE = 2;
   u32* wl[2] = {P<u32>(flag_), P<u32>(score_)};
   u32* ring[3] = {sc + 12, sc + 13, sc + 14};
-  // the election from scratch with 'lds' bytes reserved per step
-  // workgroup and 'lanes' per candidate; sc[6] counts the worklist passes
-  // that had work
-  auto elect = [&](u32 lds, u32 lanes) {
-    fill_u32(P<u32>(pos_), NOPOS, (size_t)V_ + 1, st_);
-    k_lcve_positions(P<u32>(cand_), ncand, P<u32>(pos_), st_);
-    fill_u32(P<u32>(state_), 0, ncand, st_);
-    if (a.clause_max != INF) k_lcve_reject(P<u32>(cand_), ncand, P<u8>(cflag_), P<u32>(pos_), P<u32>(state_), st_);
-    fill_u32(P<u32>(key_), NOPOS, ncand, st_);  // the sort keys are consumed: blockers
-    fill_u32(resume, 0, ncand, st_);
-    fill_u32(sc + 4, 0, 3, st_);
-    fill_u32(sc + 12, 0, 3, st_);
-    if (!ncand) return;
-    k_mis_step(db, P<u32>(cand_), nullptr, ncand, P<u32>(pos_), P<u32>(state_), P<u32>(key_), resume, wl[0],
-               ring[0], lds, lanes, st_);
-    // the first batch of worklist passes is sized for every candidate (its
-    // grid is at the cap either way on large rounds); later batches for the
-    // list length read after the previous batch
-    u32 p = 0, bound = ncand;
-    while (bound) {
-      for (int b = 0; b < 8; b++, p++) {
-        k_mis_step_dev(db, P<u32>(cand_), wl[p & 1], ring[p % 3], bound, P<u32>(pos_), P<u32>(state_),
-                       P<u32>(key_), resume, wl[(p + 1) & 1], ring[(p + 1) % 3], sc + 6, ring[(p + 2) % 3], lds,
-                       lanes, st_);
-      }
-      if (p > ncand + 8) throw DeviceFail{"LCVE election did not converge"};
-      bound = read_u32(ring[p % 3]);
+  u32 p = 0;  // worklist passes queued
+  auto passes = [&](u32 bound, u32 lds, u32 lanes) {
+    for (u32 b = 0; b < MIS_QUEUE; b++, p++) {
+      k_mis_step_dev(db, P<u32>(cand_), wl[p & 1], ring[p % 3], bound, P<u32>(pos_), P<u32>(state_),
+                     P<u32>(key_), resume, wl[(p + 1) & 1], ring[(p + 1) % 3], sc + 6, ring[(p + 2) % 3], lds,
+                     lanes, st_);
     }
+    if (p > ncand + 8) throw DeviceFail{"LCVE election did not converge"};
   };
+  // the election from scratch with 'lds' bytes reserved per step workgroup
+  // and 'lanes' per candidate: the first pass (the sort keys are consumed:
+  // blockers) and the first batch of worklist passes, sized for every
+  // candidate; ring[p % 3] tells whether there is more to do
+  auto begin = [&](u32 lds, u32 lanes) {
+    p = 0;
+    k_mis_init(P<u32>(cand_), ncand, P<u8>(cflag_), a.clause_max != INF, P<u32>(pos_), P<u32>(state_), sc, st_);
+    if (!ncand) return;
+    k_mis_step(db, P<u32>(cand_), ncand, P<u32>(pos_), P<u32>(state_), P<u32>(key_), resume, wl[0], ring[0], lds,
+               lanes, st_);
+    passes(ncand, lds, lanes);
+  };
+  auto elect = [&](u32 lds, u32 lanes) {
+    begin(lds, lanes);
+    while (const u32 bound = read_u32(ring[p % 3])) passes(bound, lds, lanes);
+  };
+  u32 lanes = 1;
   if (tune_mis_ && ncand) {
     // the election is the same set whatever the shape (the
     // lexicographically first independent set is unique): each candidate
@@ -1093,7 +1094,7 @@ bool Simplifier::lcve() {
     if (opt.mis_lanes > 0) shapes.push_back({lds0, (u32)opt.mis_lanes});
     else
       for (u32 g : {1u, 2u, 4u, 8u}) shapes.push_back({lds0, g});
-    const u32 lanes = fastest(shapes).second;
+    lanes = fastest(shapes).second;
     shapes.clear();
     if (opt.mis_lds >= 0) shapes.push_back({lds0, lanes});
     else
@@ -1105,18 +1106,30 @@ bool Simplifier::lcve() {
     tune_store();
     used_lanes_ = tune_.mis_lanes;
     used_lds_ = tune_.mis_lds;
+    begin(pick.first, pick.second);
   } else {
     used_lds_ = lds_choice();
     used_lanes_ = lanes_choice();
-    elect((u32)used_lds_, (u32)used_lanes_);
+    // neither set nor tuned: by the number of candidates
+    lanes = opt.mis_lanes > 0 || tune_.mis ? (u32)used_lanes_ : mis_lanes_for(ncand);
+    begin((u32)used_lds_, lanes);
   }
-  fill_u32(sc, 0, 1, st_);
-  fill_u32(sc + 1, ncand, 1, st_);
-  k_mis_break(P<u32>(cand_), ncand, P<u8>(cflag_), P<u32>(state_), sc + 1, st_);
-  k_mis_collect(P<u32>(cand_), ncand, P<u32>(state_), 0, P<u32>(flag_), P<u32>(pv_), sc, tmp_.p, st_);
-  u32 w7[7];  // sc[0]: elected, sc[6]: worklist passes with work
-  d2h(w7, sc, sizeof(w7), st_);
-  stream_sync(st_);
+  // the elected variables collected behind the passes queued so far; the one
+  // read that brings their number also tells whether candidates were left
+  // undecided, which takes more passes and another collection
+  u32 w15[15];  // sc[0]: elected, sc[6]: worklist passes with work, sc[12..14]: the ring
+  while (true) {
+    k_mis_break(P<u32>(cand_), ncand, P<u8>(cflag_), P<u32>(state_), sc + 1, st_);
+    // the worklist still to be read must stay: the other one is free
+    k_mis_collect(P<u32>(cand_), ncand, P<u32>(state_), 0, wl[(p + 1) & 1], P<u32>(pv_), sc, tmp_.p, st_);
+    d2h(w15, sc, sizeof(w15), st_);
+    stream_sync(st_);
+    const u32 bound = ncand ? w15[12 + p % 3] : 0;
+    if (!bound) break;
+    fill_u32(sc + 1, ncand, 1, st_);
+    passes(bound, (u32)used_lds_, lanes);
+  }
+  const u32* w7 = w15;
   E_ = w7[0];
   rounds_.back().elected = E_;
   rounds_.back().mis_iterations = ncand ? 1 + w7[6] : 0;

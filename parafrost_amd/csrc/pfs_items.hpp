@@ -48,6 +48,7 @@ PF_HD u32 at_load(const u32* p) {
   return __atomic_load_n(p, __ATOMIC_RELAXED);
 #endif
 }
+PF_HD void at_store(u32* p, u32 v) { __atomic_store_n(p, v, __ATOMIC_RELAXED); }
 PF_HD u64 at_min64(u64* p, u64 v) {
 #if defined(__HIP_DEVICE_COMPILE__)
   return atomicMin((unsigned long long*)p, (unsigned long long)v);
@@ -528,9 +529,10 @@ PF_HD bool lcve_oversize(const DB& db, u32 v, u32 limit) {
   }
   return false;
 }
+// written through to where every XCD's loads of the same launch find it
 PF_HD void mis_decide(u32* state, u32* pw, u32 i, u32 v, u32 s) {
-  state[i] = s;
-  pw[v] = (i << 2) | s;
+  at_store(&pw[v], (i << 2) | s);
+  at_store(&state[i], s);
 }
 // ---------------------------------------------------------------- shared helpers
 PF_HD bool sub_sig(u32 A, u32 B) { return !(A & ~B); }  // simplify.h:84

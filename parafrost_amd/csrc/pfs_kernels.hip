@@ -1161,9 +1161,10 @@ __device__ unsigned long long lcve_classify_var(const DB& db, const LcveArgs& a,
 void k_lcve_classify(const DB& db, const LcveArgs& a, Stream* st) {
   KLAUNCH(lcve_classify_k, std::min(grid_for(db.nvars, ST), 2048u), ST, st, db, a);
 }
-__global__ void lcve_flag_k(DB db, LcveArgs a, u32* flag) {
+__global__ void lcve_flag_k(DB db, LcveArgs a, u32* flag, u32* pos) {
   const u32 v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v > db.nvars) return;
+  pos[v] = NOPOS;
   u32 f = 0;
   if (v && a.cflag[v]) f = (((u64)a.score[v] << 32) | v) < *a.hard;
   flag[v] = f;
@@ -1176,30 +1177,31 @@ __global__ void lcve_pack_k(DB db, LcveArgs a, const u32* flag, const u32* pos, 
   cand[i] = v;
   key[i] = a.score[v];
 }
-void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u32* key, u32* ncand,
+void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u32* key, u32* pos, u32* ncand,
                    void* tmp, Stream* st) {
   const size_t n = (size_t)db.nvars + 1;
-  KLAUNCH(lcve_flag_k, grid_for(n, 256), 256, st, db, a, flag_tmp);
+  KLAUNCH(lcve_flag_k, grid_for(n, 256), 256, st, db, a, flag_tmp, pos);
   scan_u32(flag_tmp, flag_tmp, n, ncand, tmp, st);
   KLAUNCH(lcve_pack_k, grid_for(n, 256), 256, st, db, a, flag_tmp, flag_tmp, cand, key);
 }
-// packed position and state (undecided) of each candidate, for mis_step
-__global__ void lcve_pos_k(const u32* cand, u32 n, u32* pos) {
+// The state of an election before its first step: each candidate's packed
+// position and state (undecided, or decided and not elected for the ones
+// passed over) and the counters (sc: [1] the break position, [4..6] and
+// [12..14] the passes' counts), in one launch.  The positions of variables
+// that are no candidates are NOPOS from lcve_flag_k.
+__global__ void mis_init_k(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) pos[cand[i]] = i << 2;
+  if (i == 0) {
+    sc[1] = n;
+    for (u32 q = 0; q < 3; q++) sc[4 + q] = 0, sc[12 + q] = 0;
+  }
+  if (i >= n) return;
+  const u32 v = cand[i], st = reject && cflag[v] == 4 ? 2u : 0u;
+  state[i] = st;
+  pos[v] = (i << 2) | st;
 }
-void k_lcve_positions(const u32* cand, u32 n, u32* pos, Stream* st) {
-  if (!n) return;
-  KLAUNCH(lcve_pos_k, grid_for(n, 256), 256, st, cand, n, pos);
-}
-__global__ void lcve_reject_k(const u32* cand, u32 n, const u8* cflag, u32* pos, u32* state) {
-  const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || cflag[cand[i]] != 4) return;
-  mis_decide(state, pos, i, cand[i], 2);
-}
-void k_lcve_reject(const u32* cand, u32 n, const u8* cflag, u32* pos, u32* state, Stream* st) {
-  if (!n) return;
-  KLAUNCH(lcve_reject_k, grid_for(n, 256), 256, st, cand, n, cflag, pos, state);
+void k_mis_init(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc, Stream* st) {
+  KLAUNCH(mis_init_k, std::max(1u, grid_for(n, 256)), 256, st, cand, n, cflag, reject, pos, state, sc);
 }
 // One election step by a group of G lanes per candidate (G a power of two,
 // groups aligned in the wavefront): the lanes share out the entries of the
@@ -1208,18 +1210,12 @@ void k_lcve_reject(const u32* cand, u32 n, const u8* cflag, u32* pos, u32* state
 // the candidate, else the earliest entry holding an undecided earlier
 // neighbour is its blocker's entry.  The outcome is the one-lane scan's
 // (mis_step); G lanes keep G chains of loads in flight per candidate.
-// Values that steer the group's control flow are read by its first lane and
-// broadcast, so every lane of a group takes the same path.  Returns 1 if
-// the candidate stays undecided (in every lane of the group).
+// The blocker and the entry to go on from are the same in every lane of the
+// group and stay in registers (b, r) while the candidate is tried again.
+// Returns 1 if the candidate stays undecided (in every lane of the group).
 template <u32 G>
-__device__ inline u32 mis_step_group(const DB& db, u32 i, bool valid, const u32* cand, u32* pw, u32* state, u32* blk,
-                                     u32* resume) {
+__device__ inline u32 mis_try(const DB& db, u32 i, u32 v, u32* pw, u32* state, u32& b, u32& r) {
   const int lane = threadIdx.x & 63, lead = lane & ~(int)(G - 1), j = lane - lead;
-  u32 s0 = (valid && j == 0) ? at_load(&state[i]) : 0u;
-  s0 = __shfl(s0, lead, 64);
-  if (!valid || s0) return 0;
-  const u32 v = cand[i];
-  const u32 b = blk[i];
   if (b != NOPOS) {
     u32 sb = j == 0 ? at_load(&state[b]) : 0u;
     sb = __shfl(sb, lead, 64);
@@ -1229,13 +1225,11 @@ __device__ inline u32 mis_step_group(const DB& db, u32 i, bool valid, const u32*
       return 0;
     }
   }
-  const u32 r = resume[i];
   const OLV o0 = olist(db, V2L(v)), o1 = olist(db, V2L(v) | 1);
   const u32 n0 = o0.n, ntot = o0.n + o1.n;
-  const u32 start = (r >> 31) ? n0 + (r & 0x7FFFFFFFu) : r;
   u32 first = NOPOS, bpos = NOPOS;  // this lane's earliest entry with an undecided earlier neighbour
   bool frozen = false;
-  for (u32 e = start + j; e < ntot && !frozen; e += G) {
+  for (u32 e = r + j; e < ntot && !frozen; e += G) {
     const u32 c = e < n0 ? o0.r[e] : o1.r[e - n0];
     const u32 h = db.lits[c];
     if (st_deleted(hdr_flags(h))) continue;
@@ -1269,32 +1263,49 @@ __device__ inline u32 mis_step_group(const DB& db, u32 i, bool valid, const u32*
     if (j == 0) mis_decide(state, pw, i, v, 2);
     return 0;
   }
-  const u32 e = (u32)(m >> 32);
-  if (e != NOPOS) {
-    if (j == 0) {
-      blk[i] = (u32)m;
-      resume[i] = e < n0 ? e : ((1u << 31) | (e - n0));
-    }
-    return 1;
-  }
+  r = (u32)(m >> 32);
+  b = (u32)m;
+  if (r != NOPOS) return 1;
   if (j == 0) mis_decide(state, pw, i, v, 1);
   return 0;
 }
+// Candidate i (each group its own) until it is decided, at most 'tries'
+// times: a candidate's blocker is decided by another wavefront of the same
+// launch as a rule, so waiting a little costs a poll of the blocker's state
+// where another pass costs a launch, the list entries again and a worklist
+// append.  No try waits for anything: one that stays undecided leaves its
+// blocker and entry in blk / resume and is appended to 'next'.
+template <u32 G>
+__device__ inline void mis_run(const DB& db, u32 i, bool valid, bool fresh, const u32* cand, u32* pos, u32* state,
+                               u32* blk, u32* resume, u32* next, u32* nnext, u32 tries) {
+  const bool lead = (threadIdx.x & (G - 1)) == 0;
+  bool undecided = valid && state[i] == 0;  // set before this launch: nothing decides i but this group
+  u32 v = 0, b = NOPOS, r = 0;
+  if (undecided) {
+    v = cand[i];
+    if (!fresh) b = blk[i], r = resume[i];
+  }
+  for (u32 t = 0; t < tries && __any(undecided); t++) {
+    if (t) __builtin_amdgcn_s_sleep(1);
+    if (undecided) undecided = mis_try<G>(db, i, v, pos, state, b, r) != 0;
+  }
+  if (undecided && lead) {
+    blk[i] = b;
+    resume[i] = r;
+  }
+  wave_append(undecided && lead, i, next, nnext);
+}
 
-// one election step over the undecided candidates idx[0..n) (all when idx
-// is null), G lanes per candidate; the ones still undecided are appended
+// the first pass, over all candidates; the ones still undecided are appended
 // to 'next'.  The launch reserves LDS per one-wavefront workgroup only to
 // bound occupancy (option "mislds"; 20 KiB leaves 2 wavefronts per SIMD:
 // Tseitin round 0 / 20 / 40 KiB -> mis_step_k 3.34 / 2.76 / 3.18 ms)
 template <u32 G>
-__global__ void mis_step_k(DB db, const u32* cand, const u32* idx, u32 n, u32* pos, u32* state, u32* blk,
-                           u32* resume, u32* next, u32* nnext) {
+__global__ void mis_step_k(DB db, const u32* cand, u32 n, u32* pos, u32* state, u32* blk, u32* resume, u32* next,
+                           u32* nnext, u32 tries) {
   const u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x;
   const u32 q = (u32)(t / G);
-  const bool valid = q < n;
-  const u32 i = valid ? (idx ? idx[q] : q) : 0u;
-  const bool undecided = mis_step_group<G>(db, i, valid, cand, pos, state, blk, resume) != 0;
-  wave_append(valid && (threadIdx.x & (G - 1)) == 0 && undecided, i, next, nnext);
+  mis_run<G>(db, q, q < n, true, cand, pos, state, blk, resume, next, nnext, tries);
 }
 // A worklist pass whose length is read on the device (n_in): a bounded grid
 // strides over the list, so several passes are queued without a host read;
@@ -1304,7 +1315,7 @@ __global__ void mis_step_k(DB db, const u32* cand, const u32* idx, u32 n, u32* p
 // of by a launch of its own before every pass
 template <u32 G>
 __global__ void mis_step_dev_k(DB db, const u32* cand, const u32* idx, const u32* n_in, u32* pos, u32* state,
-                               u32* blk, u32* resume, u32* next, u32* nnext, u32* iters, u32* zero) {
+                               u32* blk, u32* resume, u32* next, u32* nnext, u32* iters, u32* zero, u32 tries) {
   const u32 n = *n_in;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     *zero = 0;
@@ -1312,12 +1323,8 @@ __global__ void mis_step_dev_k(DB db, const u32* cand, const u32* idx, const u32
   }
   const u64 m = (u64)n * G;
   for (u64 base = (u64)blockIdx.x * blockDim.x; base < m; base += (u64)gridDim.x * blockDim.x) {  // wave-uniform
-    const u64 t = base + threadIdx.x;
-    const u32 q = (u32)(t / G);
-    const bool valid = q < n;
-    const u32 i = valid ? idx[q] : 0u;
-    const bool undecided = mis_step_group<G>(db, i, valid, cand, pos, state, blk, resume) != 0;
-    wave_append(valid && (threadIdx.x & (G - 1)) == 0 && undecided, i, next, nnext);
+    const u32 q = (u32)((base + threadIdx.x) / G);
+    mis_run<G>(db, q < n ? idx[q] : 0u, q < n, false, cand, pos, state, blk, resume, next, nnext, tries);
   }
 }
 #define MIS_LANES(G, call) \
@@ -1325,13 +1332,33 @@ __global__ void mis_step_dev_k(DB db, const u32* cand, const u32* idx, const u32
     case 2: call(2); break; \
     case 4: call(4); break; \
     case 8: call(8); break; \
+    case 16: call(16); break; \
     default: call(1); break; \
   }
-void k_mis_step(const DB& db, const u32* cand, const u32* idx, u32 n, u32* pos, u32* state, u32* blk,
-                u32* resume, u32* next, u32* nnext, u32 lds, u32 lanes, Stream* st) {
+// tries per candidate and pass: 1 / 4 / 16 / 64 tries took the election's
+// passes on 10M heavy-tailed variables from 3.17 + 0.62 to 3.08 + 0.05 ms
+// (4 and more alike), and a 20,000-variable call from 2.43 (1) to 1.63 (4)
+// and 1.58 ms (16)
+constexpr u32 MIS_TRIES = 32;
+// lanes per candidate by their number: up to 16 while all the groups fit
+// twice the wavefronts in flight (16 per CU at 10 KiB of LDS each; once, twice
+// and four times measured alike from 301 to 340,000 clauses).  A small
+// formula's step is a chain of dependent loads per list entry, which 16
+// lanes walk 16 entries at a time: with one lane the two first passes of the
+// 20,000-variable round took 89 us, with 16 lanes 98 us with all tries but
+// the last in them.
+u32 mis_lanes_for(u32 n) {
+  constexpr u64 in_flight = 256 * 16 * 64;
+  u32 g = 16;
+  while (g > 1 && (u64)n * g > 2 * in_flight) g >>= 1;
+  return g;
+}
+void k_mis_step(const DB& db, const u32* cand, u32 n, u32* pos, u32* state, u32* blk, u32* resume, u32* next,
+                u32* nnext, u32 lds, u32 lanes, Stream* st) {
   if (!n) return;
 #define MIS_FIRST(G) \
-  KLAUNCH_LDS(mis_step_k<G>, grid_for((size_t)n * G, 64), 64, lds, st, db, cand, idx, n, pos, state, blk, resume, next, nnext)
+  KLAUNCH_LDS(mis_step_k<G>, grid_for((size_t)n * G, 64), 64, lds, st, db, cand, n, pos, state, blk, resume, next, \
+              nnext, MIS_TRIES)
   MIS_LANES(lanes, MIS_FIRST)
 #undef MIS_FIRST
 }
@@ -1341,7 +1368,7 @@ void k_mis_step_dev(const DB& db, const u32* cand, const u32* idx, const u32* n_
   if (!n_bound) return;
 #define MIS_DEV(G)                                                                                           \
   KLAUNCH_LDS(mis_step_dev_k<G>, std::min(grid_for((size_t)n_bound * G, 64), 2048u), 64, lds, st, db, cand, idx, \
-              n_in, pos, state, blk, resume, next, nnext, iters, zero)
+              n_in, pos, state, blk, resume, next, nnext, iters, zero, MIS_TRIES)
   MIS_LANES(lanes, MIS_DEV)
 #undef MIS_DEV
 }

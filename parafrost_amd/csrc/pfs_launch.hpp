@@ -114,27 +114,28 @@ struct LcveArgs {
 };
 void k_lcve_classify(const DB& db, const LcveArgs& a, Stream*);
 // compact candidates with (score, var) < hard into cand/key (var order)
-void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u32* key, u32* ncand,
+// (pos: NOPOS for every variable)
+void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u32* key, u32* pos, u32* ncand,
                    void* tmp, Stream*);
-void k_lcve_positions(const u32* cand, u32 n, u32* pos, Stream*);
-// candidates passed over for an oversize clause (cflag 4) start decided and
-// not elected: they neither block nor freeze a neighbour
-void k_lcve_reject(const u32* cand, u32 n, const u8* cflag, u32* pos, u32* state, Stream*);
-// one election step over the candidates idx[0..n) (all when null); blk: per
-// candidate, an undecided earlier neighbour (NOPOS before the first step);
-// resume: per candidate, the list entry its scan goes on from (0 before the
-// first step); the still undecided candidates are appended to next (count
-// in *nnext)
+// the state before the first step: positions, states, counters (sc[1] = n,
+// sc[4..6] = sc[12..14] = 0).  reject: candidates passed over for an oversize
+// clause (cflag 4) start decided and not elected: they neither block nor
+// freeze a neighbour
+void k_mis_init(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc, Stream*);
+// lanes per candidate where neither set nor tuned: as many as keep every
+// candidate's group in flight
+u32 mis_lanes_for(u32 n);
+// the first step, over all candidates; blk, resume: of a candidate left
+// undecided, an undecided earlier neighbour and the list entry its scan goes
+// on from; it is appended to next (count in *nnext)
+void k_mis_step(const DB& db, const u32* cand, u32 n, u32* pos, u32* state, u32* blk, u32* resume, u32* next,
+                u32* nnext, u32 lds, u32 lanes, Stream*);
 // the same over the list idx[0..*n_in) (n_in on the device, at most n_bound);
-// *iters counts the passes over a non-empty list; *zero is cleared (the
-// counter the next pass appends to)
-// lds: bytes of LDS reserved per one-wavefront workgroup (occupancy);
-// lanes: lanes per candidate (1, 2, 4 or 8)
+// *iters counts the calls that had work; *zero is cleared (the counter the
+// next pass appends to)
 void k_mis_step_dev(const DB& db, const u32* cand, const u32* idx, const u32* n_in, u32 n_bound, u32* pos,
                     u32* state, u32* blk, u32* resume, u32* next, u32* nnext, u32* iters, u32* zero, u32 lds,
                     u32 lanes, Stream*);
-void k_mis_step(const DB& db, const u32* cand, const u32* idx, u32 n, u32* pos, u32* state, u32* blk,
-                u32* resume, u32* next, u32* nnext, u32 lds, u32 lanes, Stream*);
 void k_mis_break(const u32* cand, u32 n, const u8* cflag, const u32* state, u32* brk, Stream*);
 void k_mis_collect(const u32* cand, u32 n, const u32* state, u32 brk, u32* flag_tmp, u32* out,
                    u32* nout, void* tmp, Stream*);
