@@ -79,8 +79,8 @@ void Simplifier::free_all() {
                 &ot_off_, &ot_size_, &ot_refs_, &hist_, &otp_, &assign_, &vstate_, &assumed_, &vorg_, &trail_,
                 &score_, &cflag_, &flag_, &cand_, &key_, &pos_, &state_, &pv_, &vsz_, &vbase_, &type_,
                 &def_, &vncls_, &vnlits_, &vnstack_, &clsb_, &litb_, &stkb_, &snap_ref_, &snap_flg_,
-                &snap_size_, &snap_sig_, &snap_lbd_, &snap_np_, &snap_nn_, &scratch_, &elits_, &unit_by_,
-                &recs_, &ids_, &mark_, &ht_, &erecs_, &order_, &stack_, &tmp_, &tmp2_, &tmp3_, &scal_, &in_c_off_,
+                &snap_size_, &snap_sig_, &snap_lbd_, &snap_np_, &snap_nn_, &scratch_, &unit_by_,
+                &recs_, &ids_, &mark_, &ht_, &erecs_, &stack_, &tmp_, &tmp2_, &tmp3_, &scal_, &in_c_off_,
                 &in_lits_, &in_assign_, &in_vstate_, &in_trail_buf_, &proof_, &precs_,
                 &pstamp_, &plines_, &pbytes_, &subu_, &subaff_, &sublast_, &ust_, &ulit_,
                 &map_, &map_assign_, &out_, &vrest_, &lsum_};
@@ -152,11 +152,10 @@ void Simplifier::alloc_state() {
   mem_.ensure(vorg_, V1 * 4, 0, st_, S);
   mem_.ensure(trail_, (V1 + 1) * 4, 0, st_, S);
   for (Buf* b : {&score_, &flag_, &cand_, &key_, &pos_, &state_, &pv_, &vsz_, &vbase_, &type_, &def_,
-                 &vncls_, &vnlits_, &vnstack_, &clsb_, &litb_, &stkb_, &snap_np_, &snap_nn_, &order_, &sublast_,
+                 &vncls_, &vnlits_, &vnstack_, &clsb_, &litb_, &stkb_, &snap_np_, &snap_nn_, &sublast_,
                  &ust_, &ulit_})
     mem_.ensure(*b, (V1 + 1) * 4, 0, st_, S);
   mem_.ensure(cflag_, V1, 0, st_, S);
-  mem_.ensure(elits_, 2 * (V1 + 1) * 4, 0, st_, S);
   mem_.ensure(unit_by_, L2 * 4, 0, st_);
   mem_.ensure(recs_, 3 * (V1 + 1) * 4, 0, st_, S);
   mem_.ensure(subaff_, 3 * (V1 + 1) * 4, 0, st_, S);
@@ -1150,13 +1149,10 @@ void Simplifier::sort_ot() {
   if (!E_) return;
   stage_begin(S_SORT);
   DB db = make_db(cur_);
-  k_pv_lits(P<u32>(pv_), E_, P<u32>(elits_), st_);
   mem_.ensure(scratch_, std::max<size_t>(lits_end_, 6 * (size_t)E_ + 3) * 4, 0, st_);
-  mem_.ensure(tmp2_, (10 * (size_t)E_ + 3) * 4, 0, st_);
-  mem_.ensure(tmp_, std::max(tmp_.cap, scan_tmp_bytes(2 * (size_t)E_)), 0, st_);
-  k_sort_lists(db, P<u32>(elits_), 2 * E_, P<u32>(tmp2_), P<u32>(scal_) + 24, P<u32>(scratch_), P<u32>(lsum_),
-               tmp_.p, st_);
-  if (opt.work_order) k_work_order(db, P<u32>(pv_), E_, P<u32>(tmp2_), P<u32>(order_), tmp_.p, st_);
+  mem_.ensure(tmp2_, (12 * (size_t)E_ + 3) * 4, 0, st_);
+  mem_.ensure(tmp_, std::max(tmp_.cap, 2 * scan_tmp_bytes(2 * (size_t)E_)), 0, st_);
+  k_sort_lists(db, P<u32>(pv_), E_, P<u32>(tmp2_), P<u32>(scal_) + 24, P<u32>(scratch_), P<u32>(lsum_), tmp_.p, st_);
   stage_end();
   if (profile) {  // work measures, outside the stage's time
     uint64_t w[2];
@@ -1209,7 +1205,6 @@ bool Simplifier::sub() {
   const u32 cap = V_ + 1;
   auto run = [&](const u32* idx, u32 n, const std::vector<u32>& ran, u32 pass, bool vis) {
     // vis == false: the first pass (every variable, nothing visible yet)
-    fill_u32(sc, 0, 1, st_);
     SubOut out{P<u32>(recs_), sc, cap, P<u32>(subu_), P<u32>(vbase_), proof_out(2 * O + E_ + 64),
                SubVis{vis ? P<u32>(ust_) : nullptr, vis ? P<u32>(ulit_) : nullptr}};
     k_sub(db, opt, P<u32>(pv_), idx, n, out, P<u32>(vrest_), P<u32>(lsum_), tmp_.p, vis ? nullptr : &snap, st_);
@@ -1298,7 +1293,7 @@ bool Simplifier::sub() {
   // pass 1: every variable, nothing of this stage visible
   u32 pass = 1;
   fill_u32(P<u32>(sublast_), 1, E_, st_);
-  run(work_order(), E_, {}, pass, false);
+  run(nullptr, E_, {}, pass, false);
   std::vector<u32> vis_set;   // variables with a visible stage unit
   std::vector<u32> deferred;  // affected variables past the refutation, not re-run (ascending)
   bool vis_ready = false;
@@ -1428,17 +1423,16 @@ bool Simplifier::ve() {
     S = read_u32(sc);
   }
   VeDecision d{P<u32>(type_), P<u32>(def_), P<u32>(vncls_), P<u32>(vnlits_), P<u32>(vnstack_)};
-  k_ve_decide(db, opt, P<u32>(pv_), E_, d, work_order(), P<u32>(vrest_), P<u32>(lsum_), tmp_.p, st_);
-  scan_u32(P<u32>(vncls_), P<u32>(clsb_), E_, sc, tmp_.p, st_);
-  scan_u32(P<u32>(vnlits_), P<u32>(litb_), E_, sc + 1, tmp_.p, st_);
-  scan_u32(P<u32>(vnstack_), P<u32>(stkb_), E_, sc + 2, tmp_.p, st_);
+  k_ve_decide(db, opt, P<u32>(pv_), E_, d, P<u32>(vrest_), P<u32>(lsum_), tmp_.p, st_);
+  mem_.ensure(tmp_, std::max(tmp_.cap, 3 * scan_tmp_bytes(E_)), 0, st_);
+  scan3_u32({P<u32>(vncls_), P<u32>(vnlits_), P<u32>(vnstack_)}, {P<u32>(clsb_), P<u32>(litb_), P<u32>(stkb_)}, E_, sc,
+            tmp_.p, st_);
   u32 tot[3];
   d2h(tot, sc, 12, st_);
   stream_sync(st_);
   ensure_clause_room(tot[0], tot[1]);
   ensure_stack(stack_n_ + tot[2]);
   db = make_db(cur_);
-  fill_u32(sc + 3, 0, 1, st_);
   VeApply ap;
   ap.cls_base = P<u32>(clsb_);
   ap.lit_base = P<u32>(litb_);
@@ -1453,13 +1447,12 @@ bool Simplifier::ve() {
   ap.units = UnitOut{P<u32>(recs_), sc + 3, V_ + 1};
   ap.error = sc + 6;
   ap.proof = proof_out(tot[0] + S + V_ + 64);
-  fill_u32(sc + 6, 0, 1, st_);
-  k_ve_apply(db, P<u32>(pv_), E_, d, ap, P<u32>(vrest_), P<u32>(lsum_), tmp_.p, st_);
-  // eliminated variables (markEliminated, solver.h:535-541), counted now so
-  // that one read brings it with the unit records' count and the error flag
-  k_count_nonzero(P<u32>(type_), E_, sc + 7, st_);
-  u32 w5[5];  // sc[3]: unit records, sc[6]: write error, sc[7]: eliminated
-  d2h(w5, sc + 3, sizeof(w5), st_);
+  k_ve_apply(db, P<u32>(pv_), E_, d, ap, P<u32>(vrest_), P<u32>(lsum_), sc + 3, 4, tmp_.p, st_);
+  u32 w5[5];  // sc[3]: unit records, sc[6]: write error
+  d2h(w5, sc + 3, 16, st_);
+  // eliminated variables (markEliminated, solver.h:535-541): the ones placed
+  // before the first that VE keeps
+  d2h(w5 + 4, P<u32>(vrest_) + LV_KEPT, 4, st_);
   stream_sync(st_);
   if (w5[3]) throw DeviceFail{"BVE resolvent writes disagree with the counted space"};
   ncls_ += tot[0];
@@ -1519,13 +1512,13 @@ void Simplifier::bce() {
   stage_begin(S_BCE);
   DB db = make_db(cur_);
   u32* sc = P<u32>(scal_);
-  k_bce(db, opt, P<u32>(pv_), P<u32>(type_), E_, P<u32>(vnstack_), nullptr, nullptr, true, work_order(), st_);
+  k_bce(db, opt, P<u32>(pv_), P<u32>(type_), E_, P<u32>(vnstack_), nullptr, nullptr, true, st_);
   scan_u32(P<u32>(vnstack_), P<u32>(stkb_), E_, sc, tmp_.p, st_);
   const u32 T = read_u32(sc);
   if (T) {
     ensure_stack(stack_n_ + T);
     k_bce(db, opt, P<u32>(pv_), P<u32>(type_), E_, nullptr, P<u32>(stkb_), P<u32>(stack_) + stack_n_, false,
-          work_order(), st_);
+          st_);
     stack_n_ += T;
     rounds_.back().stack_words += T;
   }

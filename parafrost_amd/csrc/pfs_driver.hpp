@@ -215,7 +215,6 @@ class Simplifier {
   ProofOut proof_out(u32 cap);                  // device record buffer for a per-variable kernel
   void proof_collect(std::vector<ProofEv>& ev, u32 below_k);  // records of the last kernel with k < below_k
   uint32_t read_u32(const void* dptr);
-  const u32* work_order() { return opt.work_order ? P<u32>(order_) : nullptr; }
   void stage_begin(Stage s);
   void stage_end();
 
@@ -243,7 +242,7 @@ class Simplifier {
   // per elected variable
   Buf vsz_, vbase_, type_, def_, vncls_, vnlits_, vnstack_, clsb_, litb_, stkb_;
   Buf snap_ref_, snap_flg_, snap_size_, snap_sig_, snap_lbd_, snap_np_, snap_nn_, scratch_;
-  Buf elits_, unit_by_, recs_, ids_, mark_, ht_, erecs_, order_, subu_;
+  Buf unit_by_, recs_, ids_, mark_, ht_, erecs_, subu_;
   Buf vrest_;  // SUB, VE: size classes and placement of the variables
   Buf lsum_;   // per elected literal (2k, 2k + 1): clause size sum of its list at the list sort
   Buf subaff_, sublast_, ust_, ulit_;  // SUB re-runs: affected flags, last pass, visible stage units

@@ -371,8 +371,17 @@ __device__ inline void store_items(u32* out, size_t b, size_t n, const u32 (&v)[
     if (b + i < n) out[b + i] = v[i];
 }
 static_assert(SIPT == 8, "two 16-byte moves per thread");
+// up to three arrays of n items scanned by the same launches, one per row
+// of the grid
+struct ScanSet {
+  const u32* in[3];
+  u32* out[3];
+  u32* total[3];
+};
 template <bool VEC>
-__global__ void scan_reduce_k(const u32* in, size_t n, u32* part) {
+__global__ void scan_reduce_k(ScanSet a, size_t n, u32* part) {
+  const u32* in = a.in[blockIdx.y];
+  part += (size_t)blockIdx.y * gridDim.x;
   __shared__ u32 lw[NW];
   u32 s = 0;
 #pragma unroll
@@ -387,7 +396,9 @@ __global__ void scan_reduce_k(const u32* in, size_t n, u32* part) {
   if (threadIdx.x == 0) part[blockIdx.x] = tot;
 }
 // exclusive scan of the workgroup partials by one workgroup
-__global__ void scan_top_k(u32* part, size_t nb, u32* total) {
+__global__ void scan_top_k(u32* part, size_t nb, ScanSet a) {
+  u32* total = a.total[blockIdx.x];
+  part += (size_t)blockIdx.x * nb;
   __shared__ u32 lw[NW];
   u32 carry = 0;
   for (size_t base = 0; base < nb; base += STILE) {
@@ -413,7 +424,10 @@ __global__ void scan_top_k(u32* part, size_t nb, u32* total) {
 // each thread reads its items before the tile's barriers and writes them
 // after, so in == out is fine
 template <bool VEC>
-__global__ void scan_down_k(const u32* in, u32* out, size_t n, const u32* part) {
+__global__ void scan_down_k(ScanSet a, size_t n, const u32* part) {
+  const u32* in = a.in[blockIdx.y];
+  u32* out = a.out[blockIdx.y];
+  part += (size_t)blockIdx.y * gridDim.x;
   __shared__ u32 lw[NW];
   u32 carry = part[blockIdx.x];
 #pragma unroll 1
@@ -436,67 +450,130 @@ __global__ void scan_down_k(const u32* in, u32* out, size_t n, const u32* part) 
     carry += tot;
   }
 }
-// short scans in one launch: one workgroup of 1024 threads walks the input
-// in tiles of 8192 items with a running carry (each thread reads its items
-// before the tile's barriers and writes them after, so in == out is fine)
+// Short scans in one launch by one workgroup of 1024 threads.  Every thread
+// loads all its items (8, 32 or 64 consecutive ones, as 16-byte words where
+// both arrays allow it) before the one prefix sum over the workgroup, so the
+// launch waits for memory once; walking 32,768 items in four tiles, each
+// with its loads, barriers and stores, took 11 us against 5.  Every item is
+// read before the barriers and written after, so in == out is fine.
 constexpr int S1_T = 1024;
-constexpr size_t S1_MAX = 4 * (size_t)S1_T * SIPT;  // at most four tiles
-__global__ void __launch_bounds__(S1_T) scan_one_k(const u32* in, u32* out, size_t n, u32* total) {
+constexpr size_t S1_MAX = 64 * (size_t)S1_T;
+template <int IPT, bool VEC>
+__global__ void __launch_bounds__(S1_T) scan_one_k(ScanSet a, u32 n) {
+  const u32* in = a.in[blockIdx.x];
+  u32 *out = a.out[blockIdx.x], *total = a.total[blockIdx.x];
   __shared__ u32 lw[S1_T / 64];
-  u32 carry = 0;
-  for (size_t base = 0; base < n; base += (size_t)S1_T * SIPT) {
-    const size_t b = base + (size_t)threadIdx.x * SIPT;
-    u32 v[SIPT];
-    u32 s = 0;
+  const u32 b = threadIdx.x * IPT;
+  u32 v[IPT / 8][8], s = 0, tot;
 #pragma unroll
-    for (int i = 0; i < SIPT; i++) {
-      v[i] = (b + i < n) ? in[b + i] : 0u;
-      s += v[i];
-    }
-    u32 tot;
-    u32 pre = block_excl_scan_w<S1_T / 64>(s, lw, &tot) + carry;
+  for (int q = 0; q < IPT / 8; q++) load_items<VEC>(in, b + 8 * q, n, v[q]);
 #pragma unroll
-    for (int i = 0; i < SIPT; i++) {
-      if (b + i < n) out[b + i] = pre;
-      pre += v[i];
+  for (int q = 0; q < IPT / 8; q++)
+#pragma unroll
+    for (int i = 0; i < 8; i++) s += v[q][i];
+  u32 pre = block_excl_scan_w<S1_T / 64>(s, lw, &tot);
+#pragma unroll
+  for (int q = 0; q < IPT / 8; q++) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const u32 x = v[q][i];
+      v[q][i] = pre;
+      pre += x;
     }
-    carry += tot;
+    store_items<VEC>(out, b + 8 * q, n, v[q]);
   }
-  if (threadIdx.x == 0 && total) *total = carry;
+  if (threadIdx.x == 0 && total) *total = tot;
 }
 size_t scan_tmp_bytes(size_t n) { return (grid_for(n, SBLK) + 64) * sizeof(u32); }
+template <bool VEC>
+static void scan_rows(const ScanSet& a, u32 rows, size_t n, void* tmp, Stream* st) {
+  if (n <= S1_MAX) {
+    if (n <= 8 * S1_T) KLAUNCH((scan_one_k<8, VEC>), rows, S1_T, st, a, (u32)n);
+    else if (n <= 32 * S1_T) KLAUNCH((scan_one_k<32, VEC>), rows, S1_T, st, a, (u32)n);
+    else KLAUNCH((scan_one_k<64, VEC>), rows, S1_T, st, a, (u32)n);
+    return;
+  }
+  const unsigned nb = grid_for(n, SBLK);
+  u32* part = (u32*)tmp;
+  KLAUNCH(scan_reduce_k<VEC>, dim3(nb, rows), ST, st, a, n, part);
+  KLAUNCH(scan_top_k, rows, ST, st, part, nb, a);
+  KLAUNCH(scan_down_k<VEC>, dim3(nb, rows), ST, st, a, n, part);
+}
+static void scan_set(const ScanSet& a, u32 rows, size_t n, void* tmp, Stream* st) {
+  uintptr_t bits = 0;
+  for (u32 q = 0; q < rows; q++) bits |= (uintptr_t)a.in[q] | (uintptr_t)a.out[q];
+  if ((bits & 15) == 0) scan_rows<true>(a, rows, n, tmp, st);
+  else scan_rows<false>(a, rows, n, tmp, st);
+}
 void scan_u32(const u32* in, u32* out, size_t n, u32* total, void* tmp, Stream* st) {
   if (n == 0) {
     if (total) fill_u32(total, 0, 1, st);
     return;
   }
-  if (n <= S1_MAX) {
-    KLAUNCH(scan_one_k, 1, S1_T, st, in, out, n, total);
+  scan_set(ScanSet{{in}, {out}, {total}}, 1, n, tmp, st);
+}
+// tmp: 3 * scan_tmp_bytes(n)
+void scan3_u32(const u32* const (&in)[3], u32* const (&out)[3], size_t n, u32* total, void* tmp, Stream* st) {
+  if (n == 0) {
+    fill_u32(total, 0, 3, st);
     return;
   }
-  const unsigned nb = grid_for(n, SBLK);
-  u32* part = (u32*)tmp;
-  if ((((uintptr_t)in | (uintptr_t)out) & 15) == 0) {
-    KLAUNCH(scan_reduce_k<true>, nb, ST, st, in, n, part);
-    KLAUNCH(scan_top_k, 1, ST, st, part, nb, total);
-    KLAUNCH(scan_down_k<true>, nb, ST, st, in, out, n, part);
-  } else {
-    KLAUNCH(scan_reduce_k<false>, nb, ST, st, in, n, part);
-    KLAUNCH(scan_top_k, 1, ST, st, part, nb, total);
-    KLAUNCH(scan_down_k<false>, nb, ST, st, in, out, n, part);
-  }
+  scan_set(ScanSet{{in[0], in[1], in[2]}, {out[0], out[1], out[2]}, {total, total + 1, total + 2}}, 3, n, tmp, st);
 }
 
 // ---------------------------------------------------------------- stable radix sort
 // LSD passes of up to 8 bits.  A pass counts each tile's digits (rs_count_k),
 // scans the digit-major counts, then every tile sorts itself by the digit
-// in LDS with stable one-bit splits and writes each digit's run to its
+// in LDS with stable two-bit splits and writes each digit's run to its
 // place (rs_scatter_k), so the stores go out in runs rather than one
 // scattered word per item.
 constexpr int RS_T = 256, RS_IPT = 8, RS_TILE = RS_T * RS_IPT;  // threads, items per thread, items per tile
 constexpr int RB = 8, RBUCK = 1 << RB;
 static_assert(RS_T == RBUCK, "one digit bin per thread");
 
+// Stable splits by two bits at a time: the four counts of a thread's items
+// are 16-bit fields of one 64-bit word, so one prefix sum over the workgroup
+// serves both bits.
+template <int W>
+__device__ inline u64 block_excl_scan64_w(u64 v, u64* lw, u64* total) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  u64 x = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const u64 y = __shfl_up((unsigned long long)x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) lw[wid] = x;
+  __syncthreads();
+  u64 pre = 0, tot = 0;
+#pragma unroll
+  for (int w = 0; w < W; w++) {
+    const u64 s = lw[w];
+    pre += (w < wid) ? s : 0ull;
+    tot += s;
+  }
+  __syncthreads();
+  *total = tot;
+  return pre + x - v;
+}
+// where this thread's items go in a stable split of the workgroup's items by
+// the two bits d[i]
+template <int T, int IPT>
+__device__ inline void split4(const u32 (&d)[IPT], u32 (&dst)[IPT], u64* lw) {
+  static_assert(T * IPT < 65536, "counts are 16-bit fields");
+  u64 c = 0, tot;
+#pragma unroll
+  for (int i = 0; i < IPT; i++) c += 1ull << (16 * d[i]);
+  u64 at = block_excl_scan64_w<T / 64>(c, lw, &tot);
+  // each field also starts behind the items of the smaller digits
+  const u64 t0 = tot & 0xFFFF, t1 = (tot >> 16) & 0xFFFF, t2 = (tot >> 32) & 0xFFFF;
+  at += (t0 << 16) + ((t0 + t1) << 32) + ((t0 + t1 + t2) << 48);
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    dst[i] = (u32)(at >> (16 * d[i])) & 0xFFFFu;
+    at += 1ull << (16 * d[i]);
+  }
+}
 __global__ void __launch_bounds__(RS_T) rs_count_k(const u32* keys, size_t n, int shift, u32 mask, u32* counts,
                                                   u32 nb) {
   __shared__ u32 h[RBUCK];
@@ -511,43 +588,47 @@ __global__ void __launch_bounds__(RS_T) rs_count_k(const u32* keys, size_t n, in
   __syncthreads();
   counts[(size_t)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
 }
+// vin null: the values are the positions; kout null: the sorted keys are
+// not wanted; starts: where the digits of q << sshift and more begin, for
+// q below nstarts
 __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* vin, u32* kout, u32* vout,
-                                                    size_t n, int shift, int width, const u32* offs, u32 nb) {
-  __shared__ u32 sk[2][RS_TILE], sv[2][RS_TILE];
+                                                    size_t n, int shift, int width, const u32* offs, u32 nb,
+                                                    u32* starts, u32 nstarts, int sshift) {
+  __shared__ u32 sk[RS_TILE], sv[RS_TILE];
   __shared__ u32 start[RBUCK];
   __shared__ u32 lw[RS_T / 64];
+  __shared__ u64 lw64[RS_T / 64];
   const u32 mask = (1u << width) - 1u;
   const size_t base = (size_t)blockIdx.x * RS_TILE;
-  const u32 cnt = (u32)min((size_t)RS_TILE, n - base);
+  const u32 cnt = (u32)min((size_t)RS_TILE, n - base), j0 = threadIdx.x * RS_IPT;
   // the tile in input order; slots past the input take the largest digit
   // and stay behind every item (they come last and the splits are stable)
 #pragma unroll
   for (int i = 0; i < RS_IPT; i++) {
     const u32 j = i * RS_T + threadIdx.x;
-    sk[0][j] = j < cnt ? kin[base + j] : (mask << shift);
-    sv[0][j] = j < cnt ? vin[base + j] : 0u;
+    sk[j] = j < cnt ? kin[base + j] : (mask << shift);
+    sv[j] = j < cnt ? (vin ? vin[base + j] : (u32)(base + j)) : 0u;
+  }
+  if (blockIdx.x == 0 && threadIdx.x < nstarts) {
+    const u32 q = threadIdx.x << sshift;
+    starts[threadIdx.x] = q <= mask ? offs[(size_t)q * nb] : (u32)n;
   }
   start[threadIdx.x] = 0;
   __syncthreads();
-  // one stable split per digit bit: thread t moves items t*IPT .. t*IPT+IPT-1
-  int b = 0;
-  for (int bit = 0; bit < width; bit++, b ^= 1) {
-    const u32 j0 = threadIdx.x * RS_IPT;
-    u32 k[RS_IPT], v[RS_IPT], z = 0;
+  // thread t moves items t*IPT .. t*IPT+IPT-1
+  for (int bit = 0; bit < width; bit += 2) {
+    u32 k[RS_IPT], v[RS_IPT], d[RS_IPT], dst[RS_IPT];
 #pragma unroll
     for (int i = 0; i < RS_IPT; i++) {
-      k[i] = sk[b][j0 + i];
-      v[i] = sv[b][j0 + i];
-      z += ((k[i] >> (shift + bit)) & 1u) ^ 1u;
+      k[i] = sk[j0 + i];
+      v[i] = sv[j0 + i];
+      d[i] = (k[i] >> (shift + bit)) & (bit + 1 < width ? 3u : 1u);
     }
-    u32 zt;
-    u32 zp = block_excl_scan_w<RS_T / 64>(z, lw, &zt);
-    u32 op = j0 - zp;  // ones before this thread's items
+    split4<RS_T, RS_IPT>(d, dst, lw64);  // its barriers follow every read above
 #pragma unroll
     for (int i = 0; i < RS_IPT; i++) {
-      const u32 dst = ((k[i] >> (shift + bit)) & 1u) ? zt + op++ : zp++;
-      sk[b ^ 1][dst] = k[i];
-      sv[b ^ 1][dst] = v[i];
+      sk[dst[i]] = k[i];
+      sv[dst[i]] = v[i];
     }
     __syncthreads();
   }
@@ -555,7 +636,7 @@ __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* 
 #pragma unroll
   for (int i = 0; i < RS_IPT; i++) {
     const u32 j = i * RS_T + threadIdx.x;
-    if (j < cnt) atomicAdd(&start[(sk[b][j] >> shift) & mask], 1u);
+    if (j < cnt) atomicAdd(&start[(sk[j] >> shift) & mask], 1u);
   }
   __syncthreads();
   u32 tot;
@@ -567,10 +648,10 @@ __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* 
   for (int i = 0; i < RS_IPT; i++) {
     const u32 j = i * RS_T + threadIdx.x;
     if (j < cnt) {
-      const u32 key = sk[b][j], d = (key >> shift) & mask;
+      const u32 key = sk[j], d = (key >> shift) & mask;
       const u32 dst = offs[(size_t)d * nb + blockIdx.x] + (j - start[d]);
-      kout[dst] = key;
-      vout[dst] = sv[b][j];
+      if (kout) kout[dst] = key;
+      vout[dst] = sv[j];
     }
   }
 }
@@ -578,10 +659,61 @@ size_t radix_tmp_bytes(size_t n) {
   const size_t nb = grid_for(n ? n : 1, RS_TILE);
   return 2 * n * sizeof(u32) + RBUCK * nb * sizeof(u32) + scan_tmp_bytes(RBUCK * nb) + 256;
 }
-// sorts by the low 'bits' bits of the keys (higher bits are ignored)
+// Sorts of up to SO_MAX items in one launch by one workgroup: T threads
+// hold IPT consecutive items each in registers, and stable splits move them
+// through LDS.  The three launches and two copies of a pass over digits cost 40-60 us whatever
+// the size; this sorts 8,192 items by 8 bits in about 12 us.
+constexpr int SO_T = 1024, SO_IPT = 8;
+constexpr u32 SO_MAX = SO_T * SO_IPT;
+// values sorted in place by the low 'bits' bits of their keys (the keys stay)
+template <int T>
+__global__ void __launch_bounds__(T) sort_one_k(const u32* keys, u32* vals, u32 n, int bits) {
+  constexpr int IPT = SO_IPT;
+  __shared__ u32 sk[T * IPT];
+  __shared__ uint16_t si[T * IPT];
+  __shared__ u64 lw[T / 64];
+  const u32 j0 = threadIdx.x * IPT;
+  u32 k[IPT], id[IPT], d[IPT], dst[IPT], v[IPT];
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    k[i] = j0 + i < n ? keys[j0 + i] : 0xFFFFFFFFu;  // slots past the input stay behind it
+    id[i] = j0 + i;
+  }
+  for (int bit = 0; bit < bits; bit += 2) {
+    const u32 m = bit + 1 < bits ? 3u : 1u;
+#pragma unroll
+    for (int i = 0; i < IPT; i++) d[i] = (k[i] >> bit) & m;
+    split4<T, IPT>(d, dst, lw);
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+      sk[dst[i]] = k[i];
+      si[dst[i]] = (uint16_t)id[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+      k[i] = sk[j0 + i];
+      id[i] = si[j0 + i];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < IPT; i++) v[i] = j0 + i < n ? vals[id[i]] : 0u;
+  __syncthreads();  // every value is read before any is written
+#pragma unroll
+  for (int i = 0; i < IPT; i++)
+    if (j0 + i < n) vals[j0 + i] = v[i];
+}
+// sorts the values by the low 'bits' bits of their keys (higher bits are
+// ignored); the keys are consumed
 void radix_sort_pairs(u32* keys, u32* vals, size_t n, int bits, void* tmp, Stream* st) {
   if (n < 2 || bits <= 0) return;
   bits = std::min(bits, 32);
+  if (n <= SO_MAX) {
+    if (n <= 256 * SO_IPT) KLAUNCH(sort_one_k<256>, 1, 256, st, keys, vals, (u32)n, bits);
+    else KLAUNCH(sort_one_k<SO_T>, 1, SO_T, st, keys, vals, (u32)n, bits);
+    return;
+  }
   const u32 nb = grid_for(n, RS_TILE);
   u32* k2 = (u32*)tmp;
   u32* v2 = k2 + n;
@@ -592,16 +724,115 @@ void radix_sort_pairs(u32* keys, u32* vals, size_t n, int bits, void* tmp, Strea
   for (int shift = 0; shift < bits; shift += RB) {
     const int width = std::min(RB, bits - shift);
     const u32 mask = (1u << width) - 1u;
+    const bool last = shift + RB >= bits;
     KLAUNCH(rs_count_k, nb, RS_T, st, ka, n, shift, mask, counts, nb);
-    scan_u32(counts, counts, (size_t)RBUCK * nb, nullptr, stmp, st);
-    KLAUNCH(rs_scatter_k, nb, RS_T, st, ka, va, kb, vb, n, shift, width, counts, nb);
+    scan_u32(counts, counts, (size_t)(mask + 1) * nb, nullptr, stmp, st);
+    KLAUNCH(rs_scatter_k, nb, RS_T, st, ka, va, last ? nullptr : kb, vb, n, shift, width, counts, nb, nullptr, 0u, 0);
     u32* t = ka; ka = kb; kb = t;
     t = va; va = vb; vb = t;
     passes++;
   }
-  if (passes & 1) {
-    d2d(keys, ka, n * sizeof(u32), st);
-    d2d(vals, va, n * sizeof(u32), st);
+  if (passes & 1) d2d(vals, va, n * sizeof(u32), st);
+}
+
+// ---------------------------------------------------------------- placement by a small key
+// The items 0..n-1 in the stable order of a small key (below 1 << bits, at
+// most 8 bits) that f computes: out receives f.val(t) in that order,
+// starts[q] for q below nstarts where the keys of q << sshift and more
+// begin.  zero: nz words cleared on
+// the way (counters of the launches that follow).  One launch by one
+// workgroup for up to SO_MAX items, else three (keys and their counts per
+// tile, one scan, the scatter); what this replaces was a launch for the keys,
+// three for the digit pass, two copies, one for the starts and a fill.
+constexpr int KEY_IDX_BITS = 13;
+static_assert(SO_MAX <= (1u << KEY_IDX_BITS), "an item's index and key share a word");
+template <int T, class F>
+__global__ void __launch_bounds__(T) place_one_k(F f, u32 n, int bits, u32* out, u32* starts, u32 nstarts, int sshift,
+                                                 u32* zero, u32 nz) {
+  constexpr int IPT = SO_IPT;
+  __shared__ u32 sk[T * IPT];
+  __shared__ u64 lw[T / 64];
+  if (threadIdx.x < nz) zero[threadIdx.x] = 0;
+  const u32 j0 = threadIdx.x * IPT;
+  const u32 top = (1u << bits) - 1u, imask = (1u << KEY_IDX_BITS) - 1u;
+  u32 x[IPT], d[IPT], dst[IPT];
+  // strided for the reads of f; slots past the input take the largest key
+  // and stay behind every item (they come last and the splits are stable)
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    const u32 j = i * T + threadIdx.x;
+    sk[j] = ((j < n ? f.key(j) : top) << KEY_IDX_BITS) | j;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < IPT; i++) x[i] = sk[j0 + i];
+  __syncthreads();
+  for (int bit = 0; bit < bits; bit += 2) {
+#pragma unroll
+    for (int i = 0; i < IPT; i++) d[i] = (x[i] >> (KEY_IDX_BITS + bit)) & (bit + 1 < bits ? 3u : 1u);
+    split4<T, IPT>(d, dst, lw);
+#pragma unroll
+    for (int i = 0; i < IPT; i++) sk[dst[i]] = x[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IPT; i++) x[i] = sk[j0 + i];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < IPT; i++) sk[j0 + i] = x[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    const u32 j = i * T + threadIdx.x;
+    if (j >= n) continue;
+    out[j] = f.val(sk[j] & imask);
+    if (nstarts) {
+      const int sh = KEY_IDX_BITS + sshift;
+      const u32 key = sk[j] >> sh;
+      for (u32 q = j ? (sk[j - 1] >> sh) + 1 : 0; q <= key && q < nstarts; q++) starts[q] = j;
+      if (j == n - 1)
+        for (u32 q = key + 1; q < nstarts; q++) starts[q] = n;
+    }
+  }
+}
+template <class F>
+__global__ void __launch_bounds__(RS_T) place_count_k(F f, u32 n, u32* keys, u32* vals, u32* counts, u32 ndig, u32 nb,
+                                                      u32* zero, u32 nz) {
+  __shared__ u32 h[RBUCK];
+  if (blockIdx.x == 0 && threadIdx.x < nz) zero[threadIdx.x] = 0;
+  h[threadIdx.x] = 0;  // RS_T == RBUCK
+  __syncthreads();
+  const u32 base = blockIdx.x * RS_TILE;
+#pragma unroll
+  for (int i = 0; i < RS_IPT; i++) {
+    const u32 j = base + i * RS_T + threadIdx.x;
+    if (j < n) {
+      const u32 k = f.key(j);
+      keys[j] = k;
+      vals[j] = f.val(j);
+      atomicAdd(&h[k], 1u);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < ndig) counts[(size_t)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
+}
+// tmp: radix_tmp_bytes(n)
+template <class F>
+void place(F f, u32 n, int bits, u32* out, u32* starts, u32 nstarts, int sshift, u32* zero, u32 nz, void* tmp,
+           Stream* st) {
+  if (n <= 256 * SO_IPT) {
+    KLAUNCH((place_one_k<256, F>), 1, 256, st, f, n, bits, out, starts, nstarts, sshift, zero, nz);
+  } else if (n <= SO_MAX) {
+    KLAUNCH((place_one_k<SO_T, F>), 1, SO_T, st, f, n, bits, out, starts, nstarts, sshift, zero, nz);
+  } else {
+    const u32 nb = grid_for(n, RS_TILE), ndig = 1u << bits;
+    u32* k2 = (u32*)tmp;
+    u32* v2 = k2 + n;
+    u32* counts = v2 + n;
+    KLAUNCH(place_count_k<F>, nb, RS_T, st, f, n, k2, v2, counts, ndig, nb, zero, nz);
+    scan_u32(counts, counts, (size_t)ndig * nb, nullptr, counts + (size_t)RBUCK * nb, st);
+    KLAUNCH(rs_scatter_k, nb, RS_T, st, k2, v2, nullptr, out, (size_t)n, 0, bits, counts, nb, starts, nstarts,
+            sshift);
   }
 }
 
@@ -908,34 +1139,50 @@ __device__ inline u32 sort_group(const DB& db, u32 lit, bool valid, u32 j, u32 g
 // heavy-tailed round's 6.1M lists; a worklist filled with one atomic per
 // wavefront on a shared counter; a second pass over every list that skips
 // the short ones; a bounded grid striding over the lists.)
+// APPEND: the longer lists go straight to the collected ones (cnt[1] middle,
+// cnt[0] long), one atomic per wavefront and kind: for up to
+// SORT_APPEND_MAX lists that is cheaper than the flags' scans and packs.
 constexpr u32 SORT_TINY = 4;
-__global__ void sort_tiny_k(DB db, const u32* lits, u32 n, u32* lsum, u32* fmid, u32* flong) {
+constexpr u32 SORT_APPEND_MAX = 1u << 17;
+// list g of the elected variables: the positive and the negative one of
+// variable g / 2
+__device__ inline u32 list_lit(const u32* pv, u32 g) { return V2L(pv[g >> 1]) | (g & 1u); }
+template <bool APPEND>
+__global__ void sort_tiny_k(DB db, const u32* pv, u32 n, u32* lsum, u32* mid, u32* big, u32* cnt) {
   const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
   const u32 g = t / SORT_TINY, j = t % SORT_TINY;
   const bool valid = g < n;
-  const u32 len = sort_group<SORT_TINY, 0>(db, valid ? lits[g] : 0u, valid, j, g, lsum);
-  if (valid && j == 0) {
-    fmid[g] = len > SORT_TINY && len <= SORT_SMALL ? 1u : 0u;
-    flong[g] = len > SORT_SMALL ? 1u : 0u;
+  const u32 len = sort_group<SORT_TINY, 0>(db, valid ? list_lit(pv, g) : 0u, valid, j, g, lsum);
+  const bool one = valid && j == 0, m = one && len > SORT_TINY && len <= SORT_SMALL, l = one && len > SORT_SMALL;
+  if (APPEND) {
+    wave_append(m, g, mid, cnt + 1);
+    wave_append(l, g, big, cnt);
+  } else if (one) {  // flags
+    mid[g] = m ? 1u : 0u;
+    big[g] = l ? 1u : 0u;
   }
+}
+__global__ void sort_pack_k(const u32* fmid, const u32* flong, const u32* pmid, const u32* plong, u32 n, u32* mid,
+                            u32* big) {
+  const u32 g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g >= n) return;
+  if (fmid[g]) mid[pmid[g]] = g;
+  if (flong[g]) big[plong[g]] = g;
 }
 // the lists mid[0..*nmid), 16 lanes each; a bounded grid strides over them
 // (the loop bound is the same for every lane of a wavefront)
-__global__ void sort_mid_k(DB db, const u32* lits, const u32* mid, const u32* nmid, u32* lsum) {
+__global__ void sort_mid_k(DB db, const u32* pv, const u32* mid, const u32* nmid, u32* lsum) {
   const u64 m = (u64)*nmid * SORT_SMALL;
   for (u64 base = (u64)blockIdx.x * blockDim.x; base < m; base += (u64)gridDim.x * blockDim.x) {
     const u64 t = base + threadIdx.x;
     const bool valid = t < m;
     const u32 g = valid ? mid[t / SORT_SMALL] : 0u;
-    sort_group<SORT_SMALL, SORT_TINY>(db, valid ? lits[g] : 0u, valid, (u32)(t % SORT_SMALL), g, lsum);
+    sort_group<SORT_SMALL, SORT_TINY>(db, valid ? list_lit(pv, g) : 0u, valid, (u32)(t % SORT_SMALL), g, lsum);
   }
 }
-// bitonic sort of one list per workgroup in LDS (16 < len <= SORT_BLOCK);
-// big: positions in lits
-__device__ void sort_block_list(DB db, const u32* lits, u32 g, u32* lsum, u64* ka, u64* kb, u32* kid, u32* lw) {
-  const u32 lit = lits[g];
+// bitonic sort of one list per workgroup in LDS (16 < len <= SORT_BLOCK)
+__device__ void sort_block_list(DB db, u32 lit, u32 g, u32* lsum, u64* ka, u64* kb, u32* kid, u32* lw) {
   const u32 len = db.ot_size[lit];
-  if (len <= SORT_SMALL || len > SORT_BLOCK) return;
   u32* r = db.ot_refs + db.ot_off[lit];
   u32 N = 1;
   while (N < len) N <<= 1;
@@ -977,26 +1224,10 @@ __device__ void sort_block_list(DB db, const u32* lits, u32 g, u32* lsum, u64* k
   }
   for (u32 i = threadIdx.x; i < len; i += blockDim.x) r[i] = kid[i];
 }
-// big: positions in lits, *nbig of them (read on the device: a bounded grid
-// strides over them, so the launch needs no host read of the count)
-__global__ void __launch_bounds__(256) sort_block_k(DB db, const u32* lits, const u32* big, const u32* nbig,
-                                                    u32* lsum) {
-  __shared__ u64 ka[SORT_BLOCK];
-  __shared__ u64 kb[SORT_BLOCK];
-  __shared__ u32 kid[SORT_BLOCK];
-  __shared__ u32 lw[NW];
-  const u32 nb = *nbig;
-  for (u32 b = blockIdx.x; b < nb; b += gridDim.x) {
-    sort_block_list(db, lits, big[b], lsum, ka, kb, kid, lw);
-    __syncthreads();
-  }
-}
 // bottom-up merge sort of one long list by one thread (rare lists above
 // SORT_BLOCK entries); 'scratch' has one slot per occurrence entry
-__device__ void sort_large_list(DB db, const u32* lits, u32 g, u32* scratch, u32* lsum) {
-  const u32 lit = lits[g];
+__device__ void sort_large_list(DB db, u32 lit, u32 g, u32* scratch, u32* lsum) {
   const u32 len = db.ot_size[lit];
-  if (len <= SORT_BLOCK) return;
   u32* a = db.ot_refs + db.ot_off[lit];
   u64 sz = 0;
   for (u32 k = 0; k < len; k++) sz += csize(db, a[k]);
@@ -1020,27 +1251,43 @@ __device__ void sort_large_list(DB db, const u32* lits, u32 g, u32* scratch, u32
   if (src != a)
     for (u32 k = 0; k < len; k++) a[k] = src[k];
 }
-// grid-stride over the *nbig collected lists (count read on the device)
-__global__ void sort_large_k(DB db, const u32* lits, const u32* big, const u32* nbig, u32* scratch, u32* lsum) {
+// the *nbig collected long lists (the count read on the device: a bounded
+// grid strides over them, so the launch needs no host read of it)
+__global__ void __launch_bounds__(256) sort_long_k(DB db, const u32* pv, const u32* big, const u32* nbig,
+                                                   u32* scratch, u32* lsum) {
+  __shared__ u64 ka[SORT_BLOCK];
+  __shared__ u64 kb[SORT_BLOCK];
+  __shared__ u32 kid[SORT_BLOCK];
+  __shared__ u32 lw[NW];
   const u32 nb = *nbig;
-  for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x)
-    sort_large_list(db, lits, big[i], scratch, lsum);
+  for (u32 b = blockIdx.x; b < nb; b += gridDim.x) {
+    const u32 g = big[b], lit = list_lit(pv, g);
+    if (db.ot_size[lit] <= SORT_BLOCK) sort_block_list(db, lit, g, lsum, ka, kb, kid, lw);
+    else if (threadIdx.x == 0) sort_large_list(db, lit, g, scratch, lsum);
+    __syncthreads();
+  }
 }
-void k_sort_lists(const DB& db, const u32* lits, u32 n, u32* classes, u32* cnt, u32* scratch, u32* lsum,
+void k_sort_lists(const DB& db, const u32* pv, u32 nvars, u32* classes, u32* cnt, u32* scratch, u32* lsum,
                   void* tmp, Stream* st) {
+  const u32 n = 2 * nvars;
   if (!n) return;
   u32* big = classes;           // lists longer than SORT_SMALL
   u32* mid = classes + n;       // lists of SORT_TINY < len <= SORT_SMALL
-  u32* fmid = classes + 2 * (size_t)n;
-  u32* flong = classes + 3 * (size_t)n;
-  u32* pos = classes + 4 * (size_t)n;
-  KLAUNCH(sort_tiny_k, grid_for((size_t)n * SORT_TINY, 256), 256, st, db, lits, n, lsum, fmid, flong);
-  k_pack_flags(fmid, n, pos, mid, cnt + 1, tmp, st);
-  k_pack_flags(flong, n, pos, big, cnt, tmp, st);
+  const unsigned grid = grid_for((size_t)n * SORT_TINY, 256);
+  if (n <= SORT_APPEND_MAX) {
+    KLAUNCH(sort_tiny_k<true>, grid, 256, st, db, pv, n, lsum, mid, big, cnt);
+  } else {
+    u32* fmid = classes + 2 * (size_t)n;
+    u32* flong = classes + 3 * (size_t)n;
+    u32* pmid = classes + 4 * (size_t)n;
+    u32* plong = classes + 5 * (size_t)n;
+    KLAUNCH(sort_tiny_k<false>, grid, 256, st, db, pv, n, lsum, fmid, flong, cnt);
+    scan_set(ScanSet{{flong, fmid}, {plong, pmid}, {cnt, cnt + 1}}, 2, n, tmp, st);
+    KLAUNCH(sort_pack_k, grid_for(n, 256), 256, st, fmid, flong, pmid, plong, n, mid, big);
+  }
   // the collected lists' launches read their counts on the device
-  KLAUNCH(sort_mid_k, std::min(grid_for((size_t)n * SORT_SMALL, 256), 4096u), 256, st, db, lits, mid, cnt + 1, lsum);
-  KLAUNCH(sort_block_k, std::min(grid_for(n, 1), 1024u), 256, st, db, lits, big, cnt, lsum);
-  KLAUNCH(sort_large_k, std::min(grid_for(n, 64), 64u), 64, st, db, lits, big, cnt, scratch, lsum);
+  KLAUNCH(sort_mid_k, std::min(grid_for((size_t)n * SORT_SMALL, 256), 4096u), 256, st, db, pv, mid, cnt + 1, lsum);
+  KLAUNCH(sort_long_k, std::min(n, 1024u), 256, st, db, pv, big, cnt, scratch, lsum);
 }
 
 // ---------------------------------------------------------------- BCP
@@ -1187,13 +1434,14 @@ void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u3
 // The state of an election before its first step: each candidate's packed
 // position and state (undecided, or decided and not elected for the ones
 // passed over) and the counters (sc: [1] the break position, [4..6] and
-// [12..14] the passes' counts), in one launch.  The positions of variables
+// [12..14] the passes' counts, [24..25] the list sort's), in one launch.  The positions of variables
 // that are no candidates are NOPOS from lcve_flag_k.
 __global__ void mis_init_k(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     sc[1] = n;
     for (u32 q = 0; q < 3; q++) sc[4 + q] = 0, sc[12 + q] = 0;
+    sc[24] = sc[25] = 0;
   }
   if (i >= n) return;
   const u32 v = cand[i], st = reject && cflag[v] == 4 ? 2u : 0u;
@@ -1425,9 +1673,6 @@ void k_list_sizes(const DB& db, const u32* pv, u32 n, u32 extra, u32* out, Strea
   if (!n) return;
   KLAUNCH(list_sizes_k, grid_for(n, 256), 256, st, db, pv, n, extra, out);
 }
-// 'order' (nullable) permutes the elected indices so that the heaviest
-// variables start first and share wavefronts with variables of similar work
-
 __global__ void sub_snapshot_k(DB db, const u32* pv, u32 n, SubSnap s) {
   const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < n) sub_snapshot_var(db, pv[k], k, s);
@@ -1512,16 +1757,19 @@ void k_oblivion(const DB& db, const u32* lits, u32 n, Stream* st) {
 // wavefront thus runs variables of like size, the largest first, and no
 // lane that reads the pool holds up lanes that work in LDS.
 //
-// work: LV_WORK_HDR words (the first positions of the sort keys 0..8 in
-// the sorted order), then n sort keys, then n elected indices.  The key
-// of a variable of class c is LV_CLASSES - 1 - c (the largest lists
-// first); VE gives the variables its gate checks settle key LV_CLASSES.
-// A stable radix sort orders the pairs, lv_bounds_k finds where each key
-// starts.  No counter is shared by the variables.
+// work: LV_WORK_HDR words (the first positions of the keys 0..8 in the
+// placed order), then n elected indices.  The key of a variable of class c
+// is LV_CLASSES - 1 - c (the largest lists first); VE execution gives the
+// variables it keeps key LV_CLASSES.  place() orders them; within a class
+// SUB and the VE decisions take the longest lists first (lv_fine), so that
+// the variables of a wavefront have similar work (without it ve_decide_k
+// took 1.11 instead of 0.89 ms on the 2M-gate circuit and sub_k 2.32 instead
+// of 2.06 ms on 10M heavy-tailed variables).
 constexpr u32 LV_CLASSES = 8;
 constexpr u32 LV_WORK_HDR = 32;
 constexpr int LV_KEY_BITS = 4;
-static_assert(LV_CLASSES + 2 <= LV_WORK_HDR && LV_CLASSES < (1u << LV_KEY_BITS), "class keys");
+static_assert(LV_CLASSES + 1 <= LV_WORK_HDR && LV_CLASSES < (1u << LV_KEY_BITS) && LV_CLASSES == LV_KEPT,
+              "class keys");
 __device__ inline u32 lv_class(u32 need, u32 cap) {
   u32 q = 0;
   while (q < LV_CLASSES - 1 && need * (64u >> q) > cap) q++;
@@ -1539,14 +1787,13 @@ __device__ inline u32 lv_class_lanes(u32 q) { return q < LV_CLASSES - 1 ? 64u >>
 #ifndef LV_FILL
 #define LV_FILL 4
 #endif
-__global__ void lv_bounds_k(const u32* keys, u32 n, u32* starts) {
-  const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && (i == 0 || keys[i] != keys[i - 1])) starts[keys[i]] = i;
-}
-// sorts the (key, elected index) pairs and finds the key starts
-void lv_sort(u32* work, u32 n, void* tmp, Stream* st) {
-  radix_sort_pairs(work + LV_WORK_HDR, work + LV_WORK_HDR + n, n, LV_KEY_BITS, tmp, st);
-  KLAUNCH(lv_bounds_k, grid_for(n, 256), 256, st, work + LV_WORK_HDR, n, work);
+// list occurrences as a descending 5-bit code: exact below 16, then four
+// steps per power of two up to 256
+constexpr int LV_FINE_BITS = 5;
+__device__ inline u32 lv_fine(u32 w) {
+  if (w < 16) return 31 - w;
+  const u32 e = 31 - __clz(w);
+  return 31 - min(31u, 16 + (e - 4) * 4 + ((w >> (e - 2)) & 3u));
 }
 // one wavefront per workgroup, grid-stride over the chunks of all classes;
 // f(k, w, slice, gl, G) runs elected index k with the LDS words
@@ -1558,16 +1805,10 @@ void lv_sort(u32* work, u32 n, void* tmp, Stream* st) {
 template <class F>
 __device__ inline void lv_chunks(const u32* work, u32 n, u32 cap, u32* lds, F f) {
   const u32 lane = threadIdx.x;
-  const u32* placed = work + LV_WORK_HDR + n;
-  // key starts (absent keys start where the next key starts)
-  u32 start[LV_CLASSES + 1];
-  u32 next = n;
+  const u32* placed = work + LV_WORK_HDR;
+  u32 start[LV_CLASSES + 1];  // absent keys start where the next key starts
 #pragma unroll
-  for (int key = LV_CLASSES; key >= 0; key--) {
-    const u32 s0 = work[key];
-    start[key] = s0 < n ? s0 : next;
-    next = start[key];
-  }
+  for (u32 key = 0; key <= LV_CLASSES; key++) start[key] = work[key];
   u32 chunks = 0;
 #pragma unroll
   for (u32 key = 0; key < LV_CLASSES; key++) {
@@ -1624,18 +1865,19 @@ static u32 lv_floor(u32 n) {
 #ifndef VE_CLASS_BUMP
 #define VE_CLASS_BUMP 1
 #endif
-__global__ void ve_class_k(DB db, const u32* pv, u32 n, const u32* order, u32* work, const u32* lsum, u32 cap,
-                           u32 least) {
-  const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const u32 k = order ? order[t] : t;
-  const u32 p = V2L(pv[k]);
-  const u64 b = lview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
-  u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
-  if (c < LV_CLASSES - 1) c = max(least, min(c + VE_CLASS_BUMP, LV_CLASSES - 2));
-  work[LV_WORK_HDR + t] = LV_CLASSES - 1 - c;
-  work[LV_WORK_HDR + n + t] = k;
-}
+struct VeClass {
+  DB db;
+  const u32 *pv, *lsum;
+  u32 cap, least, fine;
+  __device__ u32 val(u32 k) const { return k; }
+  __device__ u32 key(u32 k) const {
+    const u32 p = V2L(pv[k]), w = db.ot_size[p] + db.ot_size[p | 1];
+    const u64 b = lview_bound(w, (u64)lsum[2 * k] + lsum[2 * k + 1]);
+    u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
+    if (c < LV_CLASSES - 1) c = max(least, min(c + VE_CLASS_BUMP, LV_CLASSES - 2));
+    return ((LV_CLASSES - 1 - c) << LV_FINE_BITS) | (fine ? lv_fine(w) : 0u);
+  }
+};
 // every elected variable on an LDS copy of its lists (the checks read each
 // clause of the lists once, into LDS, instead of once per check from the
 // pool), the gate checks, searches and resolvent count shared by the group
@@ -1656,13 +1898,12 @@ __global__ void ve_decide_k(DB db, Options o, const u32* pv, VeDecision d, const
     }
   });
 }
-void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeDecision& d, const u32* order,
-                 u32* work, const u32* lsum, void* tmp, Stream* st) {
+void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeDecision& d, u32* work,
+                 const u32* lsum, void* tmp, Stream* st) {
   if (!n) return;
   const u32 cap = VR_LDS / 4;
-  fill_u32(work, n, LV_WORK_HDR, st);
-  KLAUNCH(ve_class_k, grid_for(n, 256), 256, st, db, pv, n, order, work, lsum, cap, lv_floor(n));
-  lv_sort(work, n, tmp, st);
+  place(VeClass{db, pv, lsum, cap, lv_floor(n), (u32)o.work_order}, n, 8, work + LV_WORK_HDR, work, LV_CLASSES + 1,
+        LV_FINE_BITS, nullptr, 0, tmp, st);
   KLAUNCH_LDS(ve_decide_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, o, pv, d, work, n, cap);
 }
 // SUB, staged as the VE searches (the class of a variable from the words of
@@ -1670,17 +1911,19 @@ void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeD
 #ifndef SUB_CLASS_BUMP
 #define SUB_CLASS_BUMP 0
 #endif
-__global__ void sub_class_k(DB db, const u32* pv, const u32* idx, u32 n, u32* work, const u32* lsum, u32 cap,
-                            u32 least) {
-  const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const u32 k = idx ? idx[t] : t, p = V2L(pv[k]);
-  const u64 b = sview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
-  u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
-  if (c < LV_CLASSES - 1) c = max(least, min(c + SUB_CLASS_BUMP, LV_CLASSES - 2));
-  work[LV_WORK_HDR + t] = LV_CLASSES - 1 - c;
-  work[LV_WORK_HDR + n + t] = k;
-}
+struct SubClass {
+  DB db;
+  const u32 *pv, *idx, *lsum;
+  u32 cap, least, fine;
+  __device__ u32 val(u32 t) const { return idx ? idx[t] : t; }
+  __device__ u32 key(u32 t) const {
+    const u32 k = val(t), p = V2L(pv[k]), w = db.ot_size[p] + db.ot_size[p | 1];
+    const u64 b = sview_bound(w, (u64)lsum[2 * k] + lsum[2 * k + 1]);
+    u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
+    if (c < LV_CLASSES - 1) c = max(least, min(c + SUB_CLASS_BUMP, LV_CLASSES - 2));
+    return ((LV_CLASSES - 1 - c) << LV_FINE_BITS) | (fine ? lv_fine(w) : 0u);
+  }
+};
 // take_snap: record each variable's state for the SUB re-runs just before
 // its run (a run changes only the variable's own lists and clauses, so this
 // equals a snapshot before the launch); the staged copy provides it
@@ -1708,9 +1951,8 @@ void k_sub(const DB& db, const Options& o, const u32* pv, const u32* idx, u32 n,
            const u32* lsum, void* tmp, const SubSnap* snap, Stream* st) {
   if (!n) return;
   const u32 cap = VR_LDS / 4;
-  fill_u32(work, n, LV_WORK_HDR, st);
-  KLAUNCH(sub_class_k, grid_for(n, 256), 256, st, db, pv, idx, n, work, lsum, cap, lv_floor(n));
-  lv_sort(work, n, tmp, st);
+  place(SubClass{db, pv, idx, lsum, cap, lv_floor(n), (u32)o.work_order}, n, 8, work + LV_WORK_HDR, work,
+        LV_CLASSES + 1, LV_FINE_BITS, out.n, 1, tmp, st);
   KLAUNCH_LDS(sub_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, o, pv, work, n, cap, out,
               snap ? *snap : SubSnap{}, snap ? 1u : 0u);
 }
@@ -1719,12 +1961,13 @@ void k_sub(const DB& db, const Options& o, const u32* pv, const u32* idx, u32 n,
 // in place) work on the pool, EQU_CLASS lanes' worth or more each; variables
 // VE keeps are not placed
 constexpr u32 EQU_CLASS = 3;
-__global__ void ve_apply_class_k(DB db, const u32* pv, u32 n, const u32* type, u32* work, const u32* lsum,
-                                 u32 cap, u32 least) {
-  const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  u32 key = LV_CLASSES;
-  if (type[k]) {
+struct ApplyClass {
+  DB db;
+  const u32 *pv, *type, *lsum;
+  u32 cap, least;
+  __device__ u32 val(u32 t) const { return t; }
+  __device__ u32 key(u32 k) const {
+    if (!type[k]) return LV_CLASSES;
     u32 c = EQU_CLASS;
     if (type[k] != VT_EQU) {
       const u32 p = V2L(pv[k]);
@@ -1732,11 +1975,9 @@ __global__ void ve_apply_class_k(DB db, const u32* pv, u32 n, const u32* type, u
       c = lv_class((u32)min(b, (u64)cap + 1), cap);
     }
     if (c < LV_CLASSES - 1) c = max(c, least);
-    key = LV_CLASSES - 1 - c;
+    return LV_CLASSES - 1 - c;
   }
-  work[LV_WORK_HDR + k] = key;
-  work[LV_WORK_HDR + n + k] = k;
-}
+};
 __global__ void ve_apply_k(DB db, const u32* pv, VeDecision d, VeApply a, const u32* work, u32 n, u32 cap) {
   extern __shared__ u32 lds[];
   lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
@@ -1751,19 +1992,19 @@ __global__ void ve_apply_k(DB db, const u32* pv, VeDecision d, VeApply a, const 
   });
 }
 void k_ve_apply(const DB& db, const u32* pv, u32 n, const VeDecision& d, const VeApply& a, u32* work,
-                const u32* lsum, void* tmp, Stream* st) {
+                const u32* lsum, u32* zero, u32 nz, void* tmp, Stream* st) {
   if (!n) return;
   const u32 cap = VR_LDS / 4;
-  fill_u32(work, n, LV_WORK_HDR, st);
-  KLAUNCH(ve_apply_class_k, grid_for(n, 256), 256, st, db, pv, n, d.type, work, lsum, cap, lv_floor(n));
-  lv_sort(work, n, tmp, st);
+  place(ApplyClass{db, pv, d.type, lsum, cap, lv_floor(n)}, n, LV_KEY_BITS, work + LV_WORK_HDR, work, LV_CLASSES + 1,
+        0, zero, nz, tmp, st);
   KLAUNCH_LDS(ve_apply_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, pv, d, a, work, n, cap);
 }
+// in elected order (by score, so of similar lists): heaviest lists first took
+// 0.69 instead of 0.61 ms for the two launches on 2.5M heavy-tailed variables
 __global__ void bce_k(DB db, Options o, const u32* pv, const u32* type, u32 n, u32* words,
-                      const u32* base, u32* stack, bool count, const u32* order) {
-  const u32 t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const u32 k = order ? order[t] : t;
+                      const u32* base, u32* stack, bool count) {
+  const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= n) return;
   if (type && type[k]) {
     if (count) words[k] = 0;
     return;
@@ -1772,30 +2013,9 @@ __global__ void bce_k(DB db, Options o, const u32* pv, const u32* type, u32 n, u
   else bce_var(db, o, pv[k], false, stack + base[k]);
 }
 void k_bce(const DB& db, const Options& o, const u32* pv, const u32* type, u32 n, u32* words,
-           const u32* base, u32* stack, bool count, const u32* order, Stream* st) {
+           const u32* base, u32* stack, bool count, Stream* st) {
   if (!n) return;
-  KLAUNCH(bce_k, grid_for(n, VB), VB, st, db, o, pv, type, n, words, base, stack, count, order);
-}
-// the launch order's key: list occurrences on an 8-bit log-linear scale
-// (exact below 64, then 16 steps per power of two up to 2^18), descending,
-// so the sort takes two radix passes instead of four; ties keep the elected
-// order
-__device__ inline u32 work_code(u32 w) {
-  if (w < 64) return w;
-  const u32 e = 31 - __clz(w);
-  return min(255u, 64 + (e - 6) * 16 + ((w >> (e - 4)) & 15u));
-}
-__global__ void work_keys_k(DB db, const u32* pv, u32 n, u32* key, u32* idx) {
-  const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const u32 w = db.ot_size[V2L(pv[k])] + db.ot_size[V2L(pv[k]) | 1];
-  key[k] = 255u - work_code(w);
-  idx[k] = k;
-}
-void k_work_order(const DB& db, const u32* pv, u32 n, u32* key, u32* order, void* tmp, Stream* st) {
-  if (!n) return;
-  KLAUNCH(work_keys_k, grid_for(n, 256), 256, st, db, pv, n, key, order);
-  radix_sort_pairs(key, order, n, 8, tmp, st);
+  KLAUNCH(bce_k, grid_for(n, VB), VB, st, db, o, pv, type, n, words, base, stack, count);
 }
 __global__ void ere_k(DB db, Options o, const u32* pv, u32 from, u32 n, EreOut out) {
   const u32 k = from + blockIdx.x * blockDim.x + threadIdx.x;
@@ -1892,16 +2112,6 @@ __global__ void assign_units_k(DB db, const u32* lits, u32 n) {
 void k_assign_units(const DB& db, const u32* lits, u32 n, Stream* st) {
   if (!n) return;
   KLAUNCH(assign_units_k, grid_for(n, 256), 256, st, db, lits, n);
-}
-__global__ void pv_lits_k(const u32* pv, u32 n, u32* lits) {
-  const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  lits[2 * k] = V2L(pv[k]);
-  lits[2 * k + 1] = V2L(pv[k]) | 1;
-}
-void k_pv_lits(const u32* pv, u32 n, u32* lits, Stream* st) {
-  if (!n) return;
-  KLAUNCH(pv_lits_k, grid_for(n, 256), 256, st, pv, n, lits);
 }
 __global__ void max_list_k(DB db, const u32* lits, u32 n, u32* out) {
   u32 m = 0;
@@ -2721,16 +2931,6 @@ __global__ void els_rep_k(DB db, const u32* root, u32* rep, u32* info) {
     subs += rep[l] != l;
   }
   block_count_add(subs, lw, &info[1]);
-}
-__global__ void count_nonzero_k(const u32* a, u32 n, u32* out) {
-  __shared__ u32 lw[NW];
-  u32 mine = 0;
-  for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) mine += a[i] != 0;
-  block_count_add(mine, lw, out);
-}
-void k_count_nonzero(const u32* a, u32 n, u32* out, Stream* st) {
-  fill_u32(out, 0, 1, st);
-  if (n) KLAUNCH(count_nonzero_k, std::min(grid_for(n, ST), RED_BLOCKS), ST, st, a, n, out);
 }
 void k_els_rep(const DB& db, const u32* root, u32* rep, u32* info, Stream* st) {
   KLAUNCH(els_rep_k, std::min(grid_for(2 * (size_t)db.nvars + 2, ST), RED_BLOCKS), ST, st, db, root, rep, info);

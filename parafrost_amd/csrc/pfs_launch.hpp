@@ -58,6 +58,9 @@ size_t scan_tmp_bytes(size_t n);
 // exclusive prefix sum of n u32 values; out may alias in; *total (device)
 // receives the sum when non-null
 void scan_u32(const u32* in, u32* out, size_t n, u32* total, void* tmp, Stream*);
+// the same over three arrays at once (total: three words; tmp: 3 *
+// scan_tmp_bytes(n))
+void scan3_u32(const u32* const (&in)[3], u32* const (&out)[3], size_t n, u32* total, void* tmp, Stream*);
 size_t radix_tmp_bytes(size_t n);
 // stable sort of (key, val) pairs by the low 'bits' bits of key
 void radix_sort_pairs(u32* keys, u32* vals, size_t n, int bits, void* tmp, Stream*);
@@ -87,11 +90,11 @@ bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2 = 0, int xcd = 0
 // hist = ot_size.  tmp: scan_tmp_bytes(p.ncounts)
 void k_ot_ranges(const DB& db, const OtpPlan& p, u32 n2, u32* counts, void* pairs, bool table, u32* hist,
                  void* tmp, Stream*);
-// sort the lists of the given literals (lits[0..n)) by the total order
-// classes: 5n words of scratch for the size classes; cnt: 3 device words;
-// tmp: scan_tmp_bytes(n)
-// lsum[i]: sum of the clause sizes of list lits[i] (n words)
-void k_sort_lists(const DB& db, const u32* lits, u32 n, u32* classes, u32* cnt, u32* scratch, u32* lsum, void* tmp,
+// sort the two lists of each variable pv[0..nvars) by the total order
+// classes: 12 * nvars words of scratch; cnt: 2 device words, zero; tmp:
+// 2 * scan_tmp_bytes(2 * nvars)
+// lsum[2k], lsum[2k + 1]: sums of the clause sizes of pv[k]'s lists
+void k_sort_lists(const DB& db, const u32* pv, u32 nvars, u32* classes, u32* cnt, u32* scratch, u32* lsum, void* tmp,
                   Stream*);
 
 // ---- BCP
@@ -118,7 +121,7 @@ void k_lcve_classify(const DB& db, const LcveArgs& a, Stream*);
 void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u32* key, u32* pos, u32* ncand,
                    void* tmp, Stream*);
 // the state before the first step: positions, states, counters (sc[1] = n,
-// sc[4..6] = sc[12..14] = 0).  reject: candidates passed over for an oversize
+// sc[4..6] = sc[12..14] = sc[24..25] = 0).  reject: candidates passed over for an oversize
 // clause (cflag 4) start decided and not elected: they neither block nor
 // freeze a neighbour
 void k_mis_init(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc, Stream*);
@@ -146,7 +149,8 @@ void k_list_sizes(const DB& db, const u32* pv, u32 n, u32 extra, u32* out, Strea
 // work: 2 n + 32 words of scratch (size classes and placement); lsum: the
 // list size sums of k_sort_lists over the elected literals (2k, 2k + 1);
 // tmp: radix_tmp_bytes(n); snap (nullable): take the re-run snapshot of
-// every variable run (as k_sub_snapshot would before the launch)
+// every variable run (as k_sub_snapshot would before the launch); *out.n is
+// cleared first
 void k_sub(const DB& db, const Options& o, const u32* pv, const u32* idx, u32 n, const SubOut& out, u32* work,
            const u32* lsum, void* tmp, const SubSnap* snap, Stream*);
 void k_sub_snapshot(const DB& db, const u32* pv, u32 n, const SubSnap& s, Stream*);
@@ -161,19 +165,18 @@ void k_set_vis(u32* ust, u32* ulit, const u32* entries, u32 n, Stream*);  // tri
 // indices of the nonzero flags, in order; pos: n words of scratch
 void k_pack_flags(const u32* flags, u32 n, u32* pos, u32* out, u32* count, void* tmp, Stream*);
 void k_oblivion(const DB& db, const u32* lits, u32 n, Stream*);  // delete all clauses of the lists
-void k_count_nonzero(const u32* a, u32 n, u32* out, Stream*);    // *out = number of nonzero a[i]
 // work, lsum, tmp: as for k_sub (the variables the gate checks leave open
 // are staged by size class)
-void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeDecision& d, const u32* order,
-                 u32* work, const u32* lsum, void* tmp, Stream*);
+void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeDecision& d, u32* work,
+                 const u32* lsum, void* tmp, Stream*);
 // work, lsum, tmp: as for k_sub
+// zero[0..nz): words cleared before the kernel runs (its counters);
+// work[LV_KEPT] receives the number of eliminated variables
+constexpr u32 LV_KEPT = 8;
 void k_ve_apply(const DB& db, const u32* pv, u32 n, const VeDecision& d, const VeApply& a, u32* work,
-                const u32* lsum, void* tmp,
-                Stream*);
+                const u32* lsum, u32* zero, u32 nz, void* tmp, Stream*);
 void k_bce(const DB& db, const Options& o, const u32* pv, const u32* type, u32 n, u32* words,
-           const u32* base, u32* stack, bool count, const u32* order, Stream*);
-// heaviest-first permutation of the elected indices (key: scratch of n words)
-void k_work_order(const DB& db, const u32* pv, u32 n, u32* key, u32* order, void* tmp, Stream*);
+           const u32* base, u32* stack, bool count, Stream*);
 void k_ere(const DB& db, const Options& o, const u32* pv, u32 from, u32 n, const EreOut& out,
            Stream*);
 void k_ere_dirty(const DB& db, const u32* pv, u32 from, u32 n, const u32* del_by, u32* first,
@@ -189,7 +192,6 @@ void k_ere_all_matches(const DB& db, const ErePairs& a, u32 n, const u32* off, u
 
 // ---- small helpers
 void k_assign_units(const DB& db, const u32* lits, u32 n, Stream*);  // assign + FROZEN
-void k_pv_lits(const u32* pv, u32 n, u32* lits, Stream*);            // 2 literals per variable
 void k_max_list(const DB& db, const u32* lits, u32 n, u32* out, Stream*);
 void k_reduce_lists(const DB& db, Stream*);  // drop deleted entries from every list
 void k_prep(const DB& db, u32 first, Stream*);  // clauses [first, ncls): sort literals, signature
