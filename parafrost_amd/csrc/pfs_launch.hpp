@@ -100,6 +100,9 @@ void k_sort_lists(const DB& db, const u32* pv, u32 nvars, u32* classes, u32* cnt
 // ---- BCP
 void k_bcp_visit(const DB& db, const u32* front, u32 nfront, u32* next, u32* nnext, u32* conflict,
                  Stream*);
+// levels from trail[front..end) on while they are narrow; out: the trail's
+// end, whether a conflict was met, the first literal not propagated yet
+void k_bcp_run(const DB& db, u32* trail, u32 front, u32 end, u32* out, Stream*);
 void k_bcp_mark(const DB& db, const u32* lits, u32 n, u8* mark, Stream*);
 void k_bcp_clean(const DB& db, u8* mark, Stream*);
 void k_clear_lists(const DB& db, const u32* lits, u32 n, Stream*);
