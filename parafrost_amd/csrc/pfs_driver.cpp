@@ -2199,10 +2199,11 @@ void Simplifier::download_cnf(uint64_t* offsets, uint32_t* lits, uint8_t* flags,
   uint8_t* base = P<uint8_t>(out_);
   k_pack_cnf(make_db(cur_), P<u32>(tmp2_), tmp_.p, P<u32>(scal_) + 56, (u64*)(base + o_off), (u32*)(base + o_lits),
              base + o_flags, (u32*)(base + o_lbd), st_);
-  if (offsets) d2h(offsets, base + o_off, 8 * (n + 1), st_);
-  if (lits) d2h(lits, base + o_lits, 4 * nl, st_);
-  if (flags) d2h(flags, base + o_flags, n, st_);
-  if (lbd) d2h(lbd, base + o_lbd, 4 * n, st_);
+  const D2H set[4] = {{offsets, base + o_off, offsets ? 8 * (n + 1) : 0},
+                      {lits, base + o_lits, lits ? 4 * nl : 0},
+                      {flags, base + o_flags, flags ? n : 0},
+                      {lbd, base + o_lbd, lbd ? 4 * n : 0}};
+  d2h_set(set, 4, st_);
   stream_sync(st_);
 }
 

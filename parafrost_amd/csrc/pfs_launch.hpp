@@ -26,6 +26,13 @@ void* dev_alloc(size_t bytes);  // throws std::bad_alloc on failure
 void dev_free(void*);
 void h2d(void* dst, const void* src, size_t bytes, Stream*);
 void d2h(void* dst, const void* src, size_t bytes, Stream*);
+// several downloads; large ones through the pinned ring, done on return
+struct D2H {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+void d2h_set(const D2H* set, u32 n, Stream*);
 void d2d(void* dst, const void* src, size_t bytes, Stream*);
 void fill_u32(u32* dst, u32 value, size_t n, Stream*);  // fill kernel, no memset nodes
 void fill_u8(u8* dst, u8 value, size_t n, Stream*);
