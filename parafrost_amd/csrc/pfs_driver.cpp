@@ -165,7 +165,7 @@ void Simplifier::alloc_state() {
   mem_.ensure(mark_, lcap_, 0, st_);  // per clause handle
   const size_t big = std::max<size_t>({V1 + 2, L2 + 1, ccap_});
   mem_.ensure(tmp_, std::max(scan_tmp_bytes(big), radix_tmp_bytes(V1 + 1)), 0, st_);
-  mem_.ensure(scal_, 256, 0, st_);
+  mem_.ensure(scal_, 512, 0, st_);
   mem_.ensure(stack_, (size_t)1 << 20, 0, st_);
 }
 
@@ -1003,11 +1003,11 @@ bool Simplifier::lcve() {
   if (prop_changed_) ot_counts(false);
   u32* sc = P<u32>(scal_);
   u64* hard = (u64*)(sc + 16);
-  fill_u32((u32*)hard, INF, 2, st_);
   LcveArgs a;
   a.hist = hist;
   a.score = P<u32>(score_);
   a.hard = hard;
+  a.top = sc + 64;
   a.cflag = P<u8>(cflag_);
   a.pt = (u32)opt.mu_pos << mu_inc_;
   a.nt = (u32)opt.mu_neg << mu_inc_;
@@ -1015,18 +1015,16 @@ bool Simplifier::lcve() {
   a.clause_max = opt.lcve_clause_max == INT32_MAX ? INF : (u32)opt.lcve_clause_max;
   k_lcve_classify(db, a, st_);
   k_lcve_select(db, a, P<u32>(flag_), P<u32>(cand_), P<u32>(key_), P<u32>(pos_), sc, tmp_.p, st_);
-  u32 h[4];
+  u32 h[3], tops[LCVE_TOPS];  // candidates, hard breaker's variable and score; largest scores
   d2h(h, sc, 4, st_);
-  d2h(h + 2, hard, 8, st_);
+  d2h(h + 1, hard, 8, st_);
+  d2h(tops, a.top, sizeof(tops), st_);
   stream_sync(st_);
   const u32 ncand = h[0];
-  const u64 hk = ((u64)h[3] << 32) | h[2];
-  int bits = 32;
-  if (hk != ~0ull) {
-    const u32 hs = (u32)(hk >> 32);
-    bits = 0;
-    while (bits < 32 && (hs >> bits)) bits++;
-  }
+  // the candidates stay below the hard breaker and at most at the largest score
+  const u32 most = std::min(h[2], *std::max_element(tops, tops + LCVE_TOPS));
+  int bits = 0;
+  while (bits < 32 && (most >> bits)) bits++;
   radix_sort_pairs(P<u32>(key_), P<u32>(cand_), ncand, bits, tmp_.p, st_);
   // positions share a word with the candidate's state (position << 2)
   if (ncand >= (1u << 30)) throw DeviceFail{"LCVE: too many candidates for the packed positions"};
@@ -1121,20 +1119,26 @@ bool Simplifier::lcve() {
   // the elected variables collected behind the passes queued so far; the one
   // read that brings their number also tells whether candidates were left
   // undecided, which takes more passes and another collection
-  u32 w15[15];  // sc[0]: elected, sc[6]: worklist passes with work, sc[12..14]: the ring
+  // SUB's room from the same read, unless the candidates are so many that
+  // reading their list sizes once more costs more than a read (0.1 ms for 2.5M)
+  const bool with_entries = ncand <= (1u << 18);
+  u32 w15[15];  // sc[0]: elected, sc[3]: entries of their lists, sc[6]: worklist passes with work, sc[12..14]: the ring
   while (true) {
     k_mis_break(P<u32>(cand_), ncand, P<u8>(cflag_), P<u32>(state_), sc + 1, st_);
     // the worklist still to be read must stay: the other one is free
-    k_mis_collect(P<u32>(cand_), ncand, P<u32>(state_), 0, wl[(p + 1) & 1], P<u32>(pv_), sc, tmp_.p, st_);
+    k_mis_collect(db, P<u32>(cand_), ncand, P<u32>(state_), wl[(p + 1) & 1], P<u32>(pv_), sc, with_entries, tmp_.p,
+                  st_);
     d2h(w15, sc, sizeof(w15), st_);
     stream_sync(st_);
     const u32 bound = ncand ? w15[12 + p % 3] : 0;
     if (!bound) break;
     fill_u32(sc + 1, ncand, 1, st_);
+    fill_u32(sc + 3, 0, 1, st_);
     passes(bound, (u32)used_lds_, lanes);
   }
   const u32* w7 = w15;
   E_ = w7[0];
+  elected_entries_ = with_entries ? w7[3] : NOPOS;
   rounds_.back().elected = E_;
   rounds_.back().mis_iterations = ncand ? 1 + w7[6] : 0;
   stage_end();
@@ -1187,7 +1191,7 @@ bool Simplifier::sub() {
   u32* sc = P<u32>(scal_);
   k_list_sizes(db, P<u32>(pv_), E_, 0, P<u32>(vsz_), st_);
   scan_u32(P<u32>(vsz_), P<u32>(vbase_), E_, sc + 5, tmp_.p, st_);
-  const u32 O = read_u32(sc + 5);
+  const u32 O = elected_entries_ != NOPOS ? elected_entries_ : read_u32(sc + 5);
   const size_t ob = std::max<size_t>(O, 1);
   mem_.ensure(snap_ref_, ob * 4, 0, st_);
   mem_.ensure(snap_flg_, ob, 0, st_);
@@ -1404,7 +1408,7 @@ bool Simplifier::sub() {
   }
   proof_events(pev);
   proof_flush();
-  stream_sync(st_);
+  if (pass > 1 || !committed.empty()) stream_sync(st_);  // host lists still being copied
   rounds_.back().units += (u32)committed.size();
   rounds_.back().sub_passes = pass;
   stage_end();
@@ -1527,7 +1531,6 @@ void Simplifier::bce() {
     stack_n_ += T;
     rounds_.back().stack_words += T;
   }
-  stream_sync(st_);
   stage_end();
 }
 

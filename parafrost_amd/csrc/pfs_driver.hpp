@@ -239,6 +239,7 @@ class Simplifier {
   // LCVE
   Buf score_, cflag_, flag_, cand_, key_, pos_, state_, pv_;
   uint32_t E_ = 0;
+  uint32_t elected_entries_ = 0;  // entries of the elected variables' lists (NOPOS: not summed)
   // per elected variable
   Buf vsz_, vbase_, type_, def_, vncls_, vnlits_, vnstack_, clsb_, litb_, stkb_;
   Buf snap_ref_, snap_flg_, snap_size_, snap_sig_, snap_lbd_, snap_np_, snap_nn_, scratch_;

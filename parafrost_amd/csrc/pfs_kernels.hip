@@ -18,6 +18,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -54,6 +55,19 @@ struct PinCopy {
   void* dst;
   size_t off, bytes;
 };
+// The smallest reads (a few counters before every wait) are gathered and
+// written to the pinned area by one kernel launched when the caller waits,
+// with a flag behind them that the waiting thread polls: a counter read
+// takes 9.9 us after its kernel that way, 14.3 with a copy and a wait for the
+// stream (a small formula's round waits eight times).  Anything else put on
+// the stream before the wait launches the gathered reads first, so a read
+// sees what the stream held when it was asked for.
+constexpr u32 PUB_MAX = 6, PUB_BYTES = 256;
+struct PubSet {
+  const u32* src[PUB_MAX];
+  u32* dst[PUB_MAX];
+  u32 words[PUB_MAX];
+};
 struct Stream {
   hipStream_t s;
   int device;
@@ -62,7 +76,16 @@ struct Stream {
   unsigned char* pin = nullptr;  // PIN_BYTES of pinned host memory
   size_t pin_used = 0;
   std::vector<PinCopy> pend;     // staged reads not yet copied out
+  PubSet pub = {};               // gathered reads, not launched yet
+  u32 npub = 0;
+  u32* flag = nullptr;           // in the pinned area, past PIN_BYTES
+  u32 tag = 0;                   // its value once the last gathered reads have landed
 };
+static void pub_flush(Stream* st, bool flagged);
+// before anything is put on the stream
+static inline void stream_op(Stream* st) {
+  if (st->npub) pub_flush(st, false);
+}
 static void pin_flush(Stream* st) {
   for (const PinCopy& c : st->pend) memcpy(c.dst, st->pin + c.off, c.bytes);
   st->pend.clear();
@@ -81,6 +104,7 @@ static inline unsigned grid_for(size_t n, unsigned block) {
 // the same with 'lds' bytes of dynamic LDS reserved per workgroup
 #define KLAUNCH_LDS(kern, grid, block, lds, st, ...)          \
   do {                                                         \
+    stream_op(st);                                             \
     hipEvent_t e0_ = nullptr;                                  \
     if ((st)->prof) {                                          \
       PFS_HIP(hipEventCreate(&e0_));                           \
@@ -97,6 +121,36 @@ static inline unsigned grid_for(size_t n, unsigned block) {
   } while (0)
 
 // ---------------------------------------------------------------- runtime
+__global__ void publish_k(PubSet p, u32 n, u32* flag, u32 tag) {
+  for (u32 q = 0; q < n; q++)
+    for (u32 i = threadIdx.x; i < p.words[q]; i += 64) p.dst[q][i] = p.src[q][i];
+  if (!flag) return;
+  __threadfence_system();
+  if (threadIdx.x == 0) __hip_atomic_store(flag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+static void pub_flush(Stream* st, bool flagged) {
+  const u32 n = st->npub;
+  st->npub = 0;  // first: the launch below is itself an operation on the stream
+  if (flagged) st->tag++;
+  publish_k<<<1, 64, 0, st->s>>>(st->pub, n, flagged ? st->flag : nullptr, st->tag);
+  LAUNCH_CHECK();
+}
+// waits for the flag of the gathered reads, giving the core away between
+// polls once the wait is longer than a launch; false when it is not there
+// after 20 ms (a long queue, or a device error): the caller waits for the
+// stream, which reports errors.  (Giving up after 0.3 ms cost a call on 10M
+// variables, which waits for millisecond kernels, 0.13 ms.)
+static bool pub_wait(Stream* st) {
+  pub_flush(st, true);
+  const auto t0 = std::chrono::steady_clock::now();
+  while (true) {
+    for (int i = 0; i < 256; i++)
+      if (__atomic_load_n(st->flag, __ATOMIC_ACQUIRE) == st->tag) return true;
+    const auto dt = std::chrono::steady_clock::now() - t0;
+    if (dt > std::chrono::milliseconds(20)) return false;
+    if (dt > std::chrono::microseconds(50)) std::this_thread::yield();
+  }
+}
 static void staging_retain();
 static void staging_release();
 Stream* stream_create(int device) {
@@ -104,13 +158,18 @@ Stream* stream_create(int device) {
   Stream* st = new Stream();
   st->device = device;
   PFS_HIP(hipStreamCreateWithFlags(&st->s, hipStreamNonBlocking));
-  if (hipHostMalloc((void**)&st->pin, PIN_BYTES, hipHostMallocDefault) != hipSuccess) st->pin = nullptr;
+  if (hipHostMalloc((void**)&st->pin, PIN_BYTES + 256, hipHostMallocCoherent) != hipSuccess) st->pin = nullptr;
+  if (st->pin) {
+    st->flag = (u32*)(st->pin + PIN_BYTES);
+    *st->flag = 0;
+  }
   staging_retain();
   return st;
 }
 void prof_enable(Stream* st, bool on) { st->prof = on; }
 void stream_bind(Stream* st) { PFS_HIP(hipSetDevice(st->device)); }
 void prof_collect(Stream* st, std::vector<KernelTime>& out) {
+  stream_op(st);
   PFS_HIP(hipStreamSynchronize(st->s));
   pin_flush(st);
   std::map<std::string, size_t> idx;
@@ -147,10 +206,15 @@ void stream_destroy(Stream* st) {
   staging_release();
 }
 void stream_sync(Stream* st) {
+  if (st->npub && pub_wait(st)) {  // the flag follows everything queued before it
+    pin_flush(st);
+    return;
+  }
   const hipError_t e = hipStreamSynchronize(st->s);
   if (e != hipSuccess) {
     // the staged reads did not complete: drop them (their destinations are
     // locals of frames the exception unwinds), then report
+    st->npub = 0;
     st->pend.clear();
     st->pin_used = 0;
     throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e) + " at " + __FILE__ + ":" +
@@ -160,6 +224,7 @@ void stream_sync(Stream* st) {
 }
 bool stream_quiesce(Stream* st) {
   if (!st) return true;
+  st->npub = 0;
   const bool ok = hipStreamSynchronize(st->s) == hipSuccess;
   if (!ok) (void)hipGetLastError();
   st->pend.clear();
@@ -182,6 +247,7 @@ void dev_free(void* p) {
 // data is copied there first; the area is reused only after stream_sync)
 void h2d(void* dst, const void* src, size_t bytes, Stream* st) {
   if (!bytes) return;
+  stream_op(st);
   if (st->pin && bytes <= PIN_SMALL) {
     if (st->pin_used + bytes > PIN_BYTES) stream_sync(st);
     memcpy(st->pin + st->pin_used, src, bytes);
@@ -250,6 +316,7 @@ static void staging_release() {
   g_staging.drop();
 }
 void d2h_set(const D2H* set, u32 n, Stream* st) {
+  stream_op(st);
   size_t total = 0;
   for (u32 i = 0; i < n; i++) total += set[i].bytes;
   std::unique_lock<std::mutex> lk(g_staging.use, std::defer_lock);
@@ -326,14 +393,26 @@ void d2h(void* dst, const void* src, size_t bytes, Stream* st) {
   }
   if (st->pin && bytes <= PIN_SMALL) {
     if (st->pin_used + bytes > PIN_BYTES) stream_sync(st);
+    if (bytes <= PUB_BYTES && (bytes & 3) == 0 && ((uintptr_t)src & 3) == 0) {
+      if (st->npub == PUB_MAX) pub_flush(st, false);
+      st->pub.src[st->npub] = (const u32*)src;
+      st->pub.dst[st->npub] = (u32*)(st->pin + st->pin_used);
+      st->pub.words[st->npub++] = (u32)(bytes / 4);
+      st->pend.push_back(PinCopy{dst, st->pin_used, bytes});
+      st->pin_used += (bytes + 15) & ~(size_t)15;
+      return;
+    }
+    stream_op(st);
     PFS_HIP(hipMemcpyAsync(st->pin + st->pin_used, src, bytes, hipMemcpyDeviceToHost, st->s));
     st->pend.push_back(PinCopy{dst, st->pin_used, bytes});
     st->pin_used += (bytes + 15) & ~(size_t)15;
     return;
   }
+  stream_op(st);
   PFS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st->s));
 }
 void d2d(void* dst, const void* src, size_t bytes, Stream* st) {
+  stream_op(st);
   if (bytes) PFS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, st->s));
 }
 // 16 bytes per thread: one 16-byte store where the address allows it
@@ -366,6 +445,7 @@ struct Marker {
   hipEvent_t e;
 };
 Marker* marker_record(Stream* st) {
+  stream_op(st);
   Marker* m = new Marker();
   PFS_HIP(hipEventCreateWithFlags(&m->e, hipEventDisableTiming));
   PFS_HIP(hipEventRecord(m->e, st->s));
@@ -386,6 +466,7 @@ void marker_free(Marker* m) {
   delete m;
 }
 bool stream_wait(Stream* st) {
+  stream_op(st);
   if (hipStreamSynchronize(st->s) == hipSuccess) return true;
   (void)hipGetLastError();
   return false;
@@ -397,6 +478,7 @@ void dev_mem_info(size_t* fr, size_t* tot) {
   }
 }
 Event* event_record(Stream* st) {
+  stream_op(st);
   Event* e = new Event();
   PFS_HIP(hipEventCreate(&e->e));
   PFS_HIP(hipEventRecord(e->e, st->s));
@@ -694,6 +776,9 @@ __device__ inline u64 block_excl_scan64_w(u64 v, u64* lw, u64* total) {
   *total = tot;
   return pre + x - v;
 }
+// A thread's consecutive items sit IPT words apart from its neighbour's: one
+// word of padding per 32 keeps the 64 lanes off a few banks.
+__device__ __host__ constexpr u32 lpad(u32 j) { return j + (j >> 5); }
 // where this thread's items go in a stable split of the workgroup's items by
 // the two bits d[i]
 template <int T, int IPT>
@@ -732,7 +817,7 @@ __global__ void __launch_bounds__(RS_T) rs_count_k(const u32* keys, size_t n, in
 __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* vin, u32* kout, u32* vout,
                                                     size_t n, int shift, int width, const u32* offs, u32 nb,
                                                     u32* starts, u32 nstarts, int sshift) {
-  __shared__ u32 sk[RS_TILE], sv[RS_TILE];
+  __shared__ u32 sk[lpad(RS_TILE)], sv[lpad(RS_TILE)];
   __shared__ u32 start[RBUCK];
   __shared__ u32 lw[RS_T / 64];
   __shared__ u64 lw64[RS_T / 64];
@@ -744,8 +829,8 @@ __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* 
 #pragma unroll
   for (int i = 0; i < RS_IPT; i++) {
     const u32 j = i * RS_T + threadIdx.x;
-    sk[j] = j < cnt ? kin[base + j] : (mask << shift);
-    sv[j] = j < cnt ? (vin ? vin[base + j] : (u32)(base + j)) : 0u;
+    sk[lpad(j)] = j < cnt ? kin[base + j] : (mask << shift);
+    sv[lpad(j)] = j < cnt ? (vin ? vin[base + j] : (u32)(base + j)) : 0u;
   }
   if (blockIdx.x == 0 && threadIdx.x < nstarts) {
     const u32 q = threadIdx.x << sshift;
@@ -758,15 +843,15 @@ __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* 
     u32 k[RS_IPT], v[RS_IPT], d[RS_IPT], dst[RS_IPT];
 #pragma unroll
     for (int i = 0; i < RS_IPT; i++) {
-      k[i] = sk[j0 + i];
-      v[i] = sv[j0 + i];
+      k[i] = sk[lpad(j0 + i)];
+      v[i] = sv[lpad(j0 + i)];
       d[i] = (k[i] >> (shift + bit)) & (bit + 1 < width ? 3u : 1u);
     }
     split4<RS_T, RS_IPT>(d, dst, lw64);  // its barriers follow every read above
 #pragma unroll
     for (int i = 0; i < RS_IPT; i++) {
-      sk[dst[i]] = k[i];
-      sv[dst[i]] = v[i];
+      sk[lpad(dst[i])] = k[i];
+      sv[lpad(dst[i])] = v[i];
     }
     __syncthreads();
   }
@@ -774,7 +859,7 @@ __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* 
 #pragma unroll
   for (int i = 0; i < RS_IPT; i++) {
     const u32 j = i * RS_T + threadIdx.x;
-    if (j < cnt) atomicAdd(&start[(sk[j] >> shift) & mask], 1u);
+    if (j < cnt) atomicAdd(&start[(sk[lpad(j)] >> shift) & mask], 1u);
   }
   __syncthreads();
   u32 tot;
@@ -786,10 +871,10 @@ __global__ void __launch_bounds__(RS_T) rs_scatter_k(const u32* kin, const u32* 
   for (int i = 0; i < RS_IPT; i++) {
     const u32 j = i * RS_T + threadIdx.x;
     if (j < cnt) {
-      const u32 key = sk[j], d = (key >> shift) & mask;
+      const u32 key = sk[lpad(j)], d = (key >> shift) & mask;
       const u32 dst = offs[(size_t)d * nb + blockIdx.x] + (j - start[d]);
       if (kout) kout[dst] = key;
-      vout[dst] = sv[j];
+      vout[dst] = sv[lpad(j)];
     }
   }
 }
@@ -799,16 +884,18 @@ size_t radix_tmp_bytes(size_t n) {
 }
 // Sorts of up to SO_MAX items in one launch by one workgroup: T threads
 // hold IPT consecutive items each in registers, and stable splits move them
-// through LDS.  The three launches and two copies of a pass over digits cost 40-60 us whatever
-// the size; this sorts 8,192 items by 8 bits in about 12 us.
+// through LDS.  The three launches and two copies of a pass over digits cost
+// 40-60 us whatever the size; this sorts 8,192 items by 8 bits in about 12 us.
+// (32 items per thread in one workgroup took 85 us for 20,000 candidates and
+// 11-bit keys, two digit passes 54.)
 constexpr int SO_T = 1024, SO_IPT = 8;
 constexpr u32 SO_MAX = SO_T * SO_IPT;
 // values sorted in place by the low 'bits' bits of their keys (the keys stay)
 template <int T>
 __global__ void __launch_bounds__(T) sort_one_k(const u32* keys, u32* vals, u32 n, int bits) {
   constexpr int IPT = SO_IPT;
-  __shared__ u32 sk[T * IPT];
-  __shared__ uint16_t si[T * IPT];
+  __shared__ u32 sk[lpad(T * IPT)];
+  __shared__ uint16_t si[lpad(T * IPT)];
   __shared__ u64 lw[T / 64];
   const u32 j0 = threadIdx.x * IPT;
   u32 k[IPT], id[IPT], d[IPT], dst[IPT], v[IPT];
@@ -824,14 +911,14 @@ __global__ void __launch_bounds__(T) sort_one_k(const u32* keys, u32* vals, u32 
     split4<T, IPT>(d, dst, lw);
 #pragma unroll
     for (int i = 0; i < IPT; i++) {
-      sk[dst[i]] = k[i];
-      si[dst[i]] = (uint16_t)id[i];
+      sk[lpad(dst[i])] = k[i];
+      si[lpad(dst[i])] = (uint16_t)id[i];
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < IPT; i++) {
-      k[i] = sk[j0 + i];
-      id[i] = si[j0 + i];
+      k[i] = sk[lpad(j0 + i)];
+      id[i] = si[lpad(j0 + i)];
     }
     __syncthreads();
   }
@@ -881,14 +968,16 @@ void radix_sort_pairs(u32* keys, u32* vals, size_t n, int bits, void* tmp, Strea
 // the way (counters of the launches that follow).  One launch by one
 // workgroup for up to SO_MAX items, else three (keys and their counts per
 // tile, one scan, the scatter); what this replaces was a launch for the keys,
-// three for the digit pass, two copies, one for the starts and a fill.
+// three for the digit pass, two copies, one for the starts and a fill.  (One
+// workgroup with 16 or 32 items per thread takes 37 and 116 us for 12,000 and
+// 30,000 variables, whose list sizes it reads, the three launches 28 and 30.)
 constexpr int KEY_IDX_BITS = 13;
 static_assert(SO_MAX <= (1u << KEY_IDX_BITS), "an item's index and key share a word");
 template <int T, class F>
 __global__ void __launch_bounds__(T) place_one_k(F f, u32 n, int bits, u32* out, u32* starts, u32 nstarts, int sshift,
                                                  u32* zero, u32 nz) {
   constexpr int IPT = SO_IPT;
-  __shared__ u32 sk[T * IPT];
+  __shared__ u32 sk[lpad(T * IPT)];
   __shared__ u64 lw[T / 64];
   if (threadIdx.x < nz) zero[threadIdx.x] = 0;
   const u32 j0 = threadIdx.x * IPT;
@@ -899,35 +988,35 @@ __global__ void __launch_bounds__(T) place_one_k(F f, u32 n, int bits, u32* out,
 #pragma unroll
   for (int i = 0; i < IPT; i++) {
     const u32 j = i * T + threadIdx.x;
-    sk[j] = ((j < n ? f.key(j) : top) << KEY_IDX_BITS) | j;
+    sk[lpad(j)] = ((j < n ? f.key(j) : top) << KEY_IDX_BITS) | j;
   }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < IPT; i++) x[i] = sk[j0 + i];
+  for (int i = 0; i < IPT; i++) x[i] = sk[lpad(j0 + i)];
   __syncthreads();
   for (int bit = 0; bit < bits; bit += 2) {
 #pragma unroll
     for (int i = 0; i < IPT; i++) d[i] = (x[i] >> (KEY_IDX_BITS + bit)) & (bit + 1 < bits ? 3u : 1u);
     split4<T, IPT>(d, dst, lw);
 #pragma unroll
-    for (int i = 0; i < IPT; i++) sk[dst[i]] = x[i];
+    for (int i = 0; i < IPT; i++) sk[lpad(dst[i])] = x[i];
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < IPT; i++) x[i] = sk[j0 + i];
+    for (int i = 0; i < IPT; i++) x[i] = sk[lpad(j0 + i)];
     __syncthreads();
   }
 #pragma unroll
-  for (int i = 0; i < IPT; i++) sk[j0 + i] = x[i];
+  for (int i = 0; i < IPT; i++) sk[lpad(j0 + i)] = x[i];
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < IPT; i++) {
     const u32 j = i * T + threadIdx.x;
     if (j >= n) continue;
-    out[j] = f.val(sk[j] & imask);
+    out[j] = f.val(sk[lpad(j)] & imask);
     if (nstarts) {
       const int sh = KEY_IDX_BITS + sshift;
-      const u32 key = sk[j] >> sh;
-      for (u32 q = j ? (sk[j - 1] >> sh) + 1 : 0; q <= key && q < nstarts; q++) starts[q] = j;
+      const u32 key = sk[lpad(j)] >> sh;
+      for (u32 q = j ? (sk[lpad(j - 1)] >> sh) + 1 : 0; q <= key && q < nstarts; q++) starts[q] = j;
       if (j == n - 1)
         for (u32 q = key + 1; q < nstarts; q++) starts[q] = n;
     }
@@ -1548,7 +1637,7 @@ void k_set_vstate(const DB& db, const u32* lits, u32 n, u8 state, Stream* st) {
 }
 
 // ---------------------------------------------------------------- LCVE
-__device__ unsigned long long lcve_classify_var(const DB& db, const LcveArgs& a, u32 v);
+__device__ unsigned long long lcve_classify_var(const DB& db, const LcveArgs& a, u32 v, u32& top);
 __device__ inline unsigned long long wave_min64(unsigned long long x) {
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) {
@@ -1563,20 +1652,30 @@ __device__ inline unsigned long long wave_min64(unsigned long long x) {
 // variables serialised 1 ms on the one word)
 __global__ void lcve_classify_k(DB db, LcveArgs a) {
   __shared__ unsigned long long wmin[ST / 64];
+  __shared__ u32 wmax[ST / 64];
   unsigned long long hk = ~0ull;
+  u32 top = 0;
   for (u32 v = blockIdx.x * blockDim.x + threadIdx.x + 1; v <= db.nvars; v += gridDim.x * blockDim.x) {
-    const unsigned long long k = lcve_classify_var(db, a, v);
+    const unsigned long long k = lcve_classify_var(db, a, v, top);
     hk = k < hk ? k : hk;
   }
   hk = wave_min64(hk);
-  if ((threadIdx.x & 63) == 0) wmin[threadIdx.x >> 6] = hk;
+  top = wave_max(top);
+  if ((threadIdx.x & 63) == 0) {
+    wmin[threadIdx.x >> 6] = hk;
+    wmax[threadIdx.x >> 6] = top;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (u32 w = 1; w < ST / 64; w++) hk = wmin[w] < hk ? wmin[w] : hk;
+    for (u32 w = 1; w < ST / 64; w++) {
+      hk = wmin[w] < hk ? wmin[w] : hk;
+      top = max(top, wmax[w]);
+    }
     if (hk != ~0ull) at_min64(a.hard, hk);
+    if (top) atomicMax(&a.top[blockIdx.x % LCVE_TOPS], top);
   }
 }
-__device__ unsigned long long lcve_classify_var(const DB& db, const LcveArgs& a, u32 v) {
+__device__ unsigned long long lcve_classify_var(const DB& db, const LcveArgs& a, u32 v, u32& top) {
   const u32 ps = a.hist[V2L(v)], ns = a.hist[V2L(v) | 1];
   const u32 score = ps * ns;  // 32-bit product as in the reference
   a.score[v] = score;
@@ -1590,9 +1689,15 @@ __device__ unsigned long long lcve_classify_var(const DB& db, const LcveArgs& a,
   u8 f = cand ? (brk ? 3 : 1) : 0;
   if (f == 1 && a.clause_max != 0xFFFFFFFFu && lcve_oversize(db, v, a.clause_max)) f = 4;
   a.cflag[v] = f;
+  if (f) top = max(top, score);
   return cand && hard ? ((unsigned long long)score << 32) | v : ~0ull;
 }
+__global__ void lcve_clear_k(LcveArgs a) {
+  a.top[threadIdx.x] = 0;
+  if (threadIdx.x == 0) *a.hard = ~0ull;
+}
 void k_lcve_classify(const DB& db, const LcveArgs& a, Stream* st) {
+  KLAUNCH(lcve_clear_k, 1, LCVE_TOPS, st, a);
   KLAUNCH(lcve_classify_k, std::min(grid_for(db.nvars, ST), 2048u), ST, st, db, a);
 }
 __global__ void lcve_flag_k(DB db, LcveArgs a, u32* flag, u32* pos) {
@@ -1620,13 +1725,14 @@ void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u3
 }
 // The state of an election before its first step: each candidate's packed
 // position and state (undecided, or decided and not elected for the ones
-// passed over) and the counters (sc: [1] the break position, [4..6] and
+// passed over) and the counters (sc: [1] the break position, [3..6] and
 // [12..14] the passes' counts, [24..25] the list sort's), in one launch.  The positions of variables
 // that are no candidates are NOPOS from lcve_flag_k.
 __global__ void mis_init_k(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     sc[1] = n;
+    sc[3] = 0;
     for (u32 q = 0; q < 3; q++) sc[4 + q] = 0, sc[12 + q] = 0;
     sc[24] = sc[25] = 0;
   }
@@ -1820,22 +1926,34 @@ __global__ void mis_flag_k(const u32* state, u32 n, const u32* brk, u32* flag) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) flag[i] = (state[i] == 1 && i < *brk) ? 1u : 0u;
 }
-__global__ void mis_pack_k(const u32* cand, const u32* state, u32 n, const u32* brk, const u32* pos,
-                           u32* out) {
-  const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && state[i] == 1 && i < *brk) out[pos[i]] = cand[i];
+// entries (nullable): also sums the elected lists' entries (SUB's room), which
+// the read of the number of elected variables brings along
+__global__ void __launch_bounds__(256) mis_pack_k(DB db, const u32* cand, const u32* state, u32 n, const u32* brk,
+                                                  const u32* pos, u32* out, u32* entries) {
+  u32 w = 0;
+  const u32 b = *brk;
+  for (u32 i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    if (state[i] == 1 && i < b) {
+      const u32 v = cand[i];
+      out[pos[i]] = v;
+      if (entries) w += db.ot_size[V2L(v)] + db.ot_size[V2L(v) | 1];
+    }
+  if (!entries) return;
+  __shared__ u32 lw[256 / 64];
+  u32 tot;
+  block_excl_scan_w<256 / 64>(w, lw, &tot);
+  if (threadIdx.x == 0 && tot) atomicAdd(entries, tot);
 }
-void k_mis_collect(const u32* cand, u32 n, const u32* state, u32 brk_unused, u32* flag_tmp, u32* out,
-                   u32* nout, void* tmp, Stream* st) {
-  (void)brk_unused;
-  // brk lives in nout[1] on the device; nout[0] receives the count
+void k_mis_collect(const DB& db, const u32* cand, u32 n, const u32* state, u32* flag_tmp, u32* out, u32* sc,
+                   bool entries, void* tmp, Stream* st) {
   if (!n) {
-    fill_u32(nout, 0, 1, st);
+    fill_u32(sc, 0, 1, st);
     return;
   }
-  KLAUNCH(mis_flag_k, grid_for(n, 256), 256, st, state, n, nout + 1, flag_tmp);
-  scan_u32(flag_tmp, flag_tmp, n, nout, tmp, st);
-  KLAUNCH(mis_pack_k, grid_for(n, 256), 256, st, cand, state, n, nout + 1, flag_tmp, out);
+  KLAUNCH(mis_flag_k, grid_for(n, 256), 256, st, state, n, sc + 1, flag_tmp);
+  scan_u32(flag_tmp, flag_tmp, n, sc, tmp, st);
+  KLAUNCH(mis_pack_k, entries ? std::min(grid_for(n, 256), RED_BLOCKS) : grid_for(n, 256), 256, st, db, cand, state, n,
+          sc + 1, flag_tmp, out, entries ? sc + 3 : nullptr);
 }
 
 // ---------------------------------------------------------------- per elected variable

@@ -116,10 +116,14 @@ void k_clear_lists(const DB& db, const u32* lits, u32 n, Stream*);
 void k_set_vstate(const DB& db, const u32* lits, u32 n, u8 state, Stream*);
 
 // ---- LCVE
+constexpr u32 LCVE_TOPS = 64;
 struct LcveArgs {
   const u32* hist;  // per literal
   u32* score;       // per variable
   u64* hard;        // min (score, var) over hard breakers
+  // largest score of a candidate, in LCVE_TOPS parts (2,048 workgroups on one
+  // word wait 55 us for each other)
+  u32* top;
   u8* cflag;        // per variable: 1 candidate, 3 soft breaker candidate, 4 passed over, 0 none
   u32 pt, nt;
   u32 max_occurs;   // electionsmax: break past this many occurrences of a literal
@@ -131,7 +135,7 @@ void k_lcve_classify(const DB& db, const LcveArgs& a, Stream*);
 void k_lcve_select(const DB& db, const LcveArgs& a, u32* flag_tmp, u32* cand, u32* key, u32* pos, u32* ncand,
                    void* tmp, Stream*);
 // the state before the first step: positions, states, counters (sc[1] = n,
-// sc[4..6] = sc[12..14] = sc[24..25] = 0).  reject: candidates passed over for an oversize
+// sc[3..6] = sc[12..14] = sc[24..25] = 0).  reject: candidates passed over for an oversize
 // clause (cflag 4) start decided and not elected: they neither block nor
 // freeze a neighbour
 void k_mis_init(const u32* cand, u32 n, const u8* cflag, bool reject, u32* pos, u32* state, u32* sc, Stream*);
@@ -150,8 +154,10 @@ void k_mis_step_dev(const DB& db, const u32* cand, const u32* idx, const u32* n_
                     u32* state, u32* blk, u32* resume, u32* next, u32* nnext, u32* iters, u32* zero, u32 lds,
                     u32 lanes, Stream*);
 void k_mis_break(const u32* cand, u32 n, const u8* cflag, const u32* state, u32* brk, Stream*);
-void k_mis_collect(const u32* cand, u32 n, const u32* state, u32 brk, u32* flag_tmp, u32* out,
-                   u32* nout, void* tmp, Stream*);
+// the elected ones before the break (sc[1]) to out, their number to sc[0],
+// with 'entries' the entries of their lists added to sc[3]
+void k_mis_collect(const DB& db, const u32* cand, u32 n, const u32* state, u32* flag_tmp, u32* out, u32* sc,
+                   bool entries, void* tmp, Stream*);
 
 // ---- per elected variable stages
 void k_list_sizes(const DB& db, const u32* pv, u32 n, u32 extra, u32* out, Stream*);  // |poss|+|negs|+extra
