@@ -175,66 +175,68 @@ void Simplifier::upload(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
                         const uint8_t* assumed, const uint32_t* vorg, const uint32_t* trail,
                         uint32_t ntrail) {
   V_ = maxvar;
-  // extraction order: originals, then learnts (simplify.cpp:148-149)
-  std::vector<uint64_t> order;
-  order.reserve(ncls);
-  for (uint64_t i = 0; i < ncls; i++)
-    if (!(flags && (flags[i] & 1))) order.push_back(i);
-  for (uint64_t i = 0; i < ncls; i++)
-    if (flags && (flags[i] & 1)) order.push_back(i);
-  has_learnts_ = order.size() && flags && (flags[order.back()] & 1);
   // pool words: a header per clause, then its literals
-  const uint64_t L = offsets[ncls] - offsets[0] + CL_HDR * ncls;
+  const uint64_t nl = offsets[ncls] - offsets[0], L = nl + CL_HDR * ncls;
   if (ncls >= INF / 2 || L >= INF / 4) throw AllocFail{"formula too large for 32-bit clause ids"};
-  std::vector<u32> h_off(ncls), h_lits(L);
-  uint64_t w = 0;
-  for (uint64_t k = 0; k < ncls; k++) {
-    const uint64_t i = order[k];
-    const uint64_t n = offsets[i + 1] - offsets[i];
-    if (n > CL_MAX_SIZE) throw std::invalid_argument("clause longer than 2^24-1 literals");
-    h_off[k] = (u32)w;
-    const u8 f = flags ? flags[i] : 0;
-    const bool learnt = f & 1;
-    h_lits[w] = make_hdr((u32)n, learnt ? (u8)(ST_LEARNT | (f & USAGE_MASK)) : (u8)ST_ORIGINAL);
-    h_lits[w + 1] = 0;  // signature: set by the literal sort on the device
-    h_lits[w + 2] = learnt && lbd ? (lbd[i] & 0x03FFFFFFu) : 0u;
-    for (uint64_t j = 0; j < n; j++) {
-      const u32 l = lits[offsets[i] + j];
-      if (ABS(l) == 0 || ABS(l) > maxvar) throw std::invalid_argument("literal out of range");
-      h_lits[w + CL_HDR + j] = l;
-    }
-    w += CL_HDR + n;
-  }
+  uint64_t longest = 0;
+  for (uint64_t i = 0; i < ncls; i++) longest = std::max(longest, offsets[i + 1] - offsets[i]);
+  if (longest > CL_MAX_SIZE) throw std::invalid_argument("clause longer than 2^24-1 literals");
   set_capacities(ncls, L);
   alloc_state();
   cur_ = 0;
   ncls_ = ncls;
   lits_end_ = L;
-  h2d(c_off_[0].p, h_off.data(), ncls * 4, st_);
-  h2d(lits_[0].p, h_lits.data(), L * 4, st_);
+  // The arrays go over as the caller has them and the device builds the pool
+  // (a host loop over the clauses took 2 of the 2.8 ms of an upload of 0.9M
+  // literals, and 0.7 s for 120M).  They wait in buffers that nothing uses
+  // before the first round: the literals and the offsets in the other
+  // block's pool (W + 4096 words at least, W = literals + 3 per clause), the
+  // LBDs in its handles, the flags in the marks.
+  u32* raw_lits = P<u32>(lits_[1]);
+  u64* raw_off = (u64*)(raw_lits + ((nl + 1) & ~(uint64_t)1));
+  u32* sc = P<u32>(scal_);
+  fill_u32(sc, 0, 3, st_);  // error, learnt clauses, their words
+  h2d(raw_off, offsets, (ncls + 1) * 8, st_);
+  h2d(raw_lits, lits ? lits + offsets[0] : nullptr, nl * 4, st_);
+  if (flags) h2d(mark_.p, flags, ncls, st_);
+  if (flags && lbd) h2d(c_off_[1].p, lbd, ncls * 4, st_);
+  RawClauses raw{raw_off, raw_lits, flags ? P<u8>(mark_) : nullptr, flags && lbd ? P<u32>(c_off_[1]) : nullptr,
+                 nullptr, nullptr, (u32)ncls, (u32)L, maxvar, sc};
+  if (flags) {  // extraction order: originals, then learnts (simplify.cpp:148-149)
+    mem_.ensure(tmp2_, std::max<size_t>(ncls, 1) * 4, 0, st_);
+    mem_.ensure(tmp3_, std::max<size_t>(ncls, 1) * 4, 0, st_);
+    mem_.ensure(tmp_, std::max(tmp_.cap, 2 * scan_tmp_bytes(ncls)), 0, st_);
+    raw.lrank = P<u32>(tmp2_);
+    raw.lwords = P<u32>(tmp3_);
+  }
+  k_build_clauses(make_db(0), raw, tmp_.p, st_);
+  u32 built[2];
+  d2h(built, sc, 8, st_);
   // per-variable state
   h_assign_.assign((size_t)V_ + 1, 0);
   h_touched_.clear();
   in_units_.assign(trail, trail + ntrail);
   for (u32 i = 0; i < ntrail; i++) h_assign_[ABS(trail[i])] = trail[i] + 1;
-  std::vector<u8> vs((size_t)V_ + 1, 0), as((size_t)V_ + 1, 0);
-  std::vector<u32> vo((size_t)V_ + 1);
+  const size_t V1 = (size_t)V_ + 1;
   u32 melted = 0;
+  fill_u32(P<u32>(assign_), 0, V1, st_);
+  fill_u8(P<u8>(vstate_), 0, V1, st_);
+  fill_u8(P<u8>(assumed_), 0, V1, st_);
+  if (vstate) {
+    for (u32 v = 1; v <= V_; v++) melted += (vstate[v] & (VS_MELTED | VS_SUBSTITUTED)) ? 1 : 0;
+    h2d(P<u8>(vstate_) + 1, vstate + 1, V_, st_);
+  }
+  if (assumed) h2d(P<u8>(assumed_) + 1, assumed + 1, V_, st_);
   orgmax_ = V_;
-  for (u32 v = 0; v <= V_; v++) {
-    vs[v] = v && vstate ? vstate[v] : 0;
-    as[v] = v && assumed ? assumed[v] : 0;
-    vo[v] = vorg ? vorg[v] : v;
-    orgmax_ = std::max(orgmax_, vo[v]);
-    melted += (vs[v] & (VS_MELTED | VS_SUBSTITUTED)) ? 1 : 0;
+  if (vorg) {
+    for (size_t v = 0; v < V1; v++) orgmax_ = std::max(orgmax_, vorg[v]);
+    h2d(vorg_.p, vorg, V1 * 4, st_);
+  } else {
+    iota_u32(P<u32>(vorg_), V1, st_);
   }
   map_called_ = map_applied_ = remapped_ = false;
-  for (u32 i = 0; i < ntrail; i++) vs[ABS(trail[i])] = VS_FROZEN;
-  h2d(assign_.p, h_assign_.data(), ((size_t)V_ + 1) * 4, st_);
-  h2d(vstate_.p, vs.data(), (size_t)V_ + 1, st_);
-  h2d(assumed_.p, as.data(), (size_t)V_ + 1, st_);
-  h2d(vorg_.p, vo.data(), ((size_t)V_ + 1) * 4, st_);
   h2d(trail_.p, trail, (size_t)ntrail * 4, st_);
+  k_assign_units(make_db(0), P<u32>(trail_), ntrail, st_);  // assigned and frozen
   trail_n_ = propagated_ = ntrail;
   unassigned_ = V_ - ntrail - melted;
   stack_n_ = 0;
@@ -244,8 +246,9 @@ void Simplifier::upload(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
   refuted_ = false;
   resident_ = false;
   fill_u8(P<u8>(mark_), 0, lcap_, st_);
-  // extract: sort literals, signatures
-  k_prep(make_db(0), 0, st_);
+  stream_sync(st_);
+  if (built[0]) throw std::invalid_argument("literal out of range");
+  has_learnts_ = built[1] != 0;
   save_input();
   stream_sync(st_);
 }

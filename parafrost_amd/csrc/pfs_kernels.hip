@@ -2443,12 +2443,9 @@ __global__ void reduce_lists_k(DB db) {
 void k_reduce_lists(const DB& db, Stream* st) {
   KLAUNCH(reduce_lists_k, grid_for(2 * (size_t)db.nvars, 256), 256, st, db);
 }
-__global__ void prep_k(DB db, u32 first) {
-  const u32 i = first + blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= db.ncls) return;
-  u32* h = chead(db, db.c_off[i]);
+// literals sorted, signature
+__device__ inline void prep_clause(u32* h, u32 n) {
   u32* l = h + CL_HDR;
-  const u32 n = hdr_size(h[0]);
   for (u32 q = 1; q < n; q++) {
     const u32 t = l[q];
     u32 j = q;
@@ -2456,6 +2453,62 @@ __global__ void prep_k(DB db, u32 first) {
     l[j] = t;
   }
   h[1] = calc_sig(l, n);
+}
+__global__ void prep_k(DB db, u32 first) {
+  const u32 i = first + blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= db.ncls) return;
+  u32* h = chead(db, db.c_off[i]);
+  prep_clause(h, hdr_size(h[0]));
+}
+__global__ void raw_learnt_k(RawClauses r) {
+  const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= r.n) return;
+  const bool learnt = r.flags[i] & 1;
+  r.lrank[i] = learnt ? 1u : 0u;
+  r.lwords[i] = learnt ? CL_HDR + (u32)(r.off[i + 1] - r.off[i]) : 0u;
+}
+// a thread per clause: its place is what precedes it in the given order, less
+// the learnt clauses among that, or for a learnt clause all originals and the
+// learnt ones before it
+__global__ void raw_build_k(DB db, RawClauses r) {
+  const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= r.n) return;
+  const u64 o0 = r.off[i] - r.off[0];
+  const u32 n = (u32)(r.off[i + 1] - r.off[i]);
+  const u8 f = r.flags ? r.flags[i] : 0;
+  const bool learnt = f & 1;
+  u32 at = i, handle = CL_HDR * i + (u32)o0;
+  if (r.flags) {
+    const u32 lr = r.lrank[i], lw = r.lwords[i];
+    at = learnt ? r.n - r.sc[1] + lr : at - lr;
+    handle = learnt ? r.words - r.sc[2] + lw : handle - lw;
+  }
+  u32* h = db.lits + handle;
+  const u32* src = r.lits + o0;
+  db.c_off[at] = handle;
+  h[0] = make_hdr(n, learnt ? (u8)(ST_LEARNT | (f & USAGE_MASK)) : (u8)ST_ORIGINAL);
+  h[2] = learnt && r.lbd ? (r.lbd[i] & 0x03FFFFFFu) : 0u;
+  bool bad = false;
+  for (u32 q = 0; q < n; q++) {
+    const u32 l = src[q];
+    bad |= ABS(l) == 0 || ABS(l) > r.maxvar;
+    u32 j = q;  // insertion into the sorted literals before it
+    while (j > 0 && h[CL_HDR + j - 1] > l) {
+      h[CL_HDR + j] = h[CL_HDR + j - 1];
+      j--;
+    }
+    h[CL_HDR + j] = l;
+  }
+  h[1] = calc_sig(h + CL_HDR, n);
+  if (bad) *r.sc = 1;
+}
+void k_build_clauses(const DB& db, const RawClauses& raw, void* tmp, Stream* st) {
+  if (!raw.n) return;
+  if (raw.flags) {
+    KLAUNCH(raw_learnt_k, grid_for(raw.n, 256), 256, st, raw);
+    scan_set(ScanSet{{raw.lrank, raw.lwords}, {raw.lrank, raw.lwords}, {raw.sc + 1, raw.sc + 2}}, 2, raw.n, tmp, st);
+  }
+  KLAUNCH(raw_build_k, grid_for(raw.n, 256), 256, st, db, raw);
 }
 void k_prep(const DB& db, u32 first, Stream* st) {
   if (first >= db.ncls) return;

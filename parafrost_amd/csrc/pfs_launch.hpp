@@ -210,7 +210,23 @@ void k_ere_all_matches(const DB& db, const ErePairs& a, u32 n, const u32* off, u
 void k_assign_units(const DB& db, const u32* lits, u32 n, Stream*);  // assign + FROZEN
 void k_max_list(const DB& db, const u32* lits, u32 n, u32* out, Stream*);
 void k_reduce_lists(const DB& db, Stream*);  // drop deleted entries from every list
-void k_prep(const DB& db, u32 first, Stream*);  // clauses [first, ncls): sort literals, signature
+void k_prep(const DB& db, u32 first, Stream*);
+// the clauses of a caller's database (off[n + 1], lits from off[0] on) built
+// into the pool, originals first, then learnts, each in the given order:
+// headers, literals sorted, signatures, handles.  flags (null: all original)
+// with lrank and lwords, n words each; lbd nullable; sc[0] is set for a
+// literal out of range, sc[1], sc[2] receive the learnt clauses and their
+// pool words (all three zero before); tmp: 2 * scan_tmp_bytes(n)
+struct RawClauses {
+  const u64* off;
+  const u32* lits;
+  const u8* flags;
+  const u32* lbd;
+  u32 *lrank, *lwords;
+  u32 n, words, maxvar;
+  u32* sc;
+};
+void k_build_clauses(const DB& db, const RawClauses& raw, void* tmp, Stream*);  // clauses [first, ncls): sort literals, signature
 void k_zero_sizes(const DB& db, const u32* lits, u32 n, Stream*);
 void k_clear_added(const DB& db, Stream*);  // resolvent marks of an earlier simplify call
 
