@@ -877,7 +877,13 @@ void Simplifier::ot_counts(bool table) {
   u32* hist = P<u32>(hist_);
   OtpPlan p;
   auto build = [&](int tile) {
-    if (!opt.otp_ranges || !otp_plan(n2, db.ncls, &p, tile, opt.otp_xcd) || !otp_room(p)) return false;
+    if (!opt.otp_ranges || !otp_plan(n2, db.ncls, &p, tile, opt.otp_xcd)) return false;
+    if (ot_one_fits(n2, db.ncls)) {
+      k_ot_one(db, (u32)n2, table, hist, st_);
+      used_tile_ = (int32_t)ilog2(p.ct);
+      return true;
+    }
+    if (!otp_room(p)) return false;
     mem_.ensure(tmp_, std::max(tmp_.cap, scan_tmp_bytes(p.ncounts)), 0, st_);
     u32* counts = P<u32>(otp_);
     u32* pairs = counts + ((p.ncounts + 1 + 63) & ~(size_t)63);  // 256-byte aligned
@@ -1016,21 +1022,29 @@ bool Simplifier::lcve() {
   a.nt = (u32)opt.mu_neg << mu_inc_;
   a.max_occurs = opt.lcve_max_occurs == INT32_MAX ? INF : (u32)opt.lcve_max_occurs;
   a.clause_max = opt.lcve_clause_max == INT32_MAX ? INF : (u32)opt.lcve_clause_max;
-  k_lcve_classify(db, a, st_);
-  k_lcve_select(db, a, P<u32>(flag_), P<u32>(cand_), P<u32>(key_), P<u32>(pos_), sc, tmp_.p, st_);
-  u32 h[3], tops[LCVE_TOPS];  // candidates, hard breaker's variable and score; largest scores
-  d2h(h, sc, 4, st_);
-  d2h(h + 1, hard, 8, st_);
-  d2h(tops, a.top, sizeof(tops), st_);
-  stream_sync(st_);
-  const u32 ncand = h[0];
-  // the candidates stay below the hard breaker and at most at the largest score
-  const u32 most = std::min(h[2], *std::max_element(tops, tops + LCVE_TOPS));
-  int bits = 0;
-  while (bits < 32 && (most >> bits)) bits++;
-  radix_sort_pairs(P<u32>(key_), P<u32>(cand_), ncand, bits, tmp_.p, st_);
-  // positions share a word with the candidate's state (position << 2)
-  if (ncand >= (1u << 30)) throw DeviceFail{"LCVE: too many candidates for the packed positions"};
+  // a small formula keeps its candidates' number on the device until the
+  // election's read (ncand is a bound until then)
+  const bool small = V_ <= LCVE_SMALL && !tune_mis_;
+  u32 ncand = V_;
+  if (small) {
+    k_lcve_small(db, a, a.clause_max != INF, P<u32>(pos_), P<u32>(cand_), P<u32>(state_), sc, st_);
+  } else {
+    k_lcve_classify(db, a, st_);
+    k_lcve_select(db, a, P<u32>(flag_), P<u32>(cand_), P<u32>(key_), P<u32>(pos_), sc, tmp_.p, st_);
+    u32 h[3], tops[LCVE_TOPS];  // candidates, hard breaker's variable and score; largest scores
+    d2h(h, sc, 4, st_);
+    d2h(h + 1, hard, 8, st_);
+    d2h(tops, a.top, sizeof(tops), st_);
+    stream_sync(st_);
+    ncand = h[0];
+    // the candidates stay below the hard breaker and at most at the largest score
+    const u32 most = std::min(h[2], *std::max_element(tops, tops + LCVE_TOPS));
+    int bits = 0;
+    while (bits < 32 && (most >> bits)) bits++;
+    radix_sort_pairs(P<u32>(key_), P<u32>(cand_), ncand, bits, tmp_.p, st_);
+    // positions share a word with the candidate's state (position << 2)
+    if (ncand >= (1u << 30)) throw DeviceFail{"LCVE: too many candidates for the packed positions"};
+  }
   u32* resume = P<u32>(vsz_);  // free until SUB: where each scan goes on
   // worklists of undecided candidates (the selection buffers are free now);
   // after the first pass over all candidates, passes are queued MIS_QUEUE at
@@ -1059,9 +1073,10 @@ bool Simplifier::lcve() {
   // candidate; ring[p % 3] tells whether there is more to do
   auto begin = [&](u32 lds, u32 lanes) {
     p = 0;
-    k_mis_init(P<u32>(cand_), ncand, P<u8>(cflag_), a.clause_max != INF, P<u32>(pos_), P<u32>(state_), sc, st_);
+    if (!small)
+      k_mis_init(P<u32>(cand_), ncand, P<u8>(cflag_), a.clause_max != INF, P<u32>(pos_), P<u32>(state_), sc, st_);
     if (!ncand) return;
-    k_mis_step(db, P<u32>(cand_), ncand, P<u32>(pos_), P<u32>(state_), P<u32>(key_), resume, wl[0], ring[0], lds,
+    k_mis_step(db, P<u32>(cand_), ncand, small ? sc + 2 : nullptr, P<u32>(pos_), P<u32>(state_), P<u32>(key_), resume, wl[0], ring[0], lds,
                lanes, st_);
     passes(ncand, lds, lanes);
   };
@@ -1127,18 +1142,23 @@ bool Simplifier::lcve() {
   const bool with_entries = ncand <= (1u << 18);
   u32 w15[15];  // sc[0]: elected, sc[3]: entries of their lists, sc[6]: worklist passes with work, sc[12..14]: the ring
   while (true) {
-    k_mis_break(P<u32>(cand_), ncand, P<u8>(cflag_), P<u32>(state_), sc + 1, st_);
+    if (small) k_collect_small(db, P<u32>(cand_), P<u8>(cflag_), P<u32>(state_), P<u32>(pv_), sc, st_);
+    else k_mis_break(P<u32>(cand_), ncand, P<u8>(cflag_), P<u32>(state_), sc + 1, st_);
     // the worklist still to be read must stay: the other one is free
-    k_mis_collect(db, P<u32>(cand_), ncand, P<u32>(state_), wl[(p + 1) & 1], P<u32>(pv_), sc, with_entries, tmp_.p,
-                  st_);
+    if (!small)
+      k_mis_collect(db, P<u32>(cand_), ncand, P<u32>(state_), wl[(p + 1) & 1], P<u32>(pv_), sc, with_entries,
+                    tmp_.p, st_);
     d2h(w15, sc, sizeof(w15), st_);
     stream_sync(st_);
     const u32 bound = ncand ? w15[12 + p % 3] : 0;
     if (!bound) break;
-    fill_u32(sc + 1, ncand, 1, st_);
-    fill_u32(sc + 3, 0, 1, st_);
+    if (!small) {
+      fill_u32(sc + 1, ncand, 1, st_);
+      fill_u32(sc + 3, 0, 1, st_);
+    }
     passes(bound, (u32)used_lds_, lanes);
   }
+  if (small) ncand = w15[2];
   const u32* w7 = w15;
   E_ = w7[0];
   elected_entries_ = with_entries ? w7[3] : NOPOS;

@@ -1280,6 +1280,45 @@ bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2, int xcd) {
   p->ncounts = (size_t)p->nr * p->nblk;
   return true;
 }
+// the same for a formula whose literals fit one workgroup's counters and
+// whose clauses are few (OT_ONE_LITS, OT_ONE_CLAUSES): counted, scanned and
+// placed in one launch without the pairs.  For a circuit of 5,000 variables
+// and 17,000 clauses the four launches take 52 us, most of it waiting for a
+// handful of workgroups, this one 36 us; it reads the literals twice with one
+// workgroup, so past these clauses the four are again the faster ones.
+template <bool TABLE>
+__global__ void __launch_bounds__(OTP_TB) otp_one_k(DB db, u32 n2, u32* hist) {
+  extern __shared__ u32 lc[];
+  __shared__ u32 lw[OTP_TB / 64];
+  for (u32 j = threadIdx.x; j < n2; j += OTP_TB) lc[j] = 0;
+  __syncthreads();
+  otp_tile(db, 0, db.ncls, [&](u32 l, u32) { atomicAdd(&lc[l], 1u); });
+  __syncthreads();
+  if (!TABLE) {
+    for (u32 j = threadIdx.x; j < n2; j += OTP_TB) hist[j] = lc[j];
+    return;
+  }
+  const u32 per = (n2 + OTP_TB - 1) / OTP_TB, j0 = threadIdx.x * per, j1 = min(n2, j0 + per);
+  u32 s = 0, tot;
+  for (u32 j = j0; j < j1; j++) s += lc[j];
+  u32 pre = block_excl_scan_w<OTP_TB / 64>(s, lw, &tot);
+  for (u32 j = j0; j < j1; j++) {
+    const u32 v = lc[j];
+    db.ot_off[j] = pre;
+    db.ot_size[j] = v;
+    hist[j] = v;
+    lc[j] = pre;  // the list's cursor
+    pre += v;
+  }
+  if (threadIdx.x == 0) db.ot_off[n2] = tot;
+  __syncthreads();
+  otp_tile(db, 0, db.ncls, [&](u32 l, u32 c) { db.ot_refs[atomicAdd(&lc[l], 1u)] = c; });
+}
+bool ot_one_fits(size_t n2, size_t ncls) { return n2 <= OT_ONE_LITS && ncls <= OT_ONE_CLAUSES; }
+void k_ot_one(const DB& db, u32 n2, bool table, u32* hist, Stream* st) {
+  if (table) KLAUNCH_LDS(otp_one_k<true>, 1, OTP_TB, (size_t)n2 * 4, st, db, n2, hist);
+  else KLAUNCH_LDS(otp_one_k<false>, 1, OTP_TB, (size_t)n2 * 4, st, db, n2, hist);
+}
 // counts: p.ncounts + 1 words; pairs: 8-byte aligned, two words per live
 // occurrence (table) or one (hist only); tmp: scan_tmp_bytes(p.ncounts)
 void k_ot_ranges(const DB& db, const OtpPlan& p, u32 n2, u32* counts, void* pairs, bool table, u32* hist,
@@ -1842,8 +1881,9 @@ __device__ inline void mis_run(const DB& db, u32 i, bool valid, bool fresh, cons
 // bound occupancy (option "mislds"; 20 KiB leaves 2 wavefronts per SIMD:
 // Tseitin round 0 / 20 / 40 KiB -> mis_step_k 3.34 / 2.76 / 3.18 ms)
 template <u32 G>
-__global__ void mis_step_k(DB db, const u32* cand, u32 n, u32* pos, u32* state, u32* blk, u32* resume, u32* next,
-                           u32* nnext, u32 tries) {
+__global__ void mis_step_k(DB db, const u32* cand, u32 n, const u32* n_dev, u32* pos, u32* state, u32* blk, u32* resume,
+                           u32* next, u32* nnext, u32 tries) {
+  if (n_dev) n = *n_dev;
   const u64 t = (u64)blockIdx.x * blockDim.x + threadIdx.x;
   const u32 q = (u32)(t / G);
   mis_run<G>(db, q, q < n, true, cand, pos, state, blk, resume, next, nnext, tries);
@@ -1894,12 +1934,12 @@ u32 mis_lanes_for(u32 n) {
   while (g > 1 && (u64)n * g > 2 * in_flight) g >>= 1;
   return g;
 }
-void k_mis_step(const DB& db, const u32* cand, u32 n, u32* pos, u32* state, u32* blk, u32* resume, u32* next,
-                u32* nnext, u32 lds, u32 lanes, Stream* st) {
+void k_mis_step(const DB& db, const u32* cand, u32 n, const u32* n_dev, u32* pos, u32* state, u32* blk, u32* resume,
+                u32* next, u32* nnext, u32 lds, u32 lanes, Stream* st) {
   if (!n) return;
 #define MIS_FIRST(G) \
-  KLAUNCH_LDS(mis_step_k<G>, grid_for((size_t)n * G, 64), 64, lds, st, db, cand, n, pos, state, blk, resume, next, \
-              nnext, MIS_TRIES)
+  KLAUNCH_LDS(mis_step_k<G>, grid_for((size_t)n * G, 64), 64, lds, st, db, cand, n, n_dev, pos, state, blk, resume, \
+              next, nnext, MIS_TRIES)
   MIS_LANES(lanes, MIS_FIRST)
 #undef MIS_FIRST
 }
@@ -1954,6 +1994,148 @@ void k_mis_collect(const DB& db, const u32* cand, u32 n, const u32* state, u32* 
   scan_u32(flag_tmp, flag_tmp, n, sc, tmp, st);
   KLAUNCH(mis_pack_k, entries ? std::min(grid_for(n, 256), RED_BLOCKS) : grid_for(n, 256), 256, st, db, cand, state, n,
           sc + 1, flag_tmp, out, entries ? sc + 3 : nullptr);
+}
+
+// Small formulas (up to LCVE_SMALL variables): everything around the election
+// passes in one workgroup and one launch on either side of them, with the
+// number of candidates kept on the device.  Classification, selection, sort
+// and the initial states were eight launches and a read of the candidates'
+// number, break, flags, scan and collection four more, 3-5 us each in a round
+// whose kernels run as long.  With the table above, a call takes 0.82 ms
+// instead of 0.96 at 301 variables (106 launches instead of 154) and 3.17
+// instead of 3.35 at 5,000.
+static_assert(LCVE_SMALL == SO_MAX, "one item per variable");
+__global__ void __launch_bounds__(SO_T) lcve_small_k(DB db, LcveArgs a, bool reject, u32* pos, u32* cand, u32* state,
+                                                     u32* sc) {
+  constexpr int IPT = SO_IPT, W = SO_T / 64;
+  __shared__ u32 sk[lpad(SO_MAX)];
+  __shared__ uint16_t si[lpad(SO_MAX)];
+  __shared__ u32 lw[W], wmax[W];
+  __shared__ u64 lw64[W], wmin[W];
+  unsigned long long hk = ~0ull;
+  u32 top = 0;
+  for (u32 v = threadIdx.x; v <= db.nvars; v += SO_T) {
+    pos[v] = NOPOS;
+    if (!v) continue;
+    const unsigned long long k = lcve_classify_var(db, a, v, top);
+    hk = k < hk ? k : hk;
+  }
+  hk = wave_min64(hk);
+  top = wave_max(top);
+  if ((threadIdx.x & 63) == 0) {
+    wmin[threadIdx.x >> 6] = hk;
+    wmax[threadIdx.x >> 6] = top;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < W; w++) {
+    hk = wmin[w] < hk ? wmin[w] : hk;
+    top = max(top, wmax[w]);
+  }
+  // the candidates before the hard breaker, in variable order
+  const u32 j0 = threadIdx.x * IPT;
+  u32 k[IPT], id[IPT], d[IPT], dst[IPT], keep = 0, n;
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    const u32 v = j0 + i + 1;
+    k[i] = 0;
+    if (v <= db.nvars && a.cflag[v]) {
+      k[i] = a.score[v];
+      if ((((u64)k[i] << 32) | v) < hk) keep |= 1u << i;
+    }
+  }
+  u32 at = block_excl_scan_w<W>(__popc(keep), lw, &n);
+#pragma unroll
+  for (int i = 0; i < IPT; i++)
+    if (keep >> i & 1) {
+      sk[lpad(at)] = k[i];
+      si[lpad(at++)] = (uint16_t)(j0 + i);
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {  // slots past the candidates stay behind them
+    const bool in = j0 + i < n;
+    k[i] = in ? sk[lpad(j0 + i)] : 0xFFFFFFFFu;
+    id[i] = in ? si[lpad(j0 + i)] : 0u;
+  }
+  __syncthreads();
+  const u32 most = min((u32)(hk >> 32), top);
+  const int bits = most ? 32 - __clz(most) : 0;
+  for (int bit = 0; bit < bits; bit += 2) {
+#pragma unroll
+    for (int i = 0; i < IPT; i++) d[i] = (k[i] >> bit) & (bit + 1 < bits ? 3u : 1u);
+    split4<SO_T, IPT>(d, dst, lw64);
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+      sk[lpad(dst[i])] = k[i];
+      si[lpad(dst[i])] = (uint16_t)id[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < IPT; i++) {
+      k[i] = sk[lpad(j0 + i)];
+      id[i] = si[lpad(j0 + i)];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    const u32 j = j0 + i;
+    if (j >= n) continue;
+    const u32 v = id[i] + 1, st = reject && a.cflag[v] == 4 ? 2u : 0u;
+    cand[j] = v;
+    state[j] = st;
+    pos[v] = (j << 2) | st;
+  }
+  if (threadIdx.x == 0) {  // as mis_init_k, and the candidates
+    sc[1] = sc[2] = n;
+    sc[3] = 0;
+    for (u32 q = 0; q < 3; q++) sc[4 + q] = 0, sc[12 + q] = 0;
+    sc[24] = sc[25] = 0;
+  }
+}
+void k_lcve_small(const DB& db, const LcveArgs& a, bool reject, u32* pos, u32* cand, u32* state, u32* sc, Stream* st) {
+  KLAUNCH(lcve_small_k, 1, SO_T, st, db, a, reject, pos, cand, state, sc);
+}
+__global__ void __launch_bounds__(SO_T) collect_small_k(DB db, const u32* cand, const u8* cflag, const u32* state,
+                                                        u32* out, u32* sc) {
+  constexpr int IPT = SO_IPT, W = SO_T / 64;
+  __shared__ u32 lw[W];
+  __shared__ u32 brk;
+  const u32 n = sc[2], j0 = threadIdx.x * IPT;
+  if (threadIdx.x == 0) brk = n;
+  __syncthreads();
+  u32 v[IPT], el = 0;
+#pragma unroll
+  for (int i = 0; i < IPT; i++) {
+    v[i] = 0;
+    if (j0 + i >= n || state[j0 + i] != 1) continue;
+    v[i] = cand[j0 + i];
+    el |= 1u << i;
+    if (cflag[v[i]] == 3) atomicMin(&brk, j0 + i);
+  }
+  __syncthreads();
+  const u32 b = brk;
+#pragma unroll
+  for (int i = 0; i < IPT; i++)
+    if (j0 + i >= b) el &= ~(1u << i);
+  u32 tot, entries, w = 0;
+  u32 at = block_excl_scan_w<W>(__popc(el), lw, &tot);
+#pragma unroll
+  for (int i = 0; i < IPT; i++)
+    if (el >> i & 1) {
+      out[at++] = v[i];
+      w += db.ot_size[V2L(v[i])] + db.ot_size[V2L(v[i]) | 1];
+    }
+  block_excl_scan_w<W>(w, lw, &entries);
+  if (threadIdx.x == 0) {
+    sc[0] = tot;
+    sc[1] = b;
+    sc[3] = entries;
+  }
+}
+void k_collect_small(const DB& db, const u32* cand, const u8* cflag, const u32* state, u32* out, u32* sc, Stream* st) {
+  KLAUNCH(collect_small_k, 1, SO_T, st, db, cand, cflag, state, out, sc);
 }
 
 // ---------------------------------------------------------------- per elected variable

@@ -91,6 +91,10 @@ struct OtpPlan {
 // false when the literal space needs more than OTP_MAX_RANGES ranges;
 // tile_log2: clauses per tile (0: planned)
 bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2 = 0, int xcd = 0);
+// small formulas: the table (or the counts) in one launch, no pair buffer
+constexpr u32 OT_ONE_LITS = 14336, OT_ONE_CLAUSES = 32768;
+bool ot_one_fits(size_t n2, size_t ncls);
+void k_ot_one(const DB& db, u32 n2, bool table, u32* hist, Stream*);
 // counts: p.ncounts + 1 words; pairs: 8-byte aligned, two words per live
 // literal occurrence with 'table', else one.  Without 'table' only hist is
 // written; with it also ot_off (n2 + 1 words), ot_size and ot_refs, and
@@ -145,8 +149,14 @@ u32 mis_lanes_for(u32 n);
 // the first step, over all candidates; blk, resume: of a candidate left
 // undecided, an undecided earlier neighbour and the list entry its scan goes
 // on from; it is appended to next (count in *nnext)
-void k_mis_step(const DB& db, const u32* cand, u32 n, u32* pos, u32* state, u32* blk, u32* resume, u32* next,
-                u32* nnext, u32 lds, u32 lanes, Stream*);
+// (n_dev nullable: their number on the device, at most n)
+void k_mis_step(const DB& db, const u32* cand, u32 n, const u32* n_dev, u32* pos, u32* state, u32* blk, u32* resume,
+                u32* next, u32* nnext, u32 lds, u32 lanes, Stream*);
+// up to LCVE_SMALL variables: classification to initial states in one launch
+// (sc[2]: the candidates), and break to collection in another
+constexpr u32 LCVE_SMALL = 8192;
+void k_lcve_small(const DB& db, const LcveArgs& a, bool reject, u32* pos, u32* cand, u32* state, u32* sc, Stream*);
+void k_collect_small(const DB& db, const u32* cand, const u8* cflag, const u32* state, u32* out, u32* sc, Stream*);
 // the same over the list idx[0..*n_in) (n_in on the device, at most n_bound);
 // *iters counts the calls that had work; *zero is cleared (the counter the
 // next pass appends to)
