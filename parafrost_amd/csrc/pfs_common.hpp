@@ -96,6 +96,10 @@ struct Options {
   int32_t autotune = 1;
 };
 constexpr uint64_t TUNE_MIN_CLAUSES = 1ull << 20;
+// batches of at least this many clauses are appended on the device (clauses of
+// 2.6 literals over 20,000 variables: 0.142 against 0.146 ms on the host at
+// 6,000 clauses, 0.141 against 0.160 at 8,000, 0.178 against 0.620 at 66,000)
+constexpr uint64_t APPEND_DEVICE = 8192;
 
 // Device view of the clause database and per-variable state.  Root
 // assignments are kept per variable (assign[v] = true literal + 1) so that

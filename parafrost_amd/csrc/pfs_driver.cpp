@@ -562,6 +562,95 @@ void Simplifier::append(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
   counts_known_ = false;
   if (maxvar < V_) throw std::invalid_argument("append cannot reduce the number of variables");
   if (maxvar > V_) grow_vars(maxvar);
+  if (!append_device(ncls, offsets, lits)) append_host(ncls, offsets, lits);
+  if (!pending_units_.empty()) {
+    // new root units: assigned and frozen like enqueueUnit, appended to the
+    // trail unpropagated
+    mem_.ensure(ids_, pending_units_.size() * 4, 0, st_);
+    h2d(ids_.p, pending_units_.data(), pending_units_.size() * 4, st_);
+    k_assign_units(make_db(cur_), P<u32>(ids_), (u32)pending_units_.size(), st_);
+    h2d(P<u32>(trail_) + trail_n_, pending_units_.data(), pending_units_.size() * 4, st_);
+    trail_n_ += pending_units_.size();
+    for (u32 u : pending_units_) units_out_.push_back(u);
+    unassigned_ -= (u32)pending_units_.size();
+    pending_units_.clear();
+  }
+  stream_sync(st_);
+}
+
+// Many clauses on the device; false, with nothing changed, if the host has to
+// do it: few clauses (below APPEND_DEVICE the copies and launches take longer
+// than the loop), a refuted or renumbered formula, units of a failed call,
+// clauses that the kernels refuse (malformed, out of range, long, chains of
+// more than AP_PASSES units), or no room for the buffers.
+bool Simplifier::append_device(uint64_t ncls, const uint64_t* offsets, const uint32_t* lits) {
+  if (ncls < APPEND_DEVICE || ncls >= INF / 2 || V_ > 32 * ncls || refuted_ || remapped_ ||
+      !pending_units_.empty() || offsets[ncls] < offsets[0])
+    return false;
+  const uint64_t nl = offsets[ncls] - offsets[0], V1 = (uint64_t)V_ + 1;
+  if (nl >= INF / 4 || lits_end_ + nl + CL_HDR * ncls >= INF / 4) return false;
+  const auto pad = [](uint64_t words) { return (words + 63) & ~(uint64_t)63; };
+  const uint64_t scan = 2 * scan_tmp_bytes(ncls) / 4;
+  Buf raw_d;
+  BufScope release{mem_, {&raw_d}};
+  try {
+    mem_.ensure(raw_d,
+                4 * (4 * pad(V1) + pad(2 * (ncls + 1)) + pad(nl) + pad(2 * ncls) + 3 * pad(ncls) + pad(scan) + AP_FLAGS),
+                0, st_);
+    u32* at = P<u32>(raw_d);
+    const auto take = [&](uint64_t words) { return (at += pad(words)) - pad(words); };
+    AppendArgs a{};
+    a.seen[0] = (u64*)take(2 * pad(V1));
+    a.seen[1] = (u64*)take(2 * pad(V1));
+    u64* off_d = (u64*)take(2 * (ncls + 1));
+    u32* lits_d = take(nl);
+    a.off = off_d;
+    a.lits = lits_d;
+    a.units = (u64*)take(2 * ncls);
+    a.res = take(ncls);
+    a.kept = take(ncls);
+    a.words = take(ncls);
+    void* tmp = take(scan);
+    a.fl = take(AP_FLAGS);
+    a.n = (u32)ncls;
+    a.nl = (u32)nl;
+    h2d(off_d, offsets, (ncls + 1) * 8, st_);
+    if (nl) h2d(lits_d, lits + offsets[0], nl * 4, st_);
+    fill_u32((u32*)a.seen[0], 0xFFFFFFFFu, 4 * pad(V1), st_);
+    fill_u32(a.fl, 0, AP_FLAGS, st_);
+    u32 fl[AP_FLAGS], done = 0, last = AP_PASSES;
+    while (last == AP_PASSES && done < AP_PASSES) {  // a few passes, then a look
+      for (const u32 to = done + 8; done < to; done++) k_append_pass(make_db(cur_), a, done, st_);
+      k_append_place(a, tmp, st_);
+      d2h(fl, a.fl, sizeof(fl), st_);
+      stream_sync(st_);
+      if (fl[0]) return false;
+      for (u32 p = 0; p < done && last == AP_PASSES; p++)
+        if (!fl[AP_CHANGED + p]) last = p;
+    }
+    if (last == AP_PASSES) return false;
+    if (fl[4]) ensure_clause_room(fl[4], fl[5]);
+    k_append_write(make_db(cur_), a, last, (u32)ncls_, (u32)lits_end_, st_);
+    d2h(fl, a.fl, 12, st_);
+    stream_sync(st_);
+    std::vector<u64> units(fl[2]);
+    if (fl[2]) d2h(units.data(), a.units, units.size() * 8, st_);
+    stream_sync(st_);
+    std::sort(units.begin(), units.end());  // by clause
+    for (u64 u : units) {
+      set_host_assign((u32)u);
+      pending_units_.push_back((u32)u);
+    }
+    if (fl[1]) refuted_ = true;
+    ncls_ += fl[4];
+    lits_end_ += fl[5];
+  } catch (AllocFail&) {
+    return false;
+  }
+  return true;
+}
+
+void Simplifier::append_host(uint64_t ncls, const uint64_t* offsets, const uint32_t* lits) {
   std::vector<u32> words, off;
   std::vector<u32> cl;
   uint64_t w = lits_end_;
@@ -570,7 +659,7 @@ void Simplifier::append(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
     bool sat = false;
     for (uint64_t j = offsets[i]; j < offsets[i + 1]; j++) {
       const u32 l = lits[j];
-      if (ABS(l) == 0 || ABS(l) > maxvar) throw std::invalid_argument("literal out of range");
+      if (ABS(l) == 0 || ABS(l) > V_) throw std::invalid_argument("literal out of range");
       const u32 a = h_assign_[ABS(l)];
       if (a) {
         if (a - 1 == l) sat = true;
@@ -613,18 +702,6 @@ void Simplifier::append(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
     ncls_ += nadd;
     lits_end_ += words.size();
     k_prep(make_db(cur_), first, st_);
-  }
-  if (!pending_units_.empty()) {
-    // new root units: assigned and frozen like enqueueUnit, appended to the
-    // trail unpropagated
-    mem_.ensure(ids_, pending_units_.size() * 4, 0, st_);
-    h2d(ids_.p, pending_units_.data(), pending_units_.size() * 4, st_);
-    k_assign_units(make_db(cur_), P<u32>(ids_), (u32)pending_units_.size(), st_);
-    h2d(P<u32>(trail_) + trail_n_, pending_units_.data(), pending_units_.size() * 4, st_);
-    trail_n_ += pending_units_.size();
-    for (u32 u : pending_units_) units_out_.push_back(u);
-    unassigned_ -= (u32)pending_units_.size();
-    pending_units_.clear();
   }
   stream_sync(st_);
 }

@@ -200,6 +200,8 @@ class Simplifier {
   void ere();
   bool ere_pairs();   // pair-parallel ERE; false when it must fall back
   void ere_per_var(); // per-variable ERE with speculative re-runs
+  bool append_device(uint64_t ncls, const uint64_t* offsets, const uint32_t* lits);
+  void append_host(uint64_t ncls, const uint64_t* offsets, const uint32_t* lits);
   void ensure_clause_room(uint64_t add_cls, uint64_t add_lits);
   void ensure_stack(uint64_t words);
   void grow_vars(uint32_t maxvar);

@@ -220,7 +220,7 @@ void k_ere_all_matches(const DB& db, const ErePairs& a, u32 n, const u32* off, u
 void k_assign_units(const DB& db, const u32* lits, u32 n, Stream*);  // assign + FROZEN
 void k_max_list(const DB& db, const u32* lits, u32 n, u32* out, Stream*);
 void k_reduce_lists(const DB& db, Stream*);  // drop deleted entries from every list
-void k_prep(const DB& db, u32 first, Stream*);
+void k_prep(const DB& db, u32 first, Stream*);  // clauses [first, ncls): sort literals, signature
 // the clauses of a caller's database (off[n + 1], lits from off[0] on) built
 // into the pool, originals first, then learnts, each in the given order:
 // headers, literals sorted, signatures, handles.  flags (null: all original)
@@ -236,7 +236,29 @@ struct RawClauses {
   u32 n, words, maxvar;
   u32* sc;
 };
-void k_build_clauses(const DB& db, const RawClauses& raw, void* tmp, Stream*);  // clauses [first, ncls): sort literals, signature
+void k_build_clauses(const DB& db, const RawClauses& raw, void* tmp, Stream*);
+// clauses appended in order under the root assignment, each unit assigning its
+// literal for the clauses after it: passes over all of them until the units
+// stay the same (a pass after that returns at once).  seen[p & 1][variable]:
+// the earliest unit of pass p (pass_word << 32 | clause << 1 | sign), res: per
+// clause its unit literal, 1 if it is empty, else 0; kept, words: 1 and its
+// pool words if it stays with two literals or more.  fl (AP_FLAGS words,
+// zero before): 0 not for the device, 1 an empty clause, 2 units, 4 and 5 the
+// totals of kept and words, AP_CHANGED + p pass p found other units than p - 1
+constexpr u32 AP_PASSES = 32, AP_CHANGED = 8, AP_FLAGS = AP_CHANGED + AP_PASSES, AP_LONG = 128;
+struct AppendArgs {
+  const u64* off;
+  const u32* lits;
+  u32 n, nl;
+  u64* seen[2];
+  u32 *res, *kept, *words, *fl;
+  u64* units;  // (clause << 32 | literal) of the clauses that assign one, any order
+};
+void k_append_pass(const DB& db, const AppendArgs& a, u32 pass, Stream*);
+void k_append_place(const AppendArgs& a, void* tmp, Stream*);  // scans; tmp: 2 * scan_tmp_bytes(n)
+// after pass 'last', the first that changed nothing: the kept clauses into
+// the pool from handle w0 and index c0 on, and the units
+void k_append_write(const DB& db, const AppendArgs& a, u32 last, u32 c0, u32 w0, Stream*);
 void k_zero_sizes(const DB& db, const u32* lits, u32 n, Stream*);
 void k_clear_added(const DB& db, Stream*);  // resolvent marks of an earlier simplify call
 
