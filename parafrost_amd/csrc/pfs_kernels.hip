@@ -2140,17 +2140,6 @@ void k_collect_small(const DB& db, const u32* cand, const u8* cflag, const u32* 
 
 // ---------------------------------------------------------------- per elected variable
 constexpr int VB = 64;  // one wavefront per workgroup for divergent per-variable work
-// Occupancy of the per-variable kernels that walk the pool (the VE gate
-// checks): each of their one-wavefront workgroups reserves PV_LDS bytes of
-// LDS, so at most 160 KiB / PV_LDS of them share a CU: 20 KiB gives 8
-// wavefronts per CU, 2 per SIMD.  Fewer waves keep more of each wave's
-// clauses in L1/L2 while it re-reads them (Tseitin round on MI355X, when
-// SUB and all VE decisions walked the pool: 0 / 12 / 20 / 40 KiB -> 18.1 /
-// 17.4 / 17.25 / 17.35 ms).  The staged kernels use the same size as their
-// working LDS (VR_LDS).
-#ifndef PV_LDS
-#define PV_LDS 20480
-#endif
 
 __global__ void list_sizes_k(DB db, const u32* pv, u32 n, u32 extra, u32* out) {
   const u32 k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2237,12 +2226,23 @@ void k_oblivion(const DB& db, const u32* lits, u32 n, Stream* st) {
 // Per-variable searches over a variable's own two occurrence lists (SUB,
 // the VE decisions that are not settled by the gate checks) re-read those
 // lists all along.  Each variable copies them (lview_words / sview_words
-// words) into LDS and works there.  A wavefront's LDS (cap words) is
-// shared by the variables of one size class: class q < LV_CLASSES - 1
-// gives 64 >> q lanes cap / (64 >> q) words each; the last class (lists
-// larger than cap) works on the pool, 64 lanes to a wavefront.  A
-// wavefront thus runs variables of like size, the largest first, and no
-// lane that reads the pool holds up lanes that work in LDS.
+// words) into LDS and works there.  A workgroup of LV_WAVES wavefronts has
+// LV_WAVE_LDS bytes (cap words) for each.  A wavefront's share is divided
+// among the variables of one size class: class q < LV_BIG gives 32 >> q of
+// them 2 << q lanes and cap / (32 >> q) words each.  Lists larger than that
+// (class LV_BIG) take the whole workgroup's LDS, one variable at a time on
+// its first wavefront, and the last class, larger still, works on the pool,
+// 64 variables to a wavefront.  A wavefront thus runs variables of like size,
+// the largest first, and no lane that reads the pool holds up lanes that work
+// in LDS.
+//
+// The kernels are bound by chains of dependent LDS reads, so by how many
+// wavefronts hide each other's: with 20 KiB to each (8 on a CU) the decisions
+// and SUB of a round took 0.90 + 0.55 ms on the circuit of 2M gates, 0.43 +
+// 0.27 ms on 77,777 variables (three rounds) and 1.04 + 0.77 ms on 100,000
+// gates (five); with 5 KiB (registers allow 24 on a CU) 0.49 + 0.32, 0.24 +
+// 0.16 and 0.60 + 0.50 ms.  3 and 4 KiB are within 10 % of it either way, and
+// with 4 KiB the largest lists that fit would be smaller.
 //
 // work: LV_WORK_HDR words (the first positions of the keys 0..8 in the
 // placed order), then n elected indices.  The key of a variable of class c
@@ -2252,28 +2252,27 @@ void k_oblivion(const DB& db, const u32* lits, u32 n, Stream* st) {
 // the variables of a wavefront have similar work (without it ve_decide_k
 // took 1.11 instead of 0.89 ms on the 2M-gate circuit and sub_k 2.32 instead
 // of 2.06 ms on 10M heavy-tailed variables).
-constexpr u32 LV_CLASSES = 8;
+constexpr u32 LV_CLASSES = 8, LV_BIG = LV_CLASSES - 2;
+constexpr u32 LV_WAVES = 4, LV_WAVE_LDS = 5120, LV_LDS = LV_WAVES * LV_WAVE_LDS, LV_CAP = LV_WAVE_LDS / 4;
 constexpr u32 LV_WORK_HDR = 32;
 constexpr int LV_KEY_BITS = 4;
 static_assert(LV_CLASSES + 1 <= LV_WORK_HDR && LV_CLASSES < (1u << LV_KEY_BITS) && LV_CLASSES == LV_KEPT,
               "class keys");
-__device__ inline u32 lv_class(u32 need, u32 cap) {
+__device__ inline u32 lv_class(u64 need) {
   u32 q = 0;
-  while (q < LV_CLASSES - 1 && need * (64u >> q) > cap) q++;
-  return q;
+  while (q < LV_BIG && need * (32u >> q) > LV_CAP) q++;
+  return q == LV_BIG && need > LV_WAVES * LV_CAP ? LV_CLASSES - 1 : q;
 }
-__device__ inline u32 lv_class_lanes(u32 q) { return q < LV_CLASSES - 1 ? 64u >> q : 64u; }
+__device__ inline u32 lv_class_lanes(u32 q) { return q < LV_BIG ? 32u >> q : 64u; }
 // The least class of a launch over n variables: where they would leave
-// lanes idle, each takes the largest group that keeps the launch within
-// LV_FILL rounds of the resident wavefronts.  A variable's chain of
-// dependent loads and LDS reads is then walked G entries at a time, and the
-// chunks spread over the CUs.  Measured per launch (ve_decide_k, sub_k): 45
-// elected variables 290 + 155 -> 48 + 27 us; 3,206: 350 + 260 -> 86 + 51 us;
-// 43,123: 596 + 303 -> 220 + 151 us (LV_FILL 1 / 2 / 4 / 8: 348 / 286 / 220 /
-// 178 us there, 119 / 116 / 141 / 219 us for 12,314 variables).
-#ifndef LV_FILL
-#define LV_FILL 4
-#endif
+// lanes idle, each takes the largest group that keeps the launch within the
+// lanes of LV_BLOCKS workgroups.  A variable's chain of dependent loads and
+// LDS reads is then walked G entries at a time, and the chunks spread over
+// the CUs.  Against a lane per variable, per launch (ve_decide_k, sub_k): 45
+// elected variables 290 + 155 -> 48 + 27 us; 3,206: 350 + 260 -> 55 + 60 us.
+// Twice and four times the lanes: 0.35 + 0.22 instead of 0.24 + 0.16 ms on
+// 77,777 variables (three launches), 0.17 and 0.19 instead of 0.16 ms on
+// 300,000, 0.59 and 0.55 instead of 0.60 ms on 100,000 gates (five).
 // list occurrences as a descending 5-bit code: exact below 16, then four
 // steps per power of two up to 256
 constexpr int LV_FINE_BITS = 5;
@@ -2282,62 +2281,77 @@ __device__ inline u32 lv_fine(u32 w) {
   const u32 e = 31 - __clz(w);
   return 31 - min(31u, 16 + (e - 4) * 4 + ((w >> (e - 2)) & 3u));
 }
-// one wavefront per workgroup, grid-stride over the chunks of all classes;
+// grid-stride over the chunks of all classes, a wavefront to a chunk;
 // f(k, w, slice, gl, G) runs elected index k with the LDS words
 // [w, w + slice) (w null: on the pool) on a group of G lanes (gl = the
-// lane's place in it): a chunk of class c < LV_CLASSES - 1 holds 64 >> c
-// variables, each on 1 << c lanes.  A class is chosen from a bound on the
-// words the variable needs; the staging checks the slice and falls back to
-// the pool (one lane per variable).
+// lane's place in it): a chunk of class c < LV_BIG holds 32 >> c variables,
+// each on 2 << c lanes.  The variables of class LV_BIG come first, a
+// workgroup to each.  A class is chosen from a bound on the words the
+// variable needs; the staging checks the slice and falls back to the pool
+// (one lane per variable).
 template <class F>
-__device__ inline void lv_chunks(const u32* work, u32 n, u32 cap, u32* lds, F f) {
-  const u32 lane = threadIdx.x;
+__device__ inline void lv_chunks(const u32* work, u32* lds, F f) {
+  const u32 lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const u32* placed = work + LV_WORK_HDR;
   u32 start[LV_CLASSES + 1];  // absent keys start where the next key starts
 #pragma unroll
   for (u32 key = 0; key <= LV_CLASSES; key++) start[key] = work[key];
+  constexpr u32 BIG = LV_CLASSES - 1 - LV_BIG;  // its key
+  const u32 nbig = start[BIG + 1] - start[BIG];
   u32 chunks = 0;
 #pragma unroll
   for (u32 key = 0; key < LV_CLASSES; key++) {
     const u32 L = lv_class_lanes(LV_CLASSES - 1 - key);
-    chunks += (start[key + 1] - start[key] + L - 1) / L;
+    if (key != BIG) chunks += (start[key + 1] - start[key] + L - 1) / L;
   }
-  for (u32 J = blockIdx.x; J < chunks; J += gridDim.x) {
-    // the key of chunk J and its range, found by a loop over constant
-    // indices so that start[] stays in registers (a loop that stops at the
-    // key indexes it at run time, which puts the array in scratch memory)
-    u32 key = LV_CLASSES - 1, j = J, s0 = start[LV_CLASSES - 1], s1 = start[LV_CLASSES];
-    bool found = false;
+  // the first chunks go to the workgroups after those of the large variables,
+  // and to a workgroup's other wavefronts once every workgroup has one
+  u32 J = (blockIdx.x + gridDim.x - nbig % gridDim.x) % gridDim.x + wave * gridDim.x;
+  u32 big = wave ? nbig : blockIdx.x;
+  bool shared = nbig != 0;  // the LDS is the first wavefront's until it is through with them
+  while (true) {
+    u32 r, s1, L, G, slice;
+    u32* w = lds;
+    if (big < nbig) {
+      r = start[BIG] + big, s1 = r + 1, L = 1, G = 64, slice = LV_WAVES * LV_CAP;
+      big += gridDim.x;
+    } else {
+      if (shared) __syncthreads();
+      shared = false;
+      if (J >= chunks) break;
+      // the key of chunk J and its range, found by a loop over constant
+      // indices so that start[] stays in registers (a loop that stops at the
+      // key indexes it at run time, which puts the array in scratch memory)
+      u32 key = LV_CLASSES - 1, j = J, s0 = start[LV_CLASSES - 1];
+      s1 = start[LV_CLASSES];
+      bool found = false;
 #pragma unroll
-    for (u32 q = 0; q < LV_CLASSES - 1; q++) {
-      const u32 L = lv_class_lanes(LV_CLASSES - 1 - q), m = (start[q + 1] - start[q] + L - 1) / L;
-      if (!found) {
-        if (j < m) {
-          key = q, s0 = start[q], s1 = start[q + 1];
-          found = true;
-        } else {
-          j -= m;
+      for (u32 q = 0; q < LV_CLASSES - 1; q++) {
+        if (q == BIG) continue;
+        const u32 Lq = lv_class_lanes(LV_CLASSES - 1 - q), m = (start[q + 1] - start[q] + Lq - 1) / Lq;
+        if (!found) {
+          if (j < m) {
+            key = q, s0 = start[q], s1 = start[q + 1];
+            found = true;
+          } else {
+            j -= m;
+          }
         }
       }
+      L = lv_class_lanes(LV_CLASSES - 1 - key), G = 64 / L, slice = LV_CAP / L;
+      r = s0 + j * L + lane / G;
+      w = key ? lds + wave * LV_CAP + lane / G * slice : nullptr;
+      J += gridDim.x * LV_WAVES;
     }
-    const u32 c = LV_CLASSES - 1 - key, L = lv_class_lanes(c), G = 64 / L;
-    const u32 slot = lane / G, r = s0 + j * L + slot;
-    if (r < s1)
-      f(placed[r], c < LV_CLASSES - 1 ? lds + slot * (cap / L) : nullptr, cap / L, lane % G, G);
-    __syncthreads();  // the next chunk reuses the LDS
+    if (r < s1) f(placed[r], w, slice, lane % G, G);
+    group_sync();  // the next chunk reuses the LDS
   }
 }
-// LDS of each one-wavefront workgroup of the staged launches, and their
-// workgroups: as many as fit the CUs, at most one per variable (a chunk of
-// the upper classes holds one: a workgroup per 64 variables left the chunks
-// of a small formula to one wavefront)
-#ifndef VR_LDS
-#define VR_LDS PV_LDS
-#endif
-constexpr u32 LV_BLOCKS = 256 * (160 * 1024 / VR_LDS);
+// as many workgroups as the LDS lets onto the CUs, at most one per variable
+constexpr u32 LV_BLOCKS = 256 * (160 * 1024 / LV_LDS);
 static u32 lv_floor(u32 n) {
   u32 c = 0;
-  while (c < LV_CLASSES - 2 && ((u64)n << (c + 1)) <= (u64)LV_FILL * LV_BLOCKS * 64) c++;
+  while (c < LV_BIG - 1 && ((u64)n << (c + 2)) <= (u64)LV_BLOCKS * LV_WAVES * 64) c++;
   return c;
 }
 
@@ -2355,24 +2369,25 @@ static u32 lv_floor(u32 n) {
 struct VeClass {
   DB db;
   const u32 *pv, *lsum;
-  u32 cap, least, fine;
+  u32 least, fine;
   __device__ u32 val(u32 k) const { return k; }
   __device__ u32 key(u32 k) const {
     const u32 p = V2L(pv[k]), w = db.ot_size[p] + db.ot_size[p | 1];
     const u64 b = lview_bound(w, (u64)lsum[2 * k] + lsum[2 * k + 1]);
-    u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
-    if (c < LV_CLASSES - 1) c = max(least, min(c + VE_CLASS_BUMP, LV_CLASSES - 2));
+    u32 c = lv_class(b);
+    if (c < LV_BIG) c = max(least, min(c + VE_CLASS_BUMP, LV_BIG - 1));
     return ((LV_CLASSES - 1 - c) << LV_FINE_BITS) | (fine ? lv_fine(w) : 0u);
   }
 };
 // every elected variable on an LDS copy of its lists (the checks read each
 // clause of the lists once, into LDS, instead of once per check from the
 // pool), the gate checks, searches and resolvent count shared by the group
-// (LV_FILL: a few lanes or all 64 per variable).  Bound by chains of LDS
+// (a few lanes or all 64 per variable).  Bound by chains of LDS
 // reads per variable, so what counts is how many of them one lane walks.
-__global__ void ve_decide_k(DB db, Options o, const u32* pv, VeDecision d, const u32* work, u32 n, u32 cap) {
+__global__ void __launch_bounds__(LV_WAVES * 64) ve_decide_k(DB db, Options o, const u32* pv, VeDecision d,
+                                                             const u32* work) {
   extern __shared__ u32 lds[];
-  lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
+  lv_chunks(work, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
     const u32 v = pv[k];
     LView lv;
     if (w && lview_stage(db, v, w, slice, lv, gl, G)) {
@@ -2388,10 +2403,9 @@ __global__ void ve_decide_k(DB db, Options o, const u32* pv, VeDecision d, const
 void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeDecision& d, u32* work,
                  const u32* lsum, void* tmp, Stream* st) {
   if (!n) return;
-  const u32 cap = VR_LDS / 4;
-  place(VeClass{db, pv, lsum, cap, lv_floor(n), (u32)o.work_order}, n, 8, work + LV_WORK_HDR, work, LV_CLASSES + 1,
+  place(VeClass{db, pv, lsum, lv_floor(n), (u32)o.work_order}, n, 8, work + LV_WORK_HDR, work, LV_CLASSES + 1,
         LV_FINE_BITS, nullptr, 0, tmp, st);
-  KLAUNCH_LDS(ve_decide_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, o, pv, d, work, n, cap);
+  KLAUNCH_LDS(ve_decide_k, std::min<u32>(n, LV_BLOCKS), LV_WAVES * 64, LV_LDS, st, db, o, pv, d, work);
 }
 // SUB, staged as the VE searches (the class of a variable from the words of
 // its SView, raised by SUB_CLASS_BUMP)
@@ -2401,23 +2415,23 @@ void k_ve_decide(const DB& db, const Options& o, const u32* pv, u32 n, const VeD
 struct SubClass {
   DB db;
   const u32 *pv, *idx, *lsum;
-  u32 cap, least, fine;
+  u32 least, fine;
   __device__ u32 val(u32 t) const { return idx ? idx[t] : t; }
   __device__ u32 key(u32 t) const {
     const u32 k = val(t), p = V2L(pv[k]), w = db.ot_size[p] + db.ot_size[p | 1];
     const u64 b = sview_bound(w, (u64)lsum[2 * k] + lsum[2 * k + 1]);
-    u32 c = lv_class((u32)min(b, (u64)cap + 1), cap);
-    if (c < LV_CLASSES - 1) c = max(least, min(c + SUB_CLASS_BUMP, LV_CLASSES - 2));
+    u32 c = lv_class(b);
+    if (c < LV_BIG) c = max(least, min(c + SUB_CLASS_BUMP, LV_BIG - 1));
     return ((LV_CLASSES - 1 - c) << LV_FINE_BITS) | (fine ? lv_fine(w) : 0u);
   }
 };
 // take_snap: record each variable's state for the SUB re-runs just before
 // its run (a run changes only the variable's own lists and clauses, so this
 // equals a snapshot before the launch); the staged copy provides it
-__global__ void sub_k(DB db, Options o, const u32* pv, const u32* work, u32 n, u32 cap, SubOut out, SubSnap snap,
-                      u32 take_snap) {
+__global__ void __launch_bounds__(LV_WAVES * 64) sub_k(DB db, Options o, const u32* pv, const u32* work, SubOut out,
+                                                       SubSnap snap, u32 take_snap) {
   extern __shared__ u32 lds[];
-  lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
+  lv_chunks(work, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
     const u32 v = pv[k];
     SView sv;
     if (w && sview_stage(db, v, w, slice, sv, gl, G)) {
@@ -2437,21 +2451,20 @@ __global__ void sub_k(DB db, Options o, const u32* pv, const u32* work, u32 n, u
 void k_sub(const DB& db, const Options& o, const u32* pv, const u32* idx, u32 n, const SubOut& out, u32* work,
            const u32* lsum, void* tmp, const SubSnap* snap, Stream* st) {
   if (!n) return;
-  const u32 cap = VR_LDS / 4;
-  place(SubClass{db, pv, idx, lsum, cap, lv_floor(n), (u32)o.work_order}, n, 8, work + LV_WORK_HDR, work,
+  place(SubClass{db, pv, idx, lsum, lv_floor(n), (u32)o.work_order}, n, 8, work + LV_WORK_HDR, work,
         LV_CLASSES + 1, LV_FINE_BITS, out.n, 1, tmp, st);
-  KLAUNCH_LDS(sub_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, o, pv, work, n, cap, out,
+  KLAUNCH_LDS(sub_k, std::min<u32>(n, LV_BLOCKS), LV_WAVES * 64, LV_LDS, st, db, o, pv, work, out,
               snap ? *snap : SubSnap{}, snap ? 1u : 0u);
 }
 // VE execution, staged as the searches: the resolvent path reads the
 // variable's lists from LDS; EQU substitutions (which rewrite their clauses
 // in place) work on the pool, EQU_CLASS lanes' worth or more each; variables
 // VE keeps are not placed
-constexpr u32 EQU_CLASS = 3;
+constexpr u32 EQU_CLASS = 2;
 struct ApplyClass {
   DB db;
   const u32 *pv, *type, *lsum;
-  u32 cap, least;
+  u32 least;
   __device__ u32 val(u32 t) const { return t; }
   __device__ u32 key(u32 k) const {
     if (!type[k]) return LV_CLASSES;
@@ -2459,15 +2472,16 @@ struct ApplyClass {
     if (type[k] != VT_EQU) {
       const u32 p = V2L(pv[k]);
       const u64 b = lview_bound(db.ot_size[p] + db.ot_size[p | 1], (u64)lsum[2 * k] + lsum[2 * k + 1]);
-      c = lv_class((u32)min(b, (u64)cap + 1), cap);
+      c = lv_class(b);
     }
-    if (c < LV_CLASSES - 1) c = max(c, least);
+    if (c < LV_BIG) c = max(c, least);
     return LV_CLASSES - 1 - c;
   }
 };
-__global__ void ve_apply_k(DB db, const u32* pv, VeDecision d, VeApply a, const u32* work, u32 n, u32 cap) {
+__global__ void __launch_bounds__(LV_WAVES * 64) ve_apply_k(DB db, const u32* pv, VeDecision d, VeApply a,
+                                                            const u32* work) {
   extern __shared__ u32 lds[];
-  lv_chunks(work, n, cap, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
+  lv_chunks(work, lds, [&](u32 k, u32* w, u32 slice, u32 gl, u32 G) {
     const u32 v = pv[k];
     LView lv;
     if (w && d.type[k] != VT_EQU && lview_stage(db, v, w, slice, lv, gl, G)) {
@@ -2481,10 +2495,9 @@ __global__ void ve_apply_k(DB db, const u32* pv, VeDecision d, VeApply a, const 
 void k_ve_apply(const DB& db, const u32* pv, u32 n, const VeDecision& d, const VeApply& a, u32* work,
                 const u32* lsum, u32* zero, u32 nz, void* tmp, Stream* st) {
   if (!n) return;
-  const u32 cap = VR_LDS / 4;
-  place(ApplyClass{db, pv, d.type, lsum, cap, lv_floor(n)}, n, LV_KEY_BITS, work + LV_WORK_HDR, work, LV_CLASSES + 1,
+  place(ApplyClass{db, pv, d.type, lsum, lv_floor(n)}, n, LV_KEY_BITS, work + LV_WORK_HDR, work, LV_CLASSES + 1,
         0, zero, nz, tmp, st);
-  KLAUNCH_LDS(ve_apply_k, std::min<u32>(n, LV_BLOCKS), VB, VR_LDS, st, db, pv, d, a, work, n, cap);
+  KLAUNCH_LDS(ve_apply_k, std::min<u32>(n, LV_BLOCKS), LV_WAVES * 64, LV_LDS, st, db, pv, d, a, work);
 }
 // in elected order (by score, so of similar lists): heaviest lists first took
 // 0.69 instead of 0.61 ms for the two launches on 2.5M heavy-tailed variables
