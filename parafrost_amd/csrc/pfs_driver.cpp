@@ -930,11 +930,12 @@ void Simplifier::create_ot() {
 // no extra memory.
 bool Simplifier::otp_room(const OtpPlan& p) {
   const size_t slots = lits_end_ >= CL_HDR * ncls_ ? lits_end_ - CL_HDR * ncls_ : lits_end_;
-  const size_t counts_words = ((p.ncounts + 1 + 63) & ~(size_t)63);
-  const size_t need = counts_words + 2 * slots + 64;
+  const auto pad = [](size_t words) { return (words + 63) & ~(size_t)63; };
+  const size_t second = p.tiles2 ? pad(p.nr + 1) + pad(p.ncounts2) : 0;
+  const size_t need = pad(p.ncounts + 1) + second + 2 * slots + 64;
   if (need * 4 <= otp_.cap) return true;
   const size_t counts_cap = (size_t)p.nr * ((std::max<size_t>(ccap_, ncls_) + p.ct - 1) / p.ct);
-  const size_t want = ((counts_cap + 1 + 63) & ~(size_t)63) + 2 * (slots + slots / 2) + 64;
+  const size_t want = pad(counts_cap + 1) + second + second / 2 + 2 * (slots + slots / 2) + 64;
   try {
     mem_.ensure(otp_, want * 4, 0, st_);
     return true;
@@ -960,10 +961,25 @@ void Simplifier::ot_counts(bool table) {
       used_tile_ = (int32_t)ilog2(p.ct);
       return true;
     }
+    const auto pad = [](size_t words) { return (words + 63) & ~(size_t)63; };  // to 256 bytes
+    const size_t slots = lits_end_ >= CL_HDR * ncls_ ? lits_end_ - CL_HDR * ncls_ : lits_end_;
+    OtpPlan two;
+    // two steps: the second one's pairs wait in the other block's pool, which
+    // nothing uses until the collection writes it
+    if (table && 2 * slots + 64 <= lcap_ && otp_plan2(n2, db.ncls, slots, &two, tile, opt.otp_xcd) && otp_room(two)) {
+      mem_.ensure(tmp_, std::max(tmp_.cap, scan_tmp_bytes(std::max(two.ncounts, two.ncounts2))), 0, st_);
+      u32* counts = P<u32>(otp_);
+      u32* tb = counts + pad(two.ncounts + 1);
+      u32* counts2 = tb + pad(two.nr + 1);
+      k_ot_ranges2(db, two, (u32)n2, counts, tb, counts2, counts2 + pad(two.ncounts2), lits_[1 - cur_].p, hist, tmp_.p,
+                   st_);
+      used_tile_ = (int32_t)ilog2(two.ct);
+      return true;
+    }
     if (!otp_room(p)) return false;
     mem_.ensure(tmp_, std::max(tmp_.cap, scan_tmp_bytes(p.ncounts)), 0, st_);
     u32* counts = P<u32>(otp_);
-    u32* pairs = counts + ((p.ncounts + 1 + 63) & ~(size_t)63);  // 256-byte aligned
+    u32* pairs = counts + pad(p.ncounts + 1);
     k_ot_ranges(db, p, (u32)n2, counts, pairs, table, hist, tmp_.p, st_);
     used_tile_ = (int32_t)ilog2(p.ct);
     return true;

@@ -1191,55 +1191,52 @@ constexpr int OTP_LD = 8;
 // more loads in flight per range and fewer table slices open at once per
 // XCD; reserving 64 KiB of LDS on top changed nothing
 constexpr int OTP_RTB = 1024;
-template <bool TABLE>
-__global__ void __launch_bounds__(OTP_RTB) otp_range_k(DB db, int bits, u32 n2, u32 nblk, const u32* offs,
-                                                  const u32* total, const void* in, u32* hist) {
+template <bool TABLE, int RTB>
+__device__ inline void otp_range(const DB& db, int bits, u32 n2, u32 b0, u32 b1, const u32* total, const void* in,
+                                 u32* hist, u32* lc) {
   const u32* plit = (const u32*)in;
   const uint2* pair = (const uint2*)in;
-  extern __shared__ u32 lc[];
-  __shared__ u32 lw[OTP_RTB / 64];
+  __shared__ u32 lw[RTB / 64];
   const u32 r = blockIdx.x, nl = 1u << bits, base = r << bits;
-  const u32 b0 = offs[(size_t)r * nblk];
-  const u32 b1 = r + 1 < gridDim.x ? offs[(size_t)(r + 1) * nblk] : *total;
-  for (u32 j = threadIdx.x; j < nl; j += OTP_RTB) lc[j] = 0;
+  for (u32 j = threadIdx.x; j < nl; j += RTB) lc[j] = 0;
   __syncthreads();
-  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * OTP_RTB) {
+  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * RTB) {
     u32 l[OTP_LD];
 #pragma unroll
     for (int q = 0; q < OTP_LD; q++)
-      l[q] = p + q * OTP_RTB < b1 ? (TABLE ? pair[p + q * OTP_RTB].x : plit[p + q * OTP_RTB]) : OTP_NONE;
+      l[q] = p + q * RTB < b1 ? (TABLE ? pair[p + q * RTB].x : plit[p + q * RTB]) : OTP_NONE;
 #pragma unroll
     for (int q = 0; q < OTP_LD; q++)
       if (l[q] != OTP_NONE) atomicAdd(&lc[l[q] - base], 1u);
   }
   __syncthreads();
   if (!TABLE) {
-    for (u32 j = threadIdx.x; j < nl; j += OTP_RTB)
+    for (u32 j = threadIdx.x; j < nl; j += RTB)
       if (base + j < n2) hist[base + j] = lc[j];
     return;
   }
-  // exclusive scan: each thread owns nl / OTP_RTB consecutive counters
-  const u32 per = nl / OTP_RTB, j0 = threadIdx.x * per;
+  // exclusive scan: each thread owns nl / RTB consecutive counters
+  const u32 per = nl / RTB, j0 = threadIdx.x * per;
   u32 s = 0;
   for (u32 k = 0; k < per; k++) s += lc[j0 + k];
   u32 tot;
-  u32 pre = block_excl_scan_w<OTP_RTB / 64>(s, lw, &tot) + b0;
+  u32 pre = block_excl_scan_w<RTB / 64>(s, lw, &tot) + b0;
   for (u32 k = 0; k < per; k++) {
     const u32 v = lc[j0 + k];
     lc[j0 + k] = pre;
     pre += v;
   }
   __syncthreads();
-  for (u32 j = threadIdx.x; j < nl; j += OTP_RTB)
+  for (u32 j = threadIdx.x; j < nl; j += RTB)
     if (base + j < n2) db.ot_off[base + j] = lc[j];
   if (r + 1 == gridDim.x && threadIdx.x == 0) db.ot_off[n2] = *total;
   // every offset is read out of LDS before any cursor moves
   __syncthreads();
-  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * OTP_RTB) {
+  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * RTB) {
     u32 l[OTP_LD], c[OTP_LD];
 #pragma unroll
     for (int q = 0; q < OTP_LD; q++) {
-      const uint2 e = p + q * OTP_RTB < b1 ? pair[p + q * OTP_RTB] : make_uint2(OTP_NONE, 0u);
+      const uint2 e = p + q * RTB < b1 ? pair[p + q * RTB] : make_uint2(OTP_NONE, 0u);
       l[q] = e.x;
       c[q] = e.y;
     }
@@ -1249,12 +1246,172 @@ __global__ void __launch_bounds__(OTP_RTB) otp_range_k(DB db, int bits, u32 n2, 
   }
   __syncthreads();
   // the cursors end at the next list's offset: size = cursor - offset
-  for (u32 j = threadIdx.x; j < nl; j += OTP_RTB)
+  for (u32 j = threadIdx.x; j < nl; j += RTB)
     if (base + j < n2) {
       const u32 sz = lc[j] - db.ot_off[base + j];
       db.ot_size[base + j] = sz;
       hist[base + j] = sz;
     }
+}
+template <bool TABLE>
+__global__ void __launch_bounds__(OTP_RTB) otp_range_k(DB db, int bits, u32 n2, u32 nblk, const u32* offs,
+                                                  const u32* total, const void* in, u32* hist) {
+  extern __shared__ u32 lc[];
+  const u32 r = blockIdx.x, b0 = offs[(size_t)r * nblk];
+  const u32 b1 = r + 1 < gridDim.x ? offs[(size_t)(r + 1) * nblk] : *total;
+  otp_range<TABLE, OTP_RTB>(db, bits, n2, b0, b1, total, in, hist, lc);
+}
+
+// In two steps for many literals.  One step needs a range per 4,096 or 8,192
+// literals: a tile's pairs go to thousands of open lines, which the L2s write
+// back a few words at a time, and a range's lists are as scattered.  Here the
+// first step fills one line per OTP2_BITS + OTP2_SUB bits of literals, the
+// pairs of each such range are partitioned again among its 1 << OTP2_SUB
+// parts, and a part's lists are put together in LDS.  10M variables in 40M
+// clauses: counts, partition and ranges 0.44 + 1.63 + 1.53 ms in one step;
+// 0.30 + 0.88, 0.19 + 0.42 and 0.48 ms here (0.72 and 0.83 for the last two
+// without LDS).
+//
+// tb: the first tile of each range (tiles of OTP2_TILE pairs, none crossing
+// ranges), tb[nr] their number
+__global__ void __launch_bounds__(OTP2_MAX_RANGES) otp2_tiles_k(const u32* offs, u32 nblk, u32 nr, const u32* total,
+                                                               u32* tb) {
+  __shared__ u32 lw[OTP2_MAX_RANGES / 64];
+  const u32 r = threadIdx.x;
+  u32 n = 0, tot;
+  if (r < nr) n = (r + 1 < nr ? offs[(size_t)(r + 1) * nblk] : *total) - offs[(size_t)r * nblk];
+  const u32 pre = block_excl_scan_w<OTP2_MAX_RANGES / 64>((n + OTP2_TILE - 1) / OTP2_TILE, lw, &tot);
+  if (r < nr) tb[r] = pre;
+  if (r == 0) tb[nr] = tot;
+}
+struct Otp2Tile {
+  u32 b0, b1;     // its pairs
+  u32 at, step;   // its count of part s is word at + s * step
+};
+__device__ inline bool otp2_tile(u32 t, const u32* offs, u32 nblk, u32 nr, const u32* total, const u32* tb,
+                                 Otp2Tile* x) {
+  if (t >= tb[nr]) return false;
+  u32 lo = 0, hi = nr;  // tb[lo] <= t < tb[hi]
+  while (hi - lo > 1) {
+    const u32 m = (lo + hi) >> 1;
+    if (tb[m] <= t) lo = m;
+    else hi = m;
+  }
+  const u32 end = lo + 1 < nr ? offs[(size_t)(lo + 1) * nblk] : *total;
+  x->b0 = offs[(size_t)lo * nblk] + (t - tb[lo]) * OTP2_TILE;
+  x->b1 = min(end, x->b0 + OTP2_TILE);
+  x->step = tb[lo + 1] - tb[lo];
+  x->at = (tb[lo] << OTP2_SUB) + (t - tb[lo]);
+  return true;
+}
+constexpr u32 OTP2_PARTS = 1u << OTP2_SUB;
+__global__ void __launch_bounds__(OTP_TB) otp2_count_k(const u32* offs, u32 nblk, u32 nr, const u32* total,
+                                                       const u32* tb, const uint2* in, u32* counts) {
+  __shared__ u32 lc[OTP2_PARTS];
+  Otp2Tile x;
+  if (!otp2_tile(blockIdx.x, offs, nblk, nr, total, tb, &x)) return;  // the whole workgroup
+  if (threadIdx.x < OTP2_PARTS) lc[threadIdx.x] = 0;
+  __syncthreads();
+  for (u32 p = x.b0 + threadIdx.x; p < x.b1; p += OTP_LD * OTP_TB) {
+    u32 l[OTP_LD];
+#pragma unroll
+    for (int q = 0; q < OTP_LD; q++) l[q] = p + q * OTP_TB < x.b1 ? in[p + q * OTP_TB].x : OTP_NONE;
+#pragma unroll
+    for (int q = 0; q < OTP_LD; q++)
+      if (l[q] != OTP_NONE) atomicAdd(&lc[(l[q] >> OTP2_BITS) & (OTP2_PARTS - 1)], 1u);
+  }
+  __syncthreads();
+  if (threadIdx.x < OTP2_PARTS) counts[x.at + threadIdx.x * x.step] = lc[threadIdx.x];
+}
+// the tile in its parts' order in LDS first, so that the stores go out in runs
+__global__ void __launch_bounds__(OTP_TB) otp2_part_k(const u32* offs, u32 nblk, u32 nr, const u32* total,
+                                                      const u32* tb, const uint2* in, const u32* counts, uint2* out) {
+  __shared__ uint2 st[OTP2_TILE];
+  __shared__ u32 cnt[OTP2_PARTS], to[OTP2_PARTS];  // to: where a part's run goes, less its place in the tile
+  __shared__ u32 lw[OTP_TB / 64];
+  Otp2Tile x;
+  if (!otp2_tile(blockIdx.x, offs, nblk, nr, total, tb, &x)) return;
+  if (threadIdx.x < OTP2_PARTS) cnt[threadIdx.x] = 0;
+  __syncthreads();
+  constexpr int PT = OTP2_TILE / OTP_TB;
+  const u32 n = x.b1 - x.b0;
+  uint2 e[PT];
+  u32 at[PT];
+#pragma unroll
+  for (int q = 0; q < PT; q++) {
+    const u32 j = q * OTP_TB + threadIdx.x;
+    if (j < n) e[q] = in[x.b0 + j];
+  }
+#pragma unroll
+  for (int q = 0; q < PT; q++)
+    if (q * OTP_TB + threadIdx.x < n) at[q] = atomicAdd(&cnt[(e[q].x >> OTP2_BITS) & (OTP2_PARTS - 1)], 1u);
+  __syncthreads();
+  u32 tot;
+  const u32 c = threadIdx.x < OTP2_PARTS ? cnt[threadIdx.x] : 0u;
+  const u32 pre = block_excl_scan_w<OTP_TB / 64>(c, lw, &tot);
+  if (threadIdx.x < OTP2_PARTS) {
+    cnt[threadIdx.x] = pre;
+    to[threadIdx.x] = counts[x.at + threadIdx.x * x.step] - pre;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PT; q++)
+    if (q * OTP_TB + threadIdx.x < n) st[cnt[(e[q].x >> OTP2_BITS) & (OTP2_PARTS - 1)] + at[q]] = e[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PT; q++) {
+    const u32 j = q * OTP_TB + threadIdx.x;
+    if (j < n) {
+      const uint2 v = st[j];
+      out[to[(v.x >> OTP2_BITS) & (OTP2_PARTS - 1)] + j] = v;
+    }
+  }
+}
+// a workgroup per part; lists of up to OTP2_STAGE entries (most parts, at 8
+// occurrences a literal) are put together in LDS and written in one run
+constexpr u32 OTP2_STAGE = 8 * OTP_RTB;
+static_assert(OTP_RTB == 1 << OTP2_BITS, "a literal to a thread");
+__global__ void __launch_bounds__(OTP_RTB) otp2_range_k(DB db, u32 n2, const u32* tb, const u32* counts,
+                                                        const u32* total, const uint2* in, u32* hist) {
+  __shared__ u32 lc[OTP_RTB], st[OTP2_STAGE], lw[OTP_RTB / 64];
+  const u32 r = blockIdx.x >> OTP2_SUB, s = blockIdx.x & (OTP2_PARTS - 1), step = tb[r + 1] - tb[r];
+  const u32 word = (tb[r] << OTP2_SUB) + s * step;  // the next part starts where the next word says
+  const u32 b0 = counts[word], b1 = counts[word + step], n = b1 - b0;
+  if (n > OTP2_STAGE) {
+    otp_range<true, OTP_RTB>(db, OTP2_BITS, n2, b0, b1, total, in, hist, lc);
+    return;
+  }
+  constexpr int PT = OTP2_STAGE / OTP_RTB;
+  const u32 base = blockIdx.x << OTP2_BITS, lit = base + threadIdx.x;
+  lc[threadIdx.x] = 0;
+  __syncthreads();
+  uint2 e[PT];
+  u32 at[PT];
+#pragma unroll
+  for (int q = 0; q < PT; q++) {
+    const u32 j = q * OTP_RTB + threadIdx.x;
+    if (j < n) e[q] = in[b0 + j];
+  }
+#pragma unroll
+  for (int q = 0; q < PT; q++)
+    if (q * OTP_RTB + threadIdx.x < n) at[q] = atomicAdd(&lc[e[q].x - base], 1u);
+  __syncthreads();
+  u32 tot;
+  const u32 size = lc[threadIdx.x];
+  const u32 pre = block_excl_scan_w<OTP_RTB / 64>(size, lw, &tot);
+  lc[threadIdx.x] = pre;
+  if (lit < n2) {
+    db.ot_off[lit] = b0 + pre;
+    db.ot_size[lit] = size;
+    hist[lit] = size;
+  }
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) db.ot_off[n2] = *total;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PT; q++)
+    if (q * OTP_RTB + threadIdx.x < n) st[lc[e[q].x - base] + at[q]] = e[q].y;
+  __syncthreads();
+  for (u32 j = threadIdx.x; j < n; j += OTP_RTB) db.ot_refs[b0 + j] = st[j];
 }
 bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2, int xcd) {
   // LDS per workgroup: nr words in the tile kernels, 1 << bits words in
@@ -1278,6 +1435,17 @@ bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2, int xcd) {
   p->ct = (u32)ct;
   p->nblk = (u32)((ncls + ct - 1) / ct);
   p->ncounts = (size_t)p->nr * p->nblk;
+  return true;
+}
+bool otp_plan2(size_t n2, size_t ncls, size_t pairs, OtpPlan* p, int tile_log2, int xcd) {
+  constexpr int bits = OTP2_BITS + OTP2_SUB;
+  const size_t nr = (n2 + ((size_t)1 << bits) - 1) >> bits;
+  if (n2 < OTP2_MIN_LITS || nr > OTP2_MAX_RANGES || !otp_plan(n2, ncls, p, tile_log2, xcd)) return false;
+  p->bits = bits;
+  p->nr = (u32)nr;
+  p->ncounts = (size_t)p->nr * p->nblk;
+  p->tiles2 = (u32)(pairs / OTP2_TILE + nr);
+  p->ncounts2 = ((size_t)p->tiles2 << OTP2_SUB) + 1;
   return true;
 }
 // the same for a formula whose literals fit one workgroup's counters and
@@ -1321,6 +1489,21 @@ void k_ot_one(const DB& db, u32 n2, bool table, u32* hist, Stream* st) {
 }
 // counts: p.ncounts + 1 words; pairs: 8-byte aligned, two words per live
 // occurrence (table) or one (hist only); tmp: scan_tmp_bytes(p.ncounts)
+void k_ot_ranges2(const DB& db, const OtpPlan& p, u32 n2, u32* counts, u32* tb, u32* counts2, void* pairs,
+                  void* pairs2, u32* hist, void* tmp, Stream* st) {
+  const size_t lds_r = (size_t)p.nr * 4;
+  const u32* total = counts + p.ncounts;
+  KLAUNCH_LDS(otp_count_k, p.nblk, OTP_TB, lds_r, st, db, p.ct, p.bits, p.nr, p.nblk, p.xcd, counts);
+  scan_u32(counts, counts, p.ncounts, counts + p.ncounts, tmp, st);
+  KLAUNCH_LDS(otp_part_k<true>, p.nblk, OTP_TB, lds_r, st, db, p.ct, p.bits, p.nr, p.nblk, p.xcd, counts, pairs);
+  KLAUNCH(otp2_tiles_k, 1, OTP2_MAX_RANGES, st, counts, p.nblk, p.nr, total, tb);
+  KLAUNCH(otp2_count_k, p.tiles2, OTP_TB, st, counts, p.nblk, p.nr, total, tb, (const uint2*)pairs, counts2);
+  scan_u32(counts2, counts2, p.ncounts2, nullptr, tmp, st);  // past the last tile's: the total
+  KLAUNCH(otp2_part_k, p.tiles2, OTP_TB, st, counts, p.nblk, p.nr, total, tb, (const uint2*)pairs, counts2,
+          (uint2*)pairs2);
+  KLAUNCH(otp2_range_k, (n2 + (1u << OTP2_BITS) - 1) >> OTP2_BITS, OTP_RTB, st, db, n2, tb, counts2, total,
+          (const uint2*)pairs2, hist);
+}
 void k_ot_ranges(const DB& db, const OtpPlan& p, u32 n2, u32* counts, void* pairs, bool table, u32* hist,
                  void* tmp, Stream* st) {
   const size_t lds_r = (size_t)p.nr * 4, lds_b = ((size_t)4 << p.bits);

@@ -87,10 +87,22 @@ struct OtpPlan {
   u32 nblk;       // tiles
   size_t ncounts; // nr * nblk
   int xcd;        // tiles spread by XCD: each of the 8 XCDs takes a run of consecutive tiles
+  // two steps: the ranges above (OTP2_SUB bits wider) are partitioned again,
+  // over at most tiles2 tiles of OTP2_TILE pairs, into ranges of 1 << OTP2_BITS
+  u32 tiles2 = 0;      // 0: one step
+  size_t ncounts2 = 0; // words of the second step's counts
 };
 // false when the literal space needs more than OTP_MAX_RANGES ranges;
 // tile_log2: clauses per tile (0: planned)
 bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2 = 0, int xcd = 0);
+// the same in two steps, for at most 'pairs' occurrences (with the table
+// only); false where one step is the faster way
+// (tables of a round, one step against two: 1M literals 0.12 and 0.12 ms, 4M
+// 0.31 and 0.32, 5M in heavy-tailed clauses 0.72 and 0.55, 20M 3.8 and 2.3)
+constexpr int OTP2_BITS = 10, OTP2_SUB = 7;
+constexpr u32 OTP2_TILE = 8192, OTP2_MAX_RANGES = 1024;
+constexpr size_t OTP2_MIN_LITS = (size_t)1 << 22;
+bool otp_plan2(size_t n2, size_t ncls, size_t pairs, OtpPlan* p, int tile_log2 = 0, int xcd = 0);
 // small formulas: the table (or the counts) in one launch, no pair buffer
 constexpr u32 OT_ONE_LITS = 14336, OT_ONE_CLAUSES = 32768;
 bool ot_one_fits(size_t n2, size_t ncls);
@@ -101,6 +113,11 @@ void k_ot_one(const DB& db, u32 n2, bool table, u32* hist, Stream*);
 // hist = ot_size.  tmp: scan_tmp_bytes(p.ncounts)
 void k_ot_ranges(const DB& db, const OtpPlan& p, u32 n2, u32* counts, void* pairs, bool table, u32* hist,
                  void* tmp, Stream*);
+// in two steps (a plan of otp_plan2): counts as above, tb: p.nr + 1 words,
+// counts2: p.ncounts2 words, pairs and pairs2: two words per occurrence each;
+// tmp: scan_tmp_bytes of the larger count
+void k_ot_ranges2(const DB& db, const OtpPlan& p, u32 n2, u32* counts, u32* tb, u32* counts2, void* pairs,
+                  void* pairs2, u32* hist, void* tmp, Stream*);
 // sort the two lists of each variable pv[0..nvars) by the total order
 // classes: 12 * nvars words of scratch; cnt: 2 device words, zero; tmp:
 // 2 * scan_tmp_bytes(2 * nvars)

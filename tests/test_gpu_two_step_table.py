@@ -1,0 +1,69 @@
+"""From 4,194,304 literals on the occurrence table is built in two steps of
+partitioning: sizes around that limit and around whole ranges, with ranges
+that hold nothing, literals that fill many tiles and lists at the ends of
+ranges, against the table of one atomic per occurrence and the oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from parafrost_amd import gen
+from tests.common import diff
+
+pytestmark = pytest.mark.gpu
+
+
+def _formula(nvars, nclauses, seed):
+    rng = np.random.default_rng(seed)
+    # variables at the ends of ranges, in a few dense stretches, and one in many clauses
+    edges = np.concatenate([np.arange(k - 3, k + 4) for k in range(0, nvars + 512, 512)])
+    edges = edges[(edges >= 1) & (edges <= nvars)]
+    dense = np.concatenate([np.arange(s, min(nvars, s + 9000)) for s in (1, nvars // 3, nvars - 8000)])
+    size = rng.choice([2, 3, 3, 4], nclauses)
+    pick = rng.random(size.sum())
+    v = np.where(pick < 0.5, rng.choice(dense, size.sum()), rng.choice(edges, size.sum()))
+    cid = np.repeat(np.arange(nclauses), size)
+    first = np.concatenate([[0], np.cumsum(size)[:-1]])
+    v[first[: nclauses // 3]] = nvars  # the last variable in a third of the clauses
+    lit = 2 * v + (rng.random(size.sum()) < 0.5)
+    key = np.unique(cid << 32 | lit)
+    keep = np.ones(len(key), bool)
+    keep[1:] = (key[1:] >> 1) != (key[:-1] >> 1)
+    key = key[keep]
+    n = np.bincount(key >> 32, minlength=nclauses)
+    key, n = key[n[key >> 32] > 1], n[n > 1]
+    off = np.zeros(len(n) + 1, np.uint64)
+    off[1:] = np.cumsum(n)
+    return gen.Cnf(nvars, off, (key & 0xFFFFFFFF).astype(np.uint32))
+
+
+def _run(cnf, **opts):
+    from parafrost_amd.simplifier import Simplifier
+    s = Simplifier(0, phases=2, bce=1, **opts)
+    try:
+        s.upload(cnf.maxvar, cnf.offsets, cnf.lits)
+        return s.result(s.simplify())
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("nvars", [2097150, 2097151, 2097152, 2162686, 2162687, 2162688, 2500001, 5242879])
+@pytest.mark.parametrize("nclauses", [3, 150000])
+def test_sizes(nvars, nclauses):
+    cnf = _formula(nvars, nclauses, nvars + nclauses)
+    a = _run(cnf)
+    print(nvars, cnf.nclauses, [x["elected"] for x in a.rounds], flush=True)
+    d = diff(a, _run(cnf, otpranges=0))
+    assert not d, d
+    if nvars in (2097151, 2162687):
+        d = diff(a, oracle.simplify(cnf.maxvar, cnf.offsets, cnf.lits, det=1, phases=2, bce_en=1))
+        assert not d, d
+
+
+@pytest.mark.parametrize("tile", [10, 13])
+def test_tiles_and_no_room(tile):
+    """Other tiles of the first step, and a pool too small for the second's pairs."""
+    cnf = _formula(2300000, 200000, tile)
+    a = _run(cnf)
+    for opts in ({"otptile": tile}, {"otptile": tile, "otpxcd": 0}, {"literalsmul": 0}):
+        d = diff(a, _run(cnf, **opts))
+        assert not d, (opts, d)
