@@ -1191,52 +1191,89 @@ constexpr int OTP_LD = 8;
 // more loads in flight per range and fewer table slices open at once per
 // XCD; reserving 64 KiB of LDS on top changed nothing
 constexpr int OTP_RTB = 1024;
-template <bool TABLE, int RTB>
+// the lists of a range with at most this many entries are put together in LDS
+// and written in one run
+constexpr u32 OTP_LISTS = OTP_LD * OTP_RTB;
+template <bool TABLE>
 __device__ inline void otp_range(const DB& db, int bits, u32 n2, u32 b0, u32 b1, const u32* total, const void* in,
-                                 u32* hist, u32* lc) {
+                                 u32* hist, u32* lc, u32* st) {
   const u32* plit = (const u32*)in;
   const uint2* pair = (const uint2*)in;
-  __shared__ u32 lw[RTB / 64];
+  __shared__ u32 lw[OTP_RTB / 64];
   const u32 r = blockIdx.x, nl = 1u << bits, base = r << bits;
-  for (u32 j = threadIdx.x; j < nl; j += RTB) lc[j] = 0;
+  for (u32 j = threadIdx.x; j < nl; j += OTP_RTB) lc[j] = 0;
   __syncthreads();
-  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * RTB) {
+  if (TABLE && b1 - b0 <= OTP_LISTS) {
+    const u32 n = b1 - b0, per = nl / OTP_RTB, j0 = threadIdx.x * per;
+    uint2 e[OTP_LD];
+    u32 at[OTP_LD];
+#pragma unroll
+    for (int q = 0; q < OTP_LD; q++)
+      if (q * OTP_RTB + threadIdx.x < n) e[q] = pair[b0 + q * OTP_RTB + threadIdx.x];
+#pragma unroll
+    for (int q = 0; q < OTP_LD; q++)
+      if (q * OTP_RTB + threadIdx.x < n) at[q] = atomicAdd(&lc[e[q].x - base], 1u);
+    __syncthreads();
+    u32 s = 0, tot;
+    for (u32 k = 0; k < per; k++) s += lc[j0 + k];
+    u32 pre = block_excl_scan_w<OTP_RTB / 64>(s, lw, &tot);
+    for (u32 k = 0; k < per; k++) {
+      const u32 v = lc[j0 + k];
+      lc[j0 + k] = pre;
+      pre += v;
+    }
+    __syncthreads();
+    for (u32 j = threadIdx.x; j < nl && base + j < n2; j += OTP_RTB) {
+      const u32 o = lc[j], sz = (j + 1 < nl ? lc[j + 1] : n) - o;
+      db.ot_off[base + j] = b0 + o;
+      db.ot_size[base + j] = sz;
+      hist[base + j] = sz;
+    }
+    if (r + 1 == gridDim.x && threadIdx.x == 0) db.ot_off[n2] = *total;
+#pragma unroll
+    for (int q = 0; q < OTP_LD; q++)
+      if (q * OTP_RTB + threadIdx.x < n) st[lc[e[q].x - base] + at[q]] = e[q].y;
+    __syncthreads();
+    for (u32 j = threadIdx.x; j < n; j += OTP_RTB) db.ot_refs[b0 + j] = st[j];
+    return;
+  }
+  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * OTP_RTB) {
     u32 l[OTP_LD];
 #pragma unroll
     for (int q = 0; q < OTP_LD; q++)
-      l[q] = p + q * RTB < b1 ? (TABLE ? pair[p + q * RTB].x : plit[p + q * RTB]) : OTP_NONE;
+      l[q] = p + q * OTP_RTB < b1 ? (TABLE ? pair[p + q * OTP_RTB].x : plit[p + q * OTP_RTB]) : OTP_NONE;
 #pragma unroll
     for (int q = 0; q < OTP_LD; q++)
       if (l[q] != OTP_NONE) atomicAdd(&lc[l[q] - base], 1u);
   }
   __syncthreads();
   if (!TABLE) {
-    for (u32 j = threadIdx.x; j < nl; j += RTB)
+    for (u32 j = threadIdx.x; j < nl; j += OTP_RTB)
       if (base + j < n2) hist[base + j] = lc[j];
     return;
   }
-  // exclusive scan: each thread owns nl / RTB consecutive counters
-  const u32 per = nl / RTB, j0 = threadIdx.x * per;
+  // exclusive scan: each thread owns nl / OTP_RTB consecutive counters
+  const u32 per = nl / OTP_RTB, j0 = threadIdx.x * per;
   u32 s = 0;
   for (u32 k = 0; k < per; k++) s += lc[j0 + k];
   u32 tot;
-  u32 pre = block_excl_scan_w<RTB / 64>(s, lw, &tot) + b0;
+  u32 pre = block_excl_scan_w<OTP_RTB / 64>(s, lw, &tot) + b0;
   for (u32 k = 0; k < per; k++) {
     const u32 v = lc[j0 + k];
     lc[j0 + k] = pre;
     pre += v;
   }
   __syncthreads();
-  for (u32 j = threadIdx.x; j < nl; j += RTB)
+  for (u32 j = threadIdx.x; j < nl; j += OTP_RTB)
     if (base + j < n2) db.ot_off[base + j] = lc[j];
   if (r + 1 == gridDim.x && threadIdx.x == 0) db.ot_off[n2] = *total;
   // every offset is read out of LDS before any cursor moves
   __syncthreads();
-  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * RTB) {
+  for (u32 p = b0 + threadIdx.x; p < b1; p += OTP_LD * OTP_RTB) {
     u32 l[OTP_LD], c[OTP_LD];
 #pragma unroll
     for (int q = 0; q < OTP_LD; q++) {
-      const uint2 e = p + q * RTB < b1 ? pair[p + q * RTB] : make_uint2(OTP_NONE, 0u);
+      const uint2 e = p + q * OTP_RTB < b1 ? pair[p + q * OTP_RTB] : make_uint2(OTP_NONE, 0u);
       l[q] = e.x;
       c[q] = e.y;
     }
@@ -1246,7 +1283,7 @@ __device__ inline void otp_range(const DB& db, int bits, u32 n2, u32 b0, u32 b1,
   }
   __syncthreads();
   // the cursors end at the next list's offset: size = cursor - offset
-  for (u32 j = threadIdx.x; j < nl; j += RTB)
+  for (u32 j = threadIdx.x; j < nl; j += OTP_RTB)
     if (base + j < n2) {
       const u32 sz = lc[j] - db.ot_off[base + j];
       db.ot_size[base + j] = sz;
@@ -1257,9 +1294,10 @@ template <bool TABLE>
 __global__ void __launch_bounds__(OTP_RTB) otp_range_k(DB db, int bits, u32 n2, u32 nblk, const u32* offs,
                                                   const u32* total, const void* in, u32* hist) {
   extern __shared__ u32 lc[];
+  __shared__ u32 st[TABLE ? OTP_LISTS : 1];
   const u32 r = blockIdx.x, b0 = offs[(size_t)r * nblk];
   const u32 b1 = r + 1 < gridDim.x ? offs[(size_t)(r + 1) * nblk] : *total;
-  otp_range<TABLE, OTP_RTB>(db, bits, n2, b0, b1, total, in, hist, lc);
+  otp_range<TABLE>(db, bits, n2, b0, b1, total, in, hist, lc, st);
 }
 
 // In two steps for many literals.  One step needs a range per 4,096 or 8,192
@@ -1367,67 +1405,34 @@ __global__ void __launch_bounds__(OTP_TB) otp2_part_k(const u32* offs, u32 nblk,
     }
   }
 }
-// a workgroup per part; lists of up to OTP2_STAGE entries (most parts, at 8
-// occurrences a literal) are put together in LDS and written in one run
-constexpr u32 OTP2_STAGE = 8 * OTP_RTB;
-static_assert(OTP_RTB == 1 << OTP2_BITS, "a literal to a thread");
+// a workgroup per part
 __global__ void __launch_bounds__(OTP_RTB) otp2_range_k(DB db, u32 n2, const u32* tb, const u32* counts,
                                                         const u32* total, const uint2* in, u32* hist) {
-  __shared__ u32 lc[OTP_RTB], st[OTP2_STAGE], lw[OTP_RTB / 64];
+  __shared__ u32 lc[1 << OTP2_BITS], st[OTP_LISTS];
   const u32 r = blockIdx.x >> OTP2_SUB, s = blockIdx.x & (OTP2_PARTS - 1), step = tb[r + 1] - tb[r];
-  const u32 word = (tb[r] << OTP2_SUB) + s * step;  // the next part starts where the next word says
-  const u32 b0 = counts[word], b1 = counts[word + step], n = b1 - b0;
-  if (n > OTP2_STAGE) {
-    otp_range<true, OTP_RTB>(db, OTP2_BITS, n2, b0, b1, total, in, hist, lc);
-    return;
-  }
-  constexpr int PT = OTP2_STAGE / OTP_RTB;
-  const u32 base = blockIdx.x << OTP2_BITS, lit = base + threadIdx.x;
-  lc[threadIdx.x] = 0;
-  __syncthreads();
-  uint2 e[PT];
-  u32 at[PT];
-#pragma unroll
-  for (int q = 0; q < PT; q++) {
-    const u32 j = q * OTP_RTB + threadIdx.x;
-    if (j < n) e[q] = in[b0 + j];
-  }
-#pragma unroll
-  for (int q = 0; q < PT; q++)
-    if (q * OTP_RTB + threadIdx.x < n) at[q] = atomicAdd(&lc[e[q].x - base], 1u);
-  __syncthreads();
-  u32 tot;
-  const u32 size = lc[threadIdx.x];
-  const u32 pre = block_excl_scan_w<OTP_RTB / 64>(size, lw, &tot);
-  lc[threadIdx.x] = pre;
-  if (lit < n2) {
-    db.ot_off[lit] = b0 + pre;
-    db.ot_size[lit] = size;
-    hist[lit] = size;
-  }
-  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) db.ot_off[n2] = *total;
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < PT; q++)
-    if (q * OTP_RTB + threadIdx.x < n) st[lc[e[q].x - base] + at[q]] = e[q].y;
-  __syncthreads();
-  for (u32 j = threadIdx.x; j < n; j += OTP_RTB) db.ot_refs[b0 + j] = st[j];
+  const u32 at = (tb[r] << OTP2_SUB) + s * step;  // the next part starts where the next word says
+  otp_range<true>(db, OTP2_BITS, n2, counts[at], counts[at + step], total, in, hist, lc, st);
 }
 bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2, int xcd) {
   // LDS per workgroup: nr words in the tile kernels, 1 << bits words in
-  // the range kernel (both within 64 KiB); ranges of 8192 literals once
-  // ranges of 4096 would number 2048 or more
-  int bits = 12;
+  // the range kernel (both within 64 KiB).  Ranges of 1,024 literals while
+  // there are few enough of them: a workgroup each, and a range's lists fit
+  // its LDS (against 4,096 in all cases, the range kernel took 9 instead of
+  // 29 us for 77,777 variables, 20 instead of 56 for 300,000, 25 instead of
+  // 67 for 500,000, the tile kernels as long as before); of 8192 literals
+  // once ranges of 4096 would number 2048 or more
+  int bits = 10;
+  while (bits < 12 && (n2 >> bits) >= 1024) bits++;
   if ((n2 >> bits) >= 2048) bits = 13;
   const size_t nr = (n2 + ((size_t)1 << bits) - 1) >> bits;
   if (nr > OTP_MAX_RANGES || ncls == 0) return false;
-  // tiles of 32 clauses per range (longer segments of pairs per range for
+  // tiles of 32 clauses per 4,096 literals (longer segments of pairs for
   // the partition's writes, fewer counts), at most 16,384 clauses: on the
   // heavy-tailed round (2,442 ranges) tiles of 16,384 clauses instead of
   // 131,072 gave 2,442 workgroups instead of 306 and took the count and
   // partition kernels from 0.56 + 2.69 to 0.38 + 2.24 ms
   size_t ct = 4096;
-  while (ct < 32 * nr && ct < 16384) ct <<= 1;
+  while (ct < 32 * (n2 >> 12) && ct < 16384) ct <<= 1;
   if (tile_log2 >= 10) ct = (size_t)1 << tile_log2;
   p->xcd = xcd;
   p->bits = bits;

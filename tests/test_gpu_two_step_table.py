@@ -17,7 +17,7 @@ def _formula(nvars, nclauses, seed):
     # variables at the ends of ranges, in a few dense stretches, and one in many clauses
     edges = np.concatenate([np.arange(k - 3, k + 4) for k in range(0, nvars + 512, 512)])
     edges = edges[(edges >= 1) & (edges <= nvars)]
-    dense = np.concatenate([np.arange(s, min(nvars, s + 9000)) for s in (1, nvars // 3, nvars - 8000)])
+    dense = np.concatenate([np.arange(s, min(nvars, s + 9000)) for s in (1, max(1, nvars // 3), max(1, nvars - 8000))])
     size = rng.choice([2, 3, 3, 4], nclauses)
     pick = rng.random(size.sum())
     v = np.where(pick < 0.5, rng.choice(dense, size.sum()), rng.choice(edges, size.sum()))
@@ -67,3 +67,11 @@ def test_tiles_and_no_room(tile):
     for opts in ({"otptile": tile}, {"otptile": tile, "otpxcd": 0}, {"literalsmul": 0}):
         d = diff(a, _run(cnf, **opts))
         assert not d, (opts, d)
+
+
+@pytest.mark.parametrize("nvars", [511, 512, 7200, 33333, 524286, 524287, 524288, 1048574, 1048575, 1048576])
+def test_range_widths(nvars):
+    """One step: ranges of 1,024 to 4,096 literals by their number."""
+    cnf = _formula(nvars, 150000, nvars)
+    d = diff(_run(cnf), _run(cnf, otpranges=0))
+    assert not d, d
