@@ -2162,8 +2162,8 @@ PF_HD int els_value(const DB& db, const ElsView& e, u32 lit, u32 p) {
 // the kept literals (mapped, duplicates dropped, first occurrence order)
 // are compacted in place, sorted, and size and signature updated; satisfied
 // and unit clauses are marked deleted.  Without write the clause is only
-// classified (an earlier kept literal is found again from the original
-// literals).
+// told to be a unit or not: a second kept literal ends it (4, whatever the
+// rest would make of it), so that one earlier literal is compared at most.
 PF_HD u32 els_clause(const DB& db, u32 c, const ElsView& e, u32 p, bool write, u32* unit, u32* m_out) {
   u32* l = clits(db, c);
   const u32 n = csize(db, c);
@@ -2186,14 +2186,9 @@ PF_HD u32 els_clause(const DB& db, u32 c, const ElsView& e, u32 p, bool write, u
     if (write) {
       for (u32 r = 0; r < m && seen < 0; r++)
         if (ABS(l[r]) == ABS(other)) seen = l[r] == other ? 0 : 1;
-    } else {
-      for (u32 r = 0; r < q && seen < 0; r++) {
-        const u32 lr = l[r];
-        if (els_value(db, e, lr, p) != -1) continue;
-        const u32 orr = e.rep[lr];
-        if (els_value(db, e, orr, p) != -1) continue;
-        if (ABS(orr) == ABS(other)) seen = orr == other ? 0 : 1;
-      }
+    } else if (m) {
+      if (ABS(first) != ABS(other)) return 4;
+      seen = first == other ? 0 : 1;
     }
     if (seen == 1) sat = true;
     if (seen != -1) continue;
