@@ -93,14 +93,21 @@ def round_bytes(r, V):
 
 def otp_counts(V, C):
     """Range-by-tile counts of the occurrence-table build (otp_plan in
-    pfs_kernels.hip): ranges of 4096 literals (8192 past 2048 such ranges),
-    tiles of the smallest power of two >= max(4096, 32 x ranges) clauses, at
-    most 16,384."""
+    pfs_kernels.hip): ranges of 1,024 to 4,096 literals, fewer than 1,024 of
+    them where possible (8,192 past 2,048 ranges of 4,096), or of 131,072 in
+    two steps (otp_plan2); tiles of the smallest power of two >= max(4096,
+    32 per 4,096 literals) clauses, at most 16,384."""
     n2 = 2 * V + 2
-    bits = 12 if (n2 >> 12) < 2048 else 13
+    bits = 10
+    while bits < 12 and (n2 >> bits) >= 1024:
+        bits += 1
+    if (n2 >> bits) >= 2048:
+        bits = 13
+    if n2 >= 1 << 22:
+        bits = 17
     nr = (n2 + (1 << bits) - 1) >> bits
     ct = 4096
-    while ct < 32 * nr and ct < 16384:
+    while ct < 32 * (n2 >> 12) and ct < 16384:
         ct <<= 1
     return nr * ((C + ct - 1) // ct)
 
@@ -129,6 +136,7 @@ def kernel_bytes(name, rounds, V):
       otp_part_k<false>   T + 4N + 4L   (the same with literals only)
       otp_range_k<true>   12L + 24V     (read the pairs, write one ref per literal, offsets, sizes, counts)
       otp_range_k<false>  4L + 8V       (read the literals, write the counts)
+      otp2_count_k, otp2_part_k, otp2_range_k   8L; 16L; 12L + 24V  (the second step of large tables, on the pairs)
     election (O_c occurrences in the candidates' lists, D_c their distinct
     clause bytes):
       lcve_classify_k     23V          (histogram 8V, list sizes 8V, states 2V; scores 4V, classes V)
@@ -155,8 +163,10 @@ def kernel_bytes(name, rounds, V):
             per.append(tl + 4 * n + 8 * l)
         elif name == "otp_part_k<false>":
             per.append(tl + 4 * n + 4 * l)
-        elif name == "otp_range_k<true>":
+        elif name in ("otp_range_k<true>", "otp2_range_k"):
             per.append(12 * l + 24 * V)
+        elif name in ("otp2_count_k", "otp2_part_k"):
+            per.append((8 if name == "otp2_count_k" else 16) * l)
         elif name == "otp_range_k<false>":
             per.append(4 * l + 8 * V)
         elif name == "hist_k":
