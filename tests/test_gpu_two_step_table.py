@@ -60,8 +60,8 @@ def test_sizes(nvars, nclauses):
 
 
 @pytest.mark.parametrize("tile", [10, 13])
-def test_tiles_and_no_room(tile):
-    """Other tiles of the first step, and a pool too small for the second's pairs."""
+def test_tiles_and_least_room(tile):
+    """Other tiles of the first step, and the least room in the pool."""
     cnf = _formula(2300000, 200000, tile)
     a = _run(cnf)
     for opts in ({"otptile": tile}, {"otptile": tile, "otpxcd": 0}, {"literalsmul": 0}):
@@ -74,4 +74,34 @@ def test_range_widths(nvars):
     """One step: ranges of 1,024 to 4,096 literals by their number."""
     cnf = _formula(nvars, 150000, nvars)
     d = diff(_run(cnf), _run(cnf, otpranges=0))
+    assert not d, d
+
+
+@pytest.mark.parametrize("nvars", [2300000, 4300000])
+def test_one_step_without_room(nvars):
+    """Long clauses and no room for resolvents: the idle pool cannot hold the
+    second step's pairs, and one step builds the table, in ranges of 4,096 or
+    8,192 literals."""
+    from parafrost_amd.simplifier import Simplifier
+    rng = np.random.default_rng(nvars)
+    v = np.sort(rng.choice(nvars, (60000, 9), replace=True) + 1, axis=1)
+    v[:20000, 0] = 1  # a list of many tiles
+    v = v[(np.diff(v, axis=1) > 0).all(axis=1)]
+    lits = (2 * v + rng.integers(0, 2, v.shape)).astype(np.uint32).ravel()
+    cnf = gen.Cnf(nvars, np.arange(len(v) + 1, dtype=np.uint64) * 9, lits)
+    s = Simplifier(0, phases=1, bce=1, profilegpu=1, literalsmul=0)
+    try:
+        s.upload(nvars, cnf.offsets, cnf.lits)
+        a = s.result(s.simplify())
+        names = set(s.kernel_times())
+    finally:
+        s.close()
+    print(sorted(n for n in names if n.startswith("otp")), flush=True)
+    assert "otp_range_k<true>" in names and "otp2_range_k" not in names
+    s = Simplifier(0, phases=1, bce=1, otpranges=0)
+    try:
+        s.upload(nvars, cnf.offsets, cnf.lits)
+        d = diff(a, s.result(s.simplify()))
+    finally:
+        s.close()
     assert not d, d
