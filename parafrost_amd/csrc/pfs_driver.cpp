@@ -21,6 +21,8 @@ static constexpr u32 INF = 0xFFFFFFFFu;
 // ---------------------------------------------------------------- memory
 void DeviceMemory::ensure(Buf& b, size_t bytes, size_t keep, Stream* st, Region r) {
   if (bytes <= b.cap) return;
+  for (Buf* s : spare)
+    if (client.used - b.cap + bytes > budget_ && s && s != &b) release(*s);
   if (client.used - b.cap + bytes > budget_)
     throw AllocFail{"device memory budget exceeded (" + std::to_string(client.used - b.cap + bytes) + " > " +
                     std::to_string(budget_) + " bytes)"};
@@ -949,7 +951,13 @@ bool Simplifier::otp_room(const OtpPlan& p) {
   return false;
 }
 
+// The pairs of the range build, like the records of ERE, are needed while it
+// runs only: in between they make way for whatever else the budget cannot
+// hold.  (A result's download was refused in a window of budgets that held
+// them and the rest but not the download, while smaller budgets, which had
+// done without, were enough.)
 void Simplifier::ot_counts(bool table) {
+  const DeviceMemory::InUse pairs_in_use(mem_, 0, &otp_);
   const size_t n2 = 2 * (size_t)V_ + 2;
   DB db = make_db(cur_);
   u32* hist = P<u32>(hist_);
@@ -1690,6 +1698,7 @@ bool Simplifier::ere_pairs() {
     }
   }
   kb.push_back(E_);
+  const DeviceMemory::InUse records_in_use(mem_, 1, &erecs_);
   bool ok = true;
   std::vector<u32> rec;                           // every chunk's records, k made global
   std::unordered_map<u32, std::vector<u32>> full;  // record -> all its matches, ascending

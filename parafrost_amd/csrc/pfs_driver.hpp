@@ -42,6 +42,15 @@ class DeviceMemory {
   size_t peak() const { return peak_; }
   size_t budget() const { return budget_; }
   void set_budget(size_t b) { budget_ = b; }
+  // buffers without lasting content, given back before a request is refused;
+  // InUse keeps one of them for as long as it is needed
+  Buf* spare[2] = {nullptr, nullptr};
+  struct InUse {
+    Buf*& slot;
+    Buf* b;
+    InUse(DeviceMemory& m, int q, Buf* buf) : slot(m.spare[q]), b(buf) { slot = nullptr; }
+    ~InUse() { slot = b; }
+  };
   DeviceArena* arena() const { return arena_; }
   ArenaClient client;
 
