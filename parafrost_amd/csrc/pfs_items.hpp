@@ -2291,4 +2291,99 @@ PF_HD u32 els_clause(const DB& db, u32 c, const ElsView& e, u32 p, bool write, u
   return 4;
 }
 
+// ---------------------------------------------------------------- appended clauses
+// clauses appended in order under the root assignment, each unit assigning its
+// literal for the clauses after it: passes over all of them until the units
+// stay the same (a pass after that returns at once).  seen[p & 1][variable]:
+// the earliest unit of pass p (pass_word << 32 | clause << 1 | sign), res: per
+// clause its unit literal, 1 if it is empty, else 0; kept, words: 1 and its
+// pool words if it stays with two literals or more.  fl (AP_FLAGS words,
+// zero before): 0 not for the device, 1 an empty clause, 2 units, 4 and 5 the
+// totals of kept and words, AP_CHANGED + p pass p found other units than p - 1
+constexpr u32 AP_PASSES = 32, AP_CHANGED = 8, AP_FLAGS = AP_CHANGED + AP_PASSES, AP_LONG = 128;
+struct AppendArgs {
+  const u64* off;
+  const u32* lits;
+  u32 n, nl;
+  u64* seen[2];
+  u32 *res, *kept, *words, *fl;
+  u64* units;  // (clause << 32 | literal) of the clauses that assign one, any order
+};
+PF_HD u32 append_word(u32 pass) { return 0xFFFFFFFEu - pass; }
+// f(literal) for each literal that stays, in order; returns whether the clause is satisfied
+template <class F>
+PF_HD bool append_clause(const DB& db, const AppendArgs& a, u32 i, const u32* l, u32 n, u32 pass, F f) {
+  bool sat = false;
+  for (u32 j = 0; j < n; j++) {
+    const u32 x = l[j], v = ABS(x), s = db.assign[v];
+    if (s) {
+      sat |= s - 1 == x;
+      continue;
+    }
+    if (pass) {
+      const u64 t = a.seen[(pass - 1) & 1][v];
+      if ((u32)(t >> 32) == append_word(pass - 1) && ((u32)t >> 1) < i) {
+        sat |= ((u32)t & 1u) == SIGN(x);
+        continue;
+      }
+    }
+    bool dup = false;
+    for (u32 k = 0; k < j; k++) {
+      dup |= l[k] == x;
+      sat |= l[k] == FLIP(x);
+    }
+    if (!dup) f(x);
+  }
+  return sat;
+}
+// Pass 0 looks at every literal; the passes after it index by them, and several
+// are queued before the host reads the flags, so none runs over a batch that
+// was refused (the flags are final once pass 0's launch has ended).
+PF_HD bool append_runs(const AppendArgs& a, u32 pass) {
+  return !pass || (!a.fl[0] && a.fl[AP_CHANGED + pass - 1]);
+}
+// returns whether the clause's unit is another than the pass before found
+PF_HD bool append_pass(const DB& db, const AppendArgs& a, u32 i, u32 pass) {
+  const u64 base = a.off[0], o0 = a.off[i] - base, o1 = a.off[i + 1] - base;
+  bool ok = o0 <= o1 && o1 <= a.nl && o1 - o0 <= AP_LONG;
+  const u32* l = a.lits + (ok ? o0 : 0);
+  const u32 n = ok ? (u32)(o1 - o0) : 0u;
+  if (!pass)
+    for (u32 j = 0; j < n; j++) ok &= ABS(l[j]) != 0 && ABS(l[j]) <= db.nvars;
+  u32 m = 0, u = 0, r = 0;
+  bool sat = true;
+  if (ok) sat = append_clause(db, a, i, l, n, pass, [&](u32 x) { m++, u = x; });
+  else a.fl[0] = 1;
+  if (!sat && m < 2) r = m ? u : 1u;
+  const bool changed = pass ? r != a.res[i] : r != 0;
+  if (r > 1) at_min64(&a.seen[pass & 1][ABS(r)], (u64)append_word(pass) << 32 | (u64)(i << 1 | SIGN(r)));
+  a.res[i] = r;
+  a.kept[i] = !sat && m > 1 ? 1u : 0u;
+  a.words[i] = !sat && m > 1 ? CL_HDR + m : 0u;
+  return changed;
+}
+PF_HD void append_write(const DB& db, const AppendArgs& a, u32 i, u32 last, u32 c0, u32 w0) {
+  const u32 r = a.res[i];
+  if (r == 1) a.fl[1] = 1;
+  if (r > 1 && ((u32)a.seen[last & 1][ABS(r)] >> 1) == i)
+    a.units[at_add(&a.fl[2], 1u)] = (u64)i << 32 | r;
+  // scanned: the clause stays if the next one's place differs
+  if ((i + 1 < a.n ? a.kept[i + 1] : a.fl[4]) == a.kept[i]) return;
+  const u64 o0 = a.off[i] - a.off[0];
+  u32* h = db.lits + w0 + a.words[i];
+  u32 m = 0;
+  append_clause(db, a, i, a.lits + o0, (u32)(a.off[i + 1] - a.off[i]), last + 1, [&](u32 x) {
+    u32 j = m++;  // insertion into the sorted literals before it
+    while (j > 0 && h[CL_HDR + j - 1] > x) {
+      h[CL_HDR + j] = h[CL_HDR + j - 1];
+      j--;
+    }
+    h[CL_HDR + j] = x;
+  });
+  db.c_off[c0 + a.kept[i]] = w0 + a.words[i];
+  h[0] = make_hdr(m, (u8)ST_ORIGINAL);
+  h[1] = calc_sig(h + CL_HDR, m);
+  h[2] = 0;
+}
+
 }  // namespace pfs

@@ -2903,81 +2903,15 @@ void k_build_clauses(const DB& db, const RawClauses& raw, void* tmp, Stream* st)
 // pass p is right for every chain of p units, and nothing changes any more
 // once it is right for all (7 passes of 3-4 us for those frames).  Clauses
 // longer than AP_LONG (quadratic in one thread) are left to the host.
-__device__ inline u32 append_word(u32 pass) { return 0xFFFFFFFEu - pass; }
-// f(literal) for each literal that stays, in order; returns whether the clause is satisfied
-template <class F>
-__device__ inline bool append_clause(const DB& db, const AppendArgs& a, u32 i, const u32* l, u32 n, u32 pass, F f) {
-  bool sat = false;
-  for (u32 j = 0; j < n; j++) {
-    const u32 x = l[j], v = ABS(x), s = db.assign[v];
-    if (s) {
-      sat |= s - 1 == x;
-      continue;
-    }
-    if (pass) {
-      const u64 t = a.seen[(pass - 1) & 1][v];
-      if ((u32)(t >> 32) == append_word(pass - 1) && ((u32)t >> 1) < i) {
-        sat |= ((u32)t & 1u) == SIGN(x);
-        continue;
-      }
-    }
-    bool dup = false;
-    for (u32 k = 0; k < j; k++) {
-      dup |= l[k] == x;
-      sat |= l[k] == FLIP(x);
-    }
-    if (!dup) f(x);
-  }
-  return sat;
-}
 __global__ void append_pass_k(DB db, AppendArgs a, u32 pass) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n || (pass && !a.fl[AP_CHANGED + pass - 1])) return;
-  const u64 base = a.off[0], o0 = a.off[i] - base, o1 = a.off[i + 1] - base;
-  bool ok = o0 <= o1 && o1 <= a.nl && o1 - o0 <= AP_LONG;
-  const u32* l = a.lits + (ok ? o0 : 0);
-  const u32 n = ok ? (u32)(o1 - o0) : 0u;
-  if (!pass)
-    for (u32 j = 0; j < n; j++) ok &= ABS(l[j]) != 0 && ABS(l[j]) <= db.nvars;
-  u32 m = 0, u = 0, r = 0;
-  bool sat = true;
-  if (ok) sat = append_clause(db, a, i, l, n, pass, [&](u32 x) { m++, u = x; });
-  else a.fl[0] = 1;
-  if (!sat && m < 2) r = m ? u : 1u;
-  const bool changed = pass ? r != a.res[i] : r != 0;
-  if (r > 1)
-    atomicMin((unsigned long long*)&a.seen[pass & 1][ABS(r)],
-              (unsigned long long)append_word(pass) << 32 | (unsigned long long)(i << 1 | SIGN(r)));
-  a.res[i] = r;
-  a.kept[i] = !sat && m > 1 ? 1u : 0u;
-  a.words[i] = !sat && m > 1 ? CL_HDR + m : 0u;
-  const u64 any = __ballot(changed);
+  if (i >= a.n || !append_runs(a, pass)) return;
+  const u64 any = __ballot(append_pass(db, a, i, pass));
   if (any && (threadIdx.x & 63) == (u32)__builtin_ctzll(any)) a.fl[AP_CHANGED + pass] = 1;
 }
 __global__ void append_write_k(DB db, AppendArgs a, u32 last, u32 c0, u32 w0) {
   const u32 i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const u32 r = a.res[i];
-  if (r == 1) a.fl[1] = 1;
-  if (r > 1 && ((u32)a.seen[last & 1][ABS(r)] >> 1) == i)
-    a.units[atomicAdd(&a.fl[2], 1u)] = (u64)i << 32 | r;
-  // scanned: the clause stays if the next one's place differs
-  if ((i + 1 < a.n ? a.kept[i + 1] : a.fl[4]) == a.kept[i]) return;
-  const u64 o0 = a.off[i] - a.off[0];
-  u32* h = db.lits + w0 + a.words[i];
-  u32 m = 0;
-  append_clause(db, a, i, a.lits + o0, (u32)(a.off[i + 1] - a.off[i]), last + 1, [&](u32 x) {
-    u32 j = m++;  // insertion into the sorted literals before it
-    while (j > 0 && h[CL_HDR + j - 1] > x) {
-      h[CL_HDR + j] = h[CL_HDR + j - 1];
-      j--;
-    }
-    h[CL_HDR + j] = x;
-  });
-  db.c_off[c0 + a.kept[i]] = w0 + a.words[i];
-  h[0] = make_hdr(m, (u8)ST_ORIGINAL);
-  h[1] = calc_sig(h + CL_HDR, m);
-  h[2] = 0;
+  if (i < a.n) append_write(db, a, i, last, c0, w0);
 }
 void k_append_pass(const DB& db, const AppendArgs& a, u32 pass, Stream* st) {
   KLAUNCH(append_pass_k, grid_for(a.n, 256), 256, st, db, a, pass);

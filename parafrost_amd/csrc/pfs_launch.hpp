@@ -254,23 +254,6 @@ struct RawClauses {
   u32* sc;
 };
 void k_build_clauses(const DB& db, const RawClauses& raw, void* tmp, Stream*);
-// clauses appended in order under the root assignment, each unit assigning its
-// literal for the clauses after it: passes over all of them until the units
-// stay the same (a pass after that returns at once).  seen[p & 1][variable]:
-// the earliest unit of pass p (pass_word << 32 | clause << 1 | sign), res: per
-// clause its unit literal, 1 if it is empty, else 0; kept, words: 1 and its
-// pool words if it stays with two literals or more.  fl (AP_FLAGS words,
-// zero before): 0 not for the device, 1 an empty clause, 2 units, 4 and 5 the
-// totals of kept and words, AP_CHANGED + p pass p found other units than p - 1
-constexpr u32 AP_PASSES = 32, AP_CHANGED = 8, AP_FLAGS = AP_CHANGED + AP_PASSES, AP_LONG = 128;
-struct AppendArgs {
-  const u64* off;
-  const u32* lits;
-  u32 n, nl;
-  u64* seen[2];
-  u32 *res, *kept, *words, *fl;
-  u64* units;  // (clause << 32 | literal) of the clauses that assign one, any order
-};
 void k_append_pass(const DB& db, const AppendArgs& a, u32 pass, Stream*);
 void k_append_place(const AppendArgs& a, void* tmp, Stream*);  // scans; tmp: 2 * scan_tmp_bytes(n)
 // after pass 'last', the first that changed nothing: the kept clauses into
