@@ -1084,7 +1084,7 @@ PF_HD bool count_res(const D& db, const Options& o, u32 x, int clsbefore, OLV me
   const int rlimit = o.ve_clause_limit;
   if (G > 1) {
     u32 cls = 0, lits = 0, over = 0;
-    const u32 np = me.n * other.n;
+    const u32 np = me.n * other.n;  // a group's lists are LDS copies: a few thousand entries at most
     for (u32 q = gl; q < np; q += G) {
       const u32 ci = me.r[q / other.n], cj = other.r[q % other.n];
       if (!is_original(db, ci) || !is_original(db, cj)) continue;
@@ -1524,7 +1524,7 @@ struct VeApply {
   u32 cls_cap, lit_cap, stack_cap;  // capacities: writes past them are refused
   u32* stack;
   UnitOut units;
-  u32* error;  // set when a write would leave its buffer
+  u32* error;  // set when a write would leave its buffer, or where fewer or more are written than counted
   ProofOut proof;
 };
 // bve.cpp:138-241, execution part
@@ -1587,10 +1587,10 @@ PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d
       if (olist(lv, dx).n > olist(lv, fx).n) { dx = n; fx = p; }
       const OLV me = olist(lv, dx), other = olist(lv, fx);
       u32 cid = a.cls0 + a.cls_base[k], lpos = a.lit0 + a.lit_base[k];
-      const u32 np = me.n * other.n;
+      const u64 np = (u64)me.n * other.n;  // lists that are not staged may be long
       u32 i = gl / other.n, j = gl % other.n;  // pair q = gl, then G further each time
       const u32 di = G / other.n, dj = G % other.n;
-      for (u32 q0 = 0; q0 < np; q0 += G) {
+      for (u64 q0 = 0; q0 < np; q0 += G) {
         u32 len = 0, ci = 0, cj = 0;
         if (q0 + gl < np) {
           ci = me.r[i];
@@ -1628,6 +1628,9 @@ PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d
         j += dj;
         if (j >= other.n) j -= other.n, i++;
       }
+      // the next variable's clauses start where this one's were counted to end
+      if (gl == 0 && (cid != a.cls0 + a.cls_base[k] + d.ncls[k] || lpos != a.lit0 + a.lit_base[k] + d.nlits[k]))
+        at_add(a.error, 1u);
     }
     save_side(lv, db, p, pOrgs, nOrgs, st, gl, G);
     delete_lists(db, p, gl, G);
