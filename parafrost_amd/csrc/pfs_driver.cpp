@@ -1051,21 +1051,22 @@ bool Simplifier::prop_visit(uint64_t front) {
   u32* trail = P<u32>(trail_);
   u32* sc = P<u32>(scal_);
   const uint64_t start_new = trail_n_;
+  // a level over the whole device, then the narrow ones after it in one
+  // launch, and one read for both; past a run's end the next level is wide
+  bool wide = trail_n_ - front > BCP_TURNS;
   while (front < trail_n_) {
     u32 h[3];
-    k_bcp_run(db, trail, (u32)front, (u32)trail_n_, sc, st_);
-    d2h(h, sc, 12, st_);
+    if (wide) {
+      fill_u32(sc, 0, 2, st_);
+      k_bcp_visit(db, trail + front, (u32)(trail_n_ - front), trail + trail_n_, sc, sc + 1, st_);
+      front = trail_n_;
+    }
+    k_bcp_run(db, trail, (u32)front, (u32)trail_n_, wide ? sc : nullptr, sc + 2, st_);
+    d2h(h, sc + 2, 12, st_);
     stream_sync(st_);
     trail_n_ = h[0];
     front = h[2];
-    if (!h[1] && front < trail_n_) {  // a wide level
-      fill_u32(sc, 0, 2, st_);
-      k_bcp_visit(db, trail + front, (u32)(trail_n_ - front), trail + trail_n_, sc, sc + 1, st_);
-      d2h(h, sc, 8, st_);
-      stream_sync(st_);
-      front = trail_n_;
-      if (!h[1]) trail_n_ += h[0];
-    }
+    wide = true;
     if (h[1]) {
       proof_line(PR_EMPTY, 0);  // learnEmpty (elimination.cpp:80-86)
       proof_flush();

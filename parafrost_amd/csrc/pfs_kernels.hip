@@ -1777,31 +1777,46 @@ void k_bcp_visit(const DB& db, const u32* front, u32 nfront, u32* next, u32* nne
 // Propagation level by level in one launch by one workgroup, as long as the
 // levels stay narrow: trail[front..end) is the frontier, a wavefront takes a
 // literal and its lanes the clauses of the list of its negation, the units
-// found follow on the trail.  Stops at the fixpoint, at a conflict (its
-// level's units are not on the trail) or before a level with more than
-// BCP_NARROW list entries, which bcp_visit_k spreads over the device;
-// out: the trail's end, the conflict, the first literal not propagated yet.
-// A level costs a chain of six dependent loads, about 6 us; a launch and a
-// read of its counters per level cost 30 us, and the unrolled circuits of
-// model checking propagate through 50-60 levels a request.
-constexpr u32 BCP_NARROW = 16384;
+// found follow on the trail.  more (nullable): the frontier is what a launch of
+// bcp_visit_k before this one appended, more[0] literals past 'end', unless
+// more[1] says that it met a conflict.  Stops at the fixpoint, at a conflict
+// (its level's units are not on the trail) or before a level that is not
+// narrow, which bcp_visit_k spreads over the device; out: the trail's end, the
+// conflict, the first literal not propagated yet.
+//
+// A wavefront spends a turn of 2.6 us, a chain of six dependent loads, on every
+// list however short (1.4 us for each further 64 entries of a long one); a level
+// by bcp_visit_k takes about 16 us with its read.  So a level is narrow by the
+// turns that it takes, BCP_TURNS of them over the 16 wavefronts and BCP_LONG
+// entries in one list.  Calls of 40 levels, all in one launch against a launch
+// and a read each: 64 literals of 1, 16 and 64 entries 0.70, 0.84 and 1.08 ms
+// against 0.87, 0.98 and 1.11; 128 literals 1.18, 1.47 and 1.95 against 1.01,
+// 1.13 and 1.35; 1,024 literals of one entry 7.6 against 1.5; one list of 256,
+// 1,024 and 16,384 entries 0.47, 1.09 and 14.8 against 0.86, 0.95 and 2.4.
+constexpr u32 BCP_LONG = 512;
 constexpr int BCP_T = 1024;
-__global__ void __launch_bounds__(BCP_T) bcp_run_k(DB db, u32* trail, u32 front, u32 end, u32* out) {
+__global__ void __launch_bounds__(BCP_T) bcp_run_k(DB db, u32* trail, u32 front, u32 end, const u32* more, u32* out) {
   __shared__ u32 s_end, s_conflict, s_work[2];
+  u32 conflict = 0;
+  if (more) {
+    conflict = more[1];
+    if (!conflict) end += more[0];
+  }
   if (threadIdx.x == 0) {
     s_end = end;
     s_conflict = 0;
     s_work[0] = s_work[1] = 0;
   }
   __syncthreads();
-  u32 conflict = 0;
-  for (u32 level = 0; front < end; level++) {
+  for (u32 level = 0; !conflict && front < end && end - front <= BCP_TURNS; level++) {
     u32 w = 0;
-    for (u32 i = front + threadIdx.x; i < end && w <= BCP_NARROW; i += BCP_T)
-      w += min(db.ot_size[FLIP(trail[i])], BCP_NARROW + 1);
-    if (w) atomicAdd(&s_work[level & 1], min(w, BCP_NARROW + 1));
+    for (u32 i = front + threadIdx.x; i < end; i += BCP_T) {
+      const u32 n = db.ot_size[FLIP(trail[i])];
+      w += n > BCP_LONG ? BCP_TURNS + 1 : max(1u, (n + 63) / 64);
+    }
+    if (w) atomicAdd(&s_work[level & 1], w);
     __syncthreads();
-    if (s_work[level & 1] > BCP_NARROW) break;
+    if (s_work[level & 1] > BCP_TURNS) break;
     if (threadIdx.x == 0) s_work[(level + 1) & 1] = 0;
     for (u32 i = front + threadIdx.x / 64; i < end; i += BCP_T / 64) {
       const OLV ol = olist(db, FLIP(trail[i]));
@@ -1820,8 +1835,8 @@ __global__ void __launch_bounds__(BCP_T) bcp_run_k(DB db, u32* trail, u32 front,
     out[2] = front;
   }
 }
-void k_bcp_run(const DB& db, u32* trail, u32 front, u32 end, u32* out, Stream* st) {
-  KLAUNCH(bcp_run_k, 1, BCP_T, st, db, trail, front, end, out);
+void k_bcp_run(const DB& db, u32* trail, u32 front, u32 end, const u32* more, u32* out, Stream* st) {
+  KLAUNCH(bcp_run_k, 1, BCP_T, st, db, trail, front, end, more, out);
 }
 __global__ void bcp_mark_k(DB db, const u32* lits, u8* mark) {
   const u32 t = lits[blockIdx.y];

@@ -128,9 +128,12 @@ void k_sort_lists(const DB& db, const u32* pv, u32 nvars, u32* classes, u32* cnt
 // ---- BCP
 void k_bcp_visit(const DB& db, const u32* front, u32 nfront, u32* next, u32* nnext, u32* conflict,
                  Stream*);
-// levels from trail[front..end) on while they are narrow; out: the trail's
-// end, whether a conflict was met, the first literal not propagated yet
-void k_bcp_run(const DB& db, u32* trail, u32 front, u32 end, u32* out, Stream*);
+// levels from trail[front..end) on while they are narrow (more: nnext and
+// conflict of a visit queued before, whose literals are the frontier, at 'end'
+// = front); out: the trail's end, whether a conflict was met, the first literal
+// not propagated yet
+constexpr u32 BCP_TURNS = 96;  // most literals of a narrow level
+void k_bcp_run(const DB& db, u32* trail, u32 front, u32 end, const u32* more, u32* out, Stream*);
 void k_bcp_mark(const DB& db, const u32* lits, u32 n, u8* mark, Stream*);
 void k_bcp_clean(const DB& db, u8* mark, Stream*);
 void k_clear_lists(const DB& db, const u32* lits, u32 n, Stream*);
