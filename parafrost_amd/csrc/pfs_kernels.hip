@@ -33,6 +33,7 @@
 #include <string>
 
 #include "pfs_launch.hpp"
+#include "pfs_staging.hpp"
 
 namespace pfs {
 
@@ -271,8 +272,8 @@ void h2d(void* dst, const void* src, size_t bytes, Stream* st) {
 // and 14.5 (slots of 1 / 2 / 4 MiB: 8.6 / 6.8 / 5.9 ms; 4, 6 and 8 threads
 // alike).
 // The ring is one per process, made by the first large download, used by one
-// call at a time (a second one copies directly) and given back with the
-// last stream.
+// call at a time (a second one copies directly, as does one that cannot start
+// the threads) and given back with the last stream.
 constexpr size_t STG_SLOT = 4 << 20, STG_MIN = 4 << 20;
 constexpr u32 STG_SLOTS = 4, STG_THREADS = 4;
 struct Staging {
@@ -318,74 +319,48 @@ static void staging_release() {
   std::lock_guard<std::mutex> use(g_staging.use);
   g_staging.drop();
 }
+// the ring as staged_copy drives it
+struct StagingRing {
+  u32 slots;
+  hipStream_t s;
+  std::atomic<hipError_t> err{hipSuccess};  // the first one
+  bool ok(hipError_t e) {
+    hipError_t none = hipSuccess;
+    if (e != hipSuccess) err.compare_exchange_strong(none, e);
+    return e == hipSuccess;
+  }
+  const unsigned char* slot(u32 k) { return g_staging.p + k * STG_SLOT; }
+  bool queue(u32 k, const StagedPiece& c) {
+    return ok(hipMemcpyAsync(g_staging.p + k * STG_SLOT, c.src, c.bytes, hipMemcpyDeviceToHost, s)) &&
+           ok(hipEventRecord(g_staging.ev[k], s));
+  }
+  bool arrived(u32 k) { return ok(hipEventSynchronize(g_staging.ev[k])); }
+  template <class F>
+  std::thread run(F f) {
+    return std::thread(f);
+  }
+};
 void d2h_set(const D2H* set, u32 n, Stream* st) {
   stream_op(st);
+  const auto direct = [&] {
+    for (u32 i = 0; i < n; i++)
+      if (set[i].bytes) PFS_HIP(hipMemcpyAsync(set[i].dst, set[i].src, set[i].bytes, hipMemcpyDeviceToHost, st->s));
+  };
   size_t total = 0;
   for (u32 i = 0; i < n; i++) total += set[i].bytes;
   std::unique_lock<std::mutex> lk(g_staging.use, std::defer_lock);
   const u32 nthr = std::min(STG_THREADS, std::max(1u, std::thread::hardware_concurrency() / 2));
-  if (total < STG_MIN || nthr < 2 || !lk.try_lock() || !g_staging.make(st->device)) {
-    for (u32 i = 0; i < n; i++)
-      if (set[i].bytes) PFS_HIP(hipMemcpyAsync(set[i].dst, set[i].src, set[i].bytes, hipMemcpyDeviceToHost, st->s));
-    return;
-  }
-  struct Piece {
-    char* dst;
-    const char* src;
-    size_t bytes;
-  };
-  std::vector<Piece> pc;
+  if (total < STG_MIN || nthr < 2 || !lk.try_lock() || !g_staging.make(st->device)) return direct();
+  std::vector<StagedPiece> pc;
   for (u32 i = 0; i < n; i++)
     for (size_t o = 0; o < set[i].bytes; o += STG_SLOT)
-      pc.push_back(Piece{(char*)set[i].dst + o, (const char*)set[i].src + o, std::min(STG_SLOT, set[i].bytes - o)});
-  const u32 np = (u32)pc.size();
-  std::vector<std::atomic<u32>> done(np);  // threads that have moved their share of a piece
-  for (auto& d : done) d.store(0, std::memory_order_relaxed);
-  std::atomic<u32> queued{0};
-  std::atomic<bool> failed{false};
-  // piece i sits in slot i % STG_SLOTS once its event has passed
-  auto mover = [&](u32 t) {
-    for (u32 i = 0; i < np; i++) {
-      while (queued.load(std::memory_order_acquire) <= i) {
-        if (failed.load(std::memory_order_relaxed)) return;
-        std::this_thread::yield();
-      }
-      if (hipEventSynchronize(g_staging.ev[i % STG_SLOTS]) != hipSuccess) {
-        failed.store(true);
-        return;
-      }
-      const size_t share = (pc[i].bytes / nthr + 63) & ~(size_t)63;
-      const size_t a = std::min(pc[i].bytes, t * share), b = t + 1 == nthr ? pc[i].bytes : std::min(pc[i].bytes, a + share);
-      memcpy(pc[i].dst + a, g_staging.p + (i % STG_SLOTS) * STG_SLOT + a, b - a);
-      done[i].fetch_add(1, std::memory_order_release);
-    }
-  };
-  std::vector<std::thread> thr;
-  hipError_t err = hipSuccess;
-  try {
-    thr.reserve(nthr);
-    for (u32 t = 0; t < nthr; t++) thr.emplace_back(mover, t);
-    for (u32 i = 0; i < np && err == hipSuccess && !failed.load(std::memory_order_relaxed); i++) {
-      // the slot is free once every thread has moved its piece before
-      while (i >= STG_SLOTS && done[i - STG_SLOTS].load(std::memory_order_acquire) < nthr &&
-             !failed.load(std::memory_order_relaxed))
-        std::this_thread::yield();
-      const u32 k = i % STG_SLOTS;
-      err = hipMemcpyAsync(g_staging.p + k * STG_SLOT, pc[i].src, pc[i].bytes, hipMemcpyDeviceToHost, st->s);
-      if (err == hipSuccess) err = hipEventRecord(g_staging.ev[k], st->s);
-      if (err == hipSuccess) queued.store(i + 1, std::memory_order_release);
-    }
-  } catch (...) {  // a thread could not be started: the ones that were return
-    failed.store(true);
-    for (std::thread& t : thr) t.join();
-    throw;
-  }
-  if (err != hipSuccess) failed.store(true);
-  for (std::thread& t : thr) t.join();
-  if (err != hipSuccess || failed.load()) {
-    (void)hipStreamSynchronize(st->s);  // nothing writes to the slots any more
-    throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(err) + " in a staged download");
-  }
+      pc.push_back({(char*)set[i].dst + o, (const char*)set[i].src + o, std::min(STG_SLOT, set[i].bytes - o)});
+  StagingRing ring{STG_SLOTS, st->s};
+  const Staged r = staged_copy(pc, nthr, ring);
+  if (r == Staged::NOT_STARTED) direct();
+  if (r != Staged::FAILED) return;
+  (void)hipStreamSynchronize(st->s);  // nothing writes to the slots any more
+  throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(ring.err.load()) + " in a staged download");
 }
 void d2h(void* dst, const void* src, size_t bytes, Stream* st) {
   if (!bytes) return;
