@@ -58,11 +58,12 @@ Staged staged_copy(const std::vector<StagedPiece>& pc, uint32_t nthr, R& ring) {
     for (std::thread& t : thr) t.join();
     return Staged::NOT_STARTED;
   }
-  for (uint32_t i = 0; i < np && !failed.load(std::memory_order_relaxed); i++) {
+  for (uint32_t i = 0; i < np; i++) {
     // the slot is free once every thread has moved its piece before
     while (i >= slots && done[i - slots].load(std::memory_order_acquire) < nthr &&
            !failed.load(std::memory_order_relaxed))
       std::this_thread::yield();
+    if (failed.load(std::memory_order_relaxed)) break;  // a thread may still read the slot
     if (ring.queue(i % slots, pc[i])) queued.store(i + 1, std::memory_order_release);
     else failed.store(true);
   }

@@ -1,5 +1,5 @@
 """The staged download on a host build (tests/staging/staging_host.cpp), under
-AddressSanitizer: whole pieces and remainders through rings
+ThreadSanitizer and AddressSanitizer: whole pieces and remainders through rings
 of one to four slots, and what it does where a thread cannot be started (leaves
 everything to the caller), a copy cannot be queued or a wait fails (says so)."""
 import json
@@ -12,7 +12,7 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-@pytest.mark.parametrize("sanitizer", ["address,undefined"])
+@pytest.mark.parametrize("sanitizer", ["thread", "address,undefined"])
 def test_staged_copy(sanitizer):
     with tempfile.TemporaryDirectory() as d:
         exe = os.path.join(d, "staging_host")
