@@ -261,13 +261,15 @@ void h2d(void* dst, const void* src, size_t bytes, Stream* st) {
   }
   PFS_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st->s));
 }
-// Large downloads.  The caller's buffers are pageable: the runtime moves such
-// a copy at 18 GB/s, and the 134 MB of a 4.4M-clause result took 7.8 ms.
-// They go through a ring of pinned slots instead: the calling thread keeps
-// the copies into the slots going, and a few threads, which live as long as
-// the call, each move their share of every slot that has arrived to the
-// caller's memory (one thread moves about 10 GB/s, the link 57, so it takes
-// several; page faults of a fresh buffer are shared out with them).
+// Large downloads.  The caller's buffers are pageable as a rule: the runtime
+// moves such a copy at 18 GB/s, and the 134 MB of a 4.4M-clause result took 7.8
+// ms.  (Into pinned buffers it moves 57 GB/s, and they are left to it: 133 MB
+// take 2.5 ms, 3.05 through the ring.)  They go through a ring of pinned slots
+// instead: the calling thread keeps the copies into the slots going, and a few
+// threads, which live as long as the call, each move their share of every slot
+// that has arrived to the caller's memory (one thread moves about 10 GB/s, the
+// link 57, so it takes several; page faults of a fresh buffer are shared out
+// with them).
 // Into buffers used before, 134 MB take 3.3 ms and 290 MB 5.9 instead of 7.8
 // and 14.5 (slots of 1 / 2 / 4 MiB: 8.6 / 6.8 / 5.9 ms; 4, 6 and 8 threads
 // alike).
@@ -340,24 +342,40 @@ struct StagingRing {
     return std::thread(f);
   }
 };
+// ordinary host memory, which a direct copy fills slowly (pinned, managed and
+// device memory it fills at the link's rate)
+static bool pageable(const void* p) {
+  hipPointerAttribute_t at{};
+  if (hipPointerGetAttributes(&at, p) == hipSuccess) return at.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
+}
 void d2h_set(const D2H* set, u32 n, Stream* st) {
   stream_op(st);
-  const auto direct = [&] {
-    for (u32 i = 0; i < n; i++)
-      if (set[i].bytes) PFS_HIP(hipMemcpyAsync(set[i].dst, set[i].src, set[i].bytes, hipMemcpyDeviceToHost, st->s));
+  const auto direct = [&](const D2H& c) {
+    if (c.bytes) PFS_HIP(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, st->s));
   };
-  size_t total = 0;
+  size_t total = 0, slow = 0;
   for (u32 i = 0; i < n; i++) total += set[i].bytes;
+  u32 staged = 0;  // bit i: set[i] goes through the ring
+  for (u32 i = 0; i < n && total >= STG_MIN; i++)
+    if (set[i].bytes && pageable(set[i].dst)) staged |= 1u << i, slow += set[i].bytes;
   std::unique_lock<std::mutex> lk(g_staging.use, std::defer_lock);
   const u32 nthr = std::min(STG_THREADS, std::max(1u, std::thread::hardware_concurrency() / 2));
-  if (total < STG_MIN || nthr < 2 || !lk.try_lock() || !g_staging.make(st->device)) return direct();
+  if (slow < STG_MIN || nthr < 2 || !lk.try_lock() || !g_staging.make(st->device)) staged = 0;
   std::vector<StagedPiece> pc;
-  for (u32 i = 0; i < n; i++)
-    for (size_t o = 0; o < set[i].bytes; o += STG_SLOT)
-      pc.push_back({(char*)set[i].dst + o, (const char*)set[i].src + o, std::min(STG_SLOT, set[i].bytes - o)});
+  for (u32 i = 0; i < n; i++) {
+    if (!(staged >> i & 1)) direct(set[i]);
+    else
+      for (size_t o = 0; o < set[i].bytes; o += STG_SLOT)
+        pc.push_back({(char*)set[i].dst + o, (const char*)set[i].src + o, std::min(STG_SLOT, set[i].bytes - o)});
+  }
+  if (!staged) return;
   StagingRing ring{STG_SLOTS, st->s};
   const Staged r = staged_copy(pc, nthr, ring);
-  if (r == Staged::NOT_STARTED) direct();
+  if (r == Staged::NOT_STARTED)
+    for (u32 i = 0; i < n; i++)
+      if (staged >> i & 1) direct(set[i]);
   if (r != Staged::FAILED) return;
   (void)hipStreamSynchronize(st->s);  // nothing writes to the slots any more
   throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(ring.err.load()) + " in a staged download");
