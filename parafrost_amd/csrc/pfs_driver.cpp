@@ -191,18 +191,22 @@ void Simplifier::upload(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
   // The arrays go over as the caller has them and the device builds the pool
   // (a host loop over the clauses took 2 of the 2.8 ms of an upload of 0.9M
   // literals, and 0.7 s for 120M).  They wait in buffers that nothing uses
-  // before the first round: the literals and the offsets in the other
-  // block's pool (W + 4096 words at least, W = literals + 3 per clause), the
-  // LBDs in its handles, the flags in the marks.
+  // before the first round: the literals, the offsets and the flags in the
+  // other block's pool (W + 4096 words at least, W = literals + 3 per clause;
+  // they take 2 1/4 per clause and 4), the LBDs in its handles.
   u32* raw_lits = P<u32>(lits_[1]);
   u64* raw_off = (u64*)(raw_lits + ((nl + 1) & ~(uint64_t)1));
+  u8* raw_flags = (u8*)(raw_off + ncls + 1);
   u32* sc = P<u32>(scal_);
-  fill_u32(sc, 0, 3, st_);  // error, learnt clauses, their words
+  const size_t V1 = (size_t)V_ + 1;
+  // the error, the learnt clauses and their words, and the state (one launch:
+  // a small upload is launches and little else)
+  zero_set({{sc, 12}, {assign_.p, V1 * 4}, {vstate_.p, V1}, {assumed_.p, V1}, {mark_.p, lcap_}}, st_);
   h2d(raw_off, offsets, (ncls + 1) * 8, st_);
   h2d(raw_lits, lits ? lits + offsets[0] : nullptr, nl * 4, st_);
-  if (flags) h2d(mark_.p, flags, ncls, st_);
+  if (flags) h2d(raw_flags, flags, ncls, st_);
   if (flags && lbd) h2d(c_off_[1].p, lbd, ncls * 4, st_);
-  RawClauses raw{raw_off, raw_lits, flags ? P<u8>(mark_) : nullptr, flags && lbd ? P<u32>(c_off_[1]) : nullptr,
+  RawClauses raw{raw_off, raw_lits, flags ? raw_flags : nullptr, flags && lbd ? P<u32>(c_off_[1]) : nullptr,
                  nullptr, nullptr, (u32)ncls, (u32)L, maxvar, sc};
   if (flags) {  // extraction order: originals, then learnts (simplify.cpp:148-149)
     mem_.ensure(tmp2_, std::max<size_t>(ncls, 1) * 4, 0, st_);
@@ -219,11 +223,7 @@ void Simplifier::upload(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
   h_touched_.clear();
   in_units_.assign(trail, trail + ntrail);
   for (u32 i = 0; i < ntrail; i++) h_assign_[ABS(trail[i])] = trail[i] + 1;
-  const size_t V1 = (size_t)V_ + 1;
   u32 melted = 0;
-  fill_u32(P<u32>(assign_), 0, V1, st_);
-  fill_u8(P<u8>(vstate_), 0, V1, st_);
-  fill_u8(P<u8>(assumed_), 0, V1, st_);
   if (vstate) {
     for (u32 v = 1; v <= V_; v++) melted += (vstate[v] & (VS_MELTED | VS_SUBSTITUTED)) ? 1 : 0;
     h2d(P<u8>(vstate_) + 1, vstate + 1, V_, st_);
@@ -247,7 +247,6 @@ void Simplifier::upload(uint32_t maxvar, uint64_t ncls, const uint64_t* offsets,
   proof_n_ = 0;
   refuted_ = false;
   resident_ = false;
-  fill_u8(P<u8>(mark_), 0, lcap_, st_);
   stream_sync(st_);
   if (built[0]) throw std::invalid_argument("literal out of range");
   has_learnts_ = built[1] != 0;

@@ -437,6 +437,31 @@ void fill_u8(u8* dst, u8 value, size_t n, Stream* st) {
   if (!n) return;
   KLAUNCH(fill_u8_k, grid_for((n + 15) / 16, 256), 256, st, dst, value, n);
 }
+// several buffers cleared by one launch, 4 KiB of one to a workgroup
+struct ZeroSet {
+  u8* p[ZERO_PARTS];
+  size_t n[ZERO_PARTS];
+  u32 end[ZERO_PARTS];  // past a buffer's last workgroup
+};
+__global__ void __launch_bounds__(256) zero_set_k(ZeroSet z) {
+  u32 q = 0;
+  while (blockIdx.x >= z.end[q]) q++;  // the last one ends the grid
+  u8* d = z.p[q];
+  const size_t n = z.n[q], i = ((size_t)(blockIdx.x - (q ? z.end[q - 1] : 0)) * 256 + threadIdx.x) * 16;
+  if (i + 16 <= n && ((uintptr_t)(d + i) & 15u) == 0) *(uint4*)(d + i) = make_uint4(0, 0, 0, 0);
+  else
+    for (size_t k = i; k < n && k < i + 16; k++) d[k] = 0;
+}
+void zero_set(const ZeroPart (&part)[ZERO_PARTS], Stream* st) {
+  ZeroSet z;
+  u32 end = 0;
+  for (u32 q = 0; q < ZERO_PARTS; q++) {
+    z.p[q] = (u8*)part[q].p;
+    z.n[q] = part[q].bytes;
+    z.end[q] = end += (u32)((part[q].bytes + 4095) / 4096);
+  }
+  if (end) KLAUNCH(zero_set_k, end, 256, st, z);
+}
 struct Marker {
   hipEvent_t e;
 };

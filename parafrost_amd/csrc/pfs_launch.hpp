@@ -36,6 +36,13 @@ void d2h_set(const D2H* set, u32 n, Stream*);
 void d2d(void* dst, const void* src, size_t bytes, Stream*);
 void fill_u32(u32* dst, u32 value, size_t n, Stream*);  // fill kernel, no memset nodes
 void fill_u8(u8* dst, u8 value, size_t n, Stream*);
+// several buffers cleared at once
+constexpr u32 ZERO_PARTS = 5;
+struct ZeroPart {
+  void* p;
+  size_t bytes;
+};
+void zero_set(const ZeroPart (&part)[ZERO_PARTS], Stream*);
 // stage timing: events recorded on the stream
 // the position of a stream at a point in its queue (a timing-free event)
 struct Marker;
