@@ -1170,10 +1170,11 @@ PF_HD u32 find_equ_gate(const D& db, u32 p, u32 gl = 0, u32 G = 1) {
   return 0;
 }
 // and.h:25-86.  The gate's long clause holds -dx and the literals implied by
-// the original binary clauses of dx, all of them and no other.  A clause of
-// -dx with one literal more than there are binaries is that clause iff each
-// of its other literals is implied by some binary: its literals are
-// distinct, so as many binaries then imply as many different literals.
+// the original binary clauses of dx, all of them and no other, as often as they
+// are implied.  A clause of -dx with one literal more than there are binaries
+// is that clause iff each of its other literals is implied by as many binaries
+// as it stands there (an uploaded clause may hold a literal twice): the numbers
+// then add up to all of them.
 template <class D>
 PF_HD bool find_ao_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int& nAddedCls, u32& nAddedLits,
                         u32 gl = 0, u32 G = 1) {
@@ -1199,6 +1200,14 @@ PF_HD bool find_ao_gate(const D& db, const Options& o, u32 dx, int nOrgCls, int&
         bool hit = false;
         for (u32 i = gl; i < it.n && !hit; i += G) hit = org_binary(db, it.r[i]) && implied(db, it.r[i], dx) == x;
         all = group_any(hit, gl, G);
+      }
+      for (u32 q = 1; q <= nb && all; q++) {  // sorted: twice stands side by side
+        const u32 x = l[q];
+        if (x != l[q - 1]) continue;
+        u32 need = x == f ? 0u : 1u, hits = 0;
+        for (u32 k = 1; k <= nb; k++) need += l[k] == x && l[k - 1] == x;
+        for (u32 i = gl; i < it.n; i += G) hits += org_binary(db, it.r[i]) && implied(db, it.r[i], dx) == x;
+        all = group_sum(hits, G) >= need;
       }
       if (!all) continue;
       for (u32 i = gl; i < it.n; i += G)
