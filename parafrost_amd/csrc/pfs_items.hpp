@@ -1596,12 +1596,15 @@ PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d
       if (olist(lv, dx).n > olist(lv, fx).n) { dx = n; fx = p; }
       const OLV me = olist(lv, dx), other = olist(lv, fx);
       u32 cid = a.cls0 + a.cls_base[k], lpos = a.lit0 + a.lit_base[k];
-      const u64 np = (u64)me.n * other.n;  // lists that are not staged may be long
-      u32 i = gl / other.n, j = gl % other.n;  // pair q = gl, then G further each time
+      const u32 cid1 = cid + d.ncls[k], lpos1 = lpos + d.nlits[k];  // where the next variable's start
+      // pair gl, then G further each time, by its row and column: the pairs of
+      // two lists that are not staged may be more than 2^32
+      u32 i = gl / other.n, j = gl % other.n;
+      u32 i0 = 0, j0 = 0;  // the group's first pair
       const u32 di = G / other.n, dj = G % other.n;
-      for (u64 q0 = 0; q0 < np; q0 += G) {
+      while (i0 < me.n) {
         u32 len = 0, ci = 0, cj = 0;
-        if (q0 + gl < np) {
+        if (i < me.n) {
           ci = me.r[i];
           cj = other.r[j];
           // a length of 0 is a tautology
@@ -1636,10 +1639,11 @@ PF_HD void ve_apply(const L& lv, const DB& db, u32 v, u32 k, const VeDecision& d
         i += di;
         j += dj;
         if (j >= other.n) j -= other.n, i++;
+        i0 += di;
+        j0 += dj;
+        if (j0 >= other.n) j0 -= other.n, i0++;
       }
-      // the next variable's clauses start where this one's were counted to end
-      if (gl == 0 && (cid != a.cls0 + a.cls_base[k] + d.ncls[k] || lpos != a.lit0 + a.lit_base[k] + d.nlits[k]))
-        at_add(a.error, 1u);
+      if (gl == 0 && ((cid ^ cid1) | (lpos ^ lpos1))) at_add(a.error, 1u);  // not as counted
     }
     save_side(lv, db, p, pOrgs, nOrgs, st, gl, G);
     delete_lists(db, p, gl, G);
