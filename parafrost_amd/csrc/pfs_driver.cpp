@@ -33,12 +33,19 @@ void DeviceMemory::ensure(Buf& b, size_t bytes, size_t keep, Stream* st, Region 
   }
   void* old = b.p;
   const size_t old_cap = b.cap;
-  try {
-    arena_->alloc(&client, bytes, r, &b.p);  // sets b.p
-  } catch (std::bad_alloc&) {
-    b.p = old;
-    throw AllocFail{"device arena allocation of " + std::to_string(bytes) + " bytes failed"};
-  }
+  const auto placed = [&] {
+    try {
+      arena_->alloc(&client, bytes, r, &b.p);  // sets b.p
+      return true;
+    } catch (std::bad_alloc&) {
+      b.p = old;
+      return false;
+    }
+  };
+  bool ok = placed();
+  for (Buf* s : spare)
+    if (!ok && s && s != &b && s->p) release(*s), ok = placed();
+  if (!ok) throw AllocFail{"device arena allocation of " + std::to_string(bytes) + " bytes failed"};
   if (old) {
     if (keep) d2d(b.p, old, std::min(keep, old_cap), st);
     arena_->release(&client, old);  // returns to the pool once the copy has run
