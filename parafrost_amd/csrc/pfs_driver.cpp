@@ -970,13 +970,13 @@ void Simplifier::ot_counts(bool table) {
   OtpPlan p;
   auto build = [&](int tile) {
     if (!opt.otp_ranges || !otp_plan(n2, db.ncls, &p, tile, opt.otp_xcd)) return false;
-    if (ot_one_fits(n2, db.ncls)) {
+    const size_t slots = lits_end_ >= CL_HDR * ncls_ ? lits_end_ - CL_HDR * ncls_ : lits_end_;
+    if (ot_one_fits(n2, db.ncls, slots)) {
       k_ot_one(db, (u32)n2, table, hist, st_);
       used_tile_ = (int32_t)ilog2(p.ct);
       return true;
     }
     const auto pad = [](size_t words) { return (words + 63) & ~(size_t)63; };  // to 256 bytes
-    const size_t slots = lits_end_ >= CL_HDR * ncls_ ? lits_end_ - CL_HDR * ncls_ : lits_end_;
     OtpPlan two;
     // two steps: the second one's pairs wait in the other block's pool, which
     // nothing uses until the collection writes it

@@ -1474,12 +1474,20 @@ bool otp_plan2(size_t n2, size_t ncls, size_t pairs, OtpPlan* p, int tile_log2, 
   p->ncounts2 = ((size_t)p->tiles2 << OTP2_SUB) + 1;
   return true;
 }
-// the same for a formula whose literals fit one workgroup's counters and
-// whose clauses are few (OT_ONE_LITS, OT_ONE_CLAUSES): counted, scanned and
-// placed in one launch without the pairs.  For a circuit of 5,000 variables
-// and 17,000 clauses the four launches take 52 us, most of it waiting for a
-// handful of workgroups, this one 36 us; it reads the literals twice with one
-// workgroup, so past these clauses the four are again the faster ones.
+// The same for a small formula: counted, scanned and placed in one launch
+// without the pairs.  One workgroup walks the clauses twice where the tile and
+// range kernels walk them once, on a workgroup per tile and per range of 1,024
+// literals; what they lose are three launches.  So it is the faster way up to
+// OT_ONE_LITS literals where there is one tile (its clauses are one workgroup's
+// in either way), or where the clauses and occurrences are few for the number
+// of ranges; past that, up to as many counters as the LDS holds, only for one
+// tile of long clauses.  Whole calls, this against
+// ranges: 500 variables, 16,000 clauses of 3 122 against 140 us; 1,000
+// variables, 8,000 of 10 197 and 235, 16,000 of 10 225 and 215; 4,000
+// variables, 4,000 of 3 118 and 117, 8,000 of 3 143 and 130, 4,000 of 100 620
+// and 850; 5,000 variables, 6,500 of 3 130 and 124; 7,000 variables, 2,300 of 3
+// 111 and 104, of 30 429 and 445, 2,000 of 1,000 3,540 and 4,480, 32,000 of 30
+// 1,520 and 355.
 template <bool TABLE>
 __global__ void __launch_bounds__(OTP_TB) otp_one_k(DB db, u32 n2, u32* hist) {
   extern __shared__ u32 lc[];
@@ -1508,7 +1516,11 @@ __global__ void __launch_bounds__(OTP_TB) otp_one_k(DB db, u32 n2, u32* hist) {
   __syncthreads();
   otp_tile(db, 0, db.ncls, [&](u32 l, u32 c) { db.ot_refs[atomicAdd(&lc[l], 1u)] = c; });
 }
-bool ot_one_fits(size_t n2, size_t ncls) { return n2 <= OT_ONE_LITS && ncls <= OT_ONE_CLAUSES; }
+bool ot_one_fits(size_t n2, size_t ncls, size_t slots) {
+  const size_t ranges = (n2 + 1023) >> 10;
+  if (n2 > OT_ONE_LITS) return n2 <= OT_ONE_LITS_LONG && ncls <= OT_ONE_TILE && slots >= 16 * ncls;
+  return ncls <= OT_ONE_TILE || (ncls * ranges <= OT_ONE_CLAUSES && slots * ranges <= OT_ONE_SLOTS);
+}
 void k_ot_one(const DB& db, u32 n2, bool table, u32* hist, Stream* st) {
   if (table) KLAUNCH_LDS(otp_one_k<true>, 1, OTP_TB, (size_t)n2 * 4, st, db, n2, hist);
   else KLAUNCH_LDS(otp_one_k<false>, 1, OTP_TB, (size_t)n2 * 4, st, db, n2, hist);

@@ -110,9 +110,10 @@ constexpr int OTP2_BITS = 10, OTP2_SUB = 7;
 constexpr u32 OTP2_TILE = 8192, OTP2_MAX_RANGES = 1024;
 constexpr size_t OTP2_MIN_LITS = (size_t)1 << 22;
 bool otp_plan2(size_t n2, size_t ncls, size_t pairs, OtpPlan* p, int tile_log2 = 0, int xcd = 0);
-// small formulas: the table (or the counts) in one launch, no pair buffer
-constexpr u32 OT_ONE_LITS = 14336, OT_ONE_CLAUSES = 32768;
-bool ot_one_fits(size_t n2, size_t ncls);
+// small formulas: the table (or the counts) in one launch, no pair buffer.
+// slots: at least the live occurrences
+constexpr u32 OT_ONE_LITS = 10240, OT_ONE_LITS_LONG = 14336, OT_ONE_TILE = 4096, OT_ONE_CLAUSES = 24576, OT_ONE_SLOTS = 320 << 10;
+bool ot_one_fits(size_t n2, size_t ncls, size_t slots);
 void k_ot_one(const DB& db, u32 n2, bool table, u32* hist, Stream*);
 // counts: p.ncounts + 1 words; pairs: 8-byte aligned, two words per live
 // literal occurrence with 'table', else one.  Without 'table' only hist is
