@@ -114,8 +114,9 @@ pfs_status pfs_arena_get_stats(pfs_arena* arena, int32_t device, pfs_arena_stats
  * "decomposemin" (1-10, default 2) is pfs_decompose's default round count.
  * "mapperc" (real in [0, 1], default 0.2) is the inactive share above which
  * pfs_map renumbers.
- * "workorder" (boolean, default on; no reference counterpart) launches the
- * per-variable kernels heaviest lists first; results do not depend on it.
+ * "workorder" (boolean, default on; no reference counterpart) runs SUB and the
+ * VE decisions longest lists first among the variables of like size; results
+ * do not depend on it.
  * GPU-build options (src/gpu/options.cpp:24-43, options.cu:36-60):
  * "electionsmax" and "lcveclausemax" cap the election (default: no cap, as
  * the CPU simplifier); "aggresivesort" sorts the result's clauses by the

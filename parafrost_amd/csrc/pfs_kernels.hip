@@ -1435,8 +1435,10 @@ __global__ void __launch_bounds__(OTP_RTB) otp2_range_k(DB db, u32 n2, const u32
   otp_range<true>(db, OTP2_BITS, n2, counts[at], counts[at + step], total, in, hist, lc, st);
 }
 bool otp_plan(size_t n2, size_t ncls, OtpPlan* p, int tile_log2, int xcd) {
-  // LDS per workgroup: nr words in the tile kernels, 1 << bits words in
-  // the range kernel (both within 64 KiB).  Ranges of 1,024 literals while
+  // LDS per workgroup: nr words in the tile kernels (up to 48 KiB); in the
+  // range kernel 1 << bits words, and for a table the 32 KiB in which a range's
+  // lists are put together: 64 KiB and 64 bytes for ranges of 8,192 literals,
+  // of the 160 KiB that a workgroup may have on gfx950.  Ranges of 1,024 literals while
   // there are few enough of them: a workgroup each, and a range's lists fit
   // its LDS (against 4,096 in all cases, the range kernel took 9 instead of
   // 29 us for 77,777 variables, 20 instead of 56 for 300,000, 25 instead of
@@ -2500,15 +2502,6 @@ __device__ inline u32 lv_class(u64 need) {
   return q == LV_BIG && need > LV_WAVES * LV_CAP ? LV_CLASSES - 1 : q;
 }
 __device__ inline u32 lv_class_lanes(u32 q) { return q < LV_BIG ? 32u >> q : 64u; }
-// The least class of a launch over n variables: where they would leave
-// lanes idle, each takes the largest group that keeps the launch within the
-// lanes of LV_BLOCKS workgroups.  A variable's chain of dependent loads and
-// LDS reads is then walked G entries at a time, and the chunks spread over
-// the CUs.  Against a lane per variable, per launch (ve_decide_k, sub_k): 45
-// elected variables 290 + 155 -> 48 + 27 us; 3,206: 350 + 260 -> 55 + 60 us.
-// Twice and four times the lanes: 0.35 + 0.22 instead of 0.24 + 0.16 ms on
-// 77,777 variables (three launches), 0.17 and 0.19 instead of 0.16 ms on
-// 300,000, 0.59 and 0.55 instead of 0.60 ms on 100,000 gates (five).
 // list occurrences as a descending 5-bit code: exact below 16, then four
 // steps per power of two up to 256
 constexpr int LV_FINE_BITS = 5;
@@ -2585,15 +2578,24 @@ __device__ inline void lv_chunks(const u32* work, u32* lds, F f) {
 }
 // as many workgroups as the LDS lets onto the CUs, at most one per variable
 constexpr u32 LV_BLOCKS = 256 * (160 * 1024 / LV_LDS);
+// The least class of a launch over n variables: where they would leave
+// lanes idle, each takes the largest group that keeps the launch within the
+// lanes of LV_BLOCKS workgroups.  A variable's chain of dependent loads and
+// LDS reads is then walked G entries at a time, and the chunks spread over
+// the CUs.  Against a lane per variable, per launch (ve_decide_k, sub_k): 45
+// elected variables 290 + 155 -> 48 + 27 us; 3,206: 350 + 260 -> 55 + 60 us.
+// Twice and four times the lanes: 0.35 + 0.22 instead of 0.24 + 0.16 ms on
+// 77,777 variables (three launches), 0.17 and 0.19 instead of 0.16 ms on
+// 300,000, 0.59 and 0.55 instead of 0.60 ms on 100,000 gates (five).
 static u32 lv_floor(u32 n) {
   u32 c = 0;
   while (c < LV_BIG - 1 && ((u64)n << (c + 2)) <= (u64)LV_BLOCKS * LV_WAVES * 64) c++;
   return c;
 }
 
-// VE decisions in two launches: the gate checks (pure, equivalence,
-// AND/OR) for every elected variable, then, staged, the variables they
-// leave open (ITE and XOR searches, resolvent count)
+// VE decisions in one launch over every elected variable's staged lists: the
+// gate checks (pure, equivalence, AND/OR), the ITE and XOR searches and the
+// resolvent count.
 // lsum[2k], lsum[2k + 1]: bounds on the clause size sums of the lists of
 // elected variable k (from the list sort).  The searches' work grows with
 // the square of the list lengths, their memory linearly: a variable's
